@@ -53,3 +53,43 @@ def test_alpha_endpoint_codebook_matches_oracle(gpu, seed, side, k):
     assert np.array_equal(ends, rends), np.nonzero(ends != rends)[0][:10]
     assert np.array_equal(rv, rrv)
     assert np.array_equal(bsel, rbsel)
+
+
+def _one_cluster_each(sizes):
+    ofs = np.zeros(len(sizes) + 1, np.uint32)
+    ofs[1:] = np.cumsum(sizes)
+    blocks = np.zeros((2, 16, 4), np.uint8)
+    return ofs, np.full(2, 0xFFFFFFFF, np.uint32), blocks
+
+
+@pytest.mark.parametrize("sizes", [(1, 2, 3, 5, 63, 65, 257, 1023, 4097), (300001,)])
+@pytest.mark.parametrize("what", ["flat", "two", "noise"])
+def test_refiner_sums_any_size(gpu, sizes, what):
+    """The refiners' parallel sums give the start of the sums in texel order:
+    clusters of any texel count, flat ones (the singular system of one colour
+    on a middle selector, whose sums round once per texel) and noisy ones."""
+    print("hc refiner", what, sizes, flush=True)
+    rng = np.random.default_rng(len(sizes))
+    ofs, bc, blocks = _one_cluster_each(sizes)
+    px = np.full((ofs[-1], 4), 255, np.uint8)
+    for a, b in zip(ofs[:-1], ofs[1:]):
+        if what == "noise":
+            px[a:b, :3] = np.clip(rng.integers(0, 256, 3) + rng.normal(0, 9, (b - a, 3)), 0, 255)
+            px[a:b, :3] &= 0xFC if b - a > 5000 else 0xFF     # few enough distinct colours for the oracle
+        else:
+            px[a:b, :3] = rng.integers(0, 256, 3)
+            if what == "two":
+                px[a + (b - a) // 3:b, :3] = rng.integers(0, 256, 3)
+    w, enc = np.ones(2, np.float32), np.zeros(2, np.uint8)
+    ends, cv, _, ne = run_gpu(px, ofs, bc, blocks, w, enc, True)
+    rends, rcv, _ = oracle.hc_color_endpoints(px, ofs, bc, blocks, w, enc, True)
+    assert ne == 0
+    assert np.array_equal(cv, rcv)
+    assert np.array_equal(ends, rends), np.nonzero(ends != rends)[0][:10]
+    vals, av = np.ascontiguousarray(px[:, 1]), blocks[:, :, 3].copy()
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    got = hc.alpha_endpoints(d(vals), d(ofs.astype(np.int32)), d(bc.view(np.int32)), d(av), d(enc))
+    torch.cuda.synchronize()
+    ref = oracle.hc_alpha_endpoints(vals, ofs, bc, av, enc)
+    assert np.array_equal(got[0].cpu().numpy().view(np.uint32), ref[0])
+    assert np.array_equal(got[1].cpu().numpy(), ref[1]) and np.array_equal(got[2].cpu().numpy(), ref[2])
