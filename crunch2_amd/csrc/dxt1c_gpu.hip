@@ -1,5 +1,5 @@
 // dxt1c_gpu.hip -- DXT1 endpoint search for pixel clusters of any size, one
-// wave per cluster (the dxt_hc endpoint-cluster case).
+// workgroup per cluster (the dxt_hc endpoint-cluster case).
 //
 // Reference: dxt1_endpoint_optimizer::compute (crnlib/crn_dxt1.cpp:2081-2246)
 // at uber quality.  Without 3-colour blocks (the path dxt_hc uses for its
@@ -14,16 +14,44 @@
 // optimize_endpoint_comps and the special cases follow crn_dxt1.cpp as in the
 // per-block kernel (dxt1_gpu.hip).
 //
-// Layout: one workgroup of one wave per cluster; the cluster's unique colours,
-// weights, selectors, colour hash and per-channel error tables live in LDS.
-// Control flow is wave-uniform (every lane holds the same search state); the
-// O(colours) integer loops (candidate errors, selectors, planes, the LSQ and
-// per-channel sums) are split across the lanes and reduced with wave
-// shuffles, which is exact for integer sums.  Float sums (means, covariance,
-// 4-means) keep the reference's sequential order so the float trajectory
-// matches the CPU restatement.
+// Layout: one workgroup per cluster; the cluster's unique colours, weights,
+// selectors and per-channel error tables live in LDS.  Wave 0 runs the search
+// (its state is wave-uniform); the other waves wait for batches of candidates
+// and score their share.
+//
+// Scoring is a contraction and runs on the matrix cores.  The distance of
+// colour c to palette entry p is |c|^2 - 2 c.p + |p|^2 under the channel
+// weights; |c|^2 is the same for every candidate and summed once, and the
+// rest is a product of [r, g, g, g, b, 1, 1, 1] with
+// [-16 pr, -32 pg, -16 pg, -2 pg, -2 pb, K2, K1, K0] (K = |p|^2 in three 8-bit
+// limbs): every factor is an integer of at most 8 significant bits times a
+// power of two, exact in bfloat16, and every partial sum an integer below
+// 2^24, exact in float32.  One v_mfma_f32_32x32x16_bf16 gives 32 colours x 8
+// palettes x 4 entries; a lane takes the minimum of its four entries and adds
+// weight x minimum in double (integers below 2^53 for clusters of up to 2^30
+// texels).  So a candidate's error is the exact integer, whatever the order.
+//
+// Candidates are scored in batches and taken in the reference's order:
+// evaluate_solution (:1312-1340) keeps a candidate when its error-plane bound
+// and then its error are below the best at its turn.  A batch holds candidates
+// whose bound is below the best at the gather; the ordered scan over
+// max(bound, error) then takes what the reference takes.  Lists that read the
+// current best (the lattice moves, optimize_endpoint_comps) are gathered again
+// after each candidate taken.
+//
+// Float sums (means, covariance, 4-means) keep the reference's sequential
+// order: a chunk of 64 colours' terms is computed by all lanes into LDS, then
+// one lane per sum adds them one after another.
+//
+// What bounds it: the chain of lists of the largest clusters, and for the many
+// small ones the vector work around the matrix instructions.  Scored by 64
+// lanes with 60 integer operations per colour and candidate, one candidate at a
+// time on one wave, the classes took 91 / 25 / 17 / 8 ms side by side on the
+// 2048^2 DXT1 chain at quality 128 (2,415 clusters, 1,388 of 2,049 to 4,096
+// texels); now 3.2 ms for the longest class.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <mutex>
@@ -33,10 +61,9 @@
 
 namespace {
 
-// Largest cluster: 4096 unique colours.  The kernel comes in four LDS sizes
-// (512, 1024, 2048 and 4096 unique colours: 18, 28, 49 and 89 KiB) so that
-// small clusters, the common case, run eight, five or three waves per CU
-// instead of one.
+// Largest cluster kept in LDS: 4096 unique colours.  The kernel comes in four
+// sizes by texel count (512, 1024, 2048 and 4096), so that small clusters, the
+// common case, share a CU, and a fifth for more texels of at most 4096 colours.
 constexpr uint32_t kMaxU = 4096;
 
 __device__ __constant__ int16_t c_uber_probe[15] = {0, 1, 2, 3, 5, 7, 9, 10, 13, 15, 19, 27, 43, 59, 91};
@@ -47,45 +74,104 @@ __device__ __constant__ int8_t c_adj[26][3] = {
     {0, 1, 1}, {1, 1, 1}};
 __device__ uint8_t g_c_om5[256][2], g_c_om6[256][2], g_c_om5_3[256][2], g_c_om6_3[256][2];
 
-template <uint32_t MaxU>
-struct LdsT {
-    static constexpr uint32_t kCapU = MaxU;        // unique colours
-    static constexpr uint32_t kCapH = 2 * MaxU;    // colour hash slots (power of two)
-    uint32_t col[MaxU];      // r | g << 8 | b << 16
-    uint32_t w[MaxU];
-    uint8_t sel[MaxU];
-    uint32_t hkey[kCapH];    // colour | 0xFF000000, 0 = empty
-    uint16_t hval[kCapH];
-    unsigned long long pl[3][64][3];   // error planes: count, sum, sum of squares per quantised value
-    uint64_t rlo[32], rhi[32], glo[64], ghi[64], blo[32], bhi[32];
+// Candidates scored together: 32, or 64 (one per lane) where eight waves share them.
+template <uint32_t W>
+constexpr uint32_t kBatchOf = W >= 8 ? 64 : 32;
+constexpr uint32_t kMaxBatch = 64;
+struct Pal {
+    int r[4], g[4], b[4];
 };
 
-// The store of the size classes whose texel count never exceeds the colour
-// capacity (512, 1024, 2048): no colour hash.  The unique-colour pass sorts
-// (colour, texel index) pairs in a buffer that overlays the search's tables
-// (dead until the search starts), and a per-texel unique index replaces the
-// hash lookup of the final selectors: 11, 16 and 29 KiB instead of 18, 28
-// and 49, so more clusters run per CU.
+constexpr uint32_t kRow = 68;       // floats per staged sum: 64 terms, the rows on different LDS banks
+constexpr uint32_t kRowD = 66;      // doubles per staged sum
+
+// Per-channel error of one selector class as a function of the class's value
+// p: W p^2 - WP2 p + WPP (the reference's compute_endpoint_component_errors
+// tables, crn_dxt1.cpp:369-418, evaluated where they are read).
+struct QErr {
+    uint64_t W[4], WP2[4], WPP[4];
+    __device__ inline uint64_t at(int sl, uint64_t p) const { return W[sl] * p * p - WP2[sl] * p + WPP[sl]; }
+};
+
+// The search's working set in LDS.
+struct SearchLds {
+    uint32_t cmd;                // candidates to score | alternate rounding << 8; 0: the search has ended
+    Pal end_pal;                 // the result, for the texels' selectors
+    uint32_t end_alpha, end_inv, end_enforce, end_enforced;
+    uint32_t cand[kMaxBatch];       // low | high << 16
+    uint32_t cidx[kMaxBatch];       // the candidate's place in its list
+    uint64_t bnd[kMaxBatch];        // its error-plane bound
+    uint64_t err[2 * kMaxBatch];    // palette sums: one per candidate, or four-colour and three-colour
+    union {
+        float f[6][kRow];
+        double d[6][kRowD];
+    } stage;                     // terms of the sequential float sums
+    uint32_t list[2][64];        // the list's colours (sweep ends, combinatorial set, means)
+    QErr q;                      // optimize_endpoint_comps
+    uint64_t brem[4], qbest;
+    int fixed[2][3];             // refine_solution's rounded endpoints / the components not being optimised
+};
+
+// Error planes (count, sum, sum of squares per quantised value) are dead once
+// the per-value bounds are made; the search's working set takes their space.
+union PlanesOrSearch {
+    unsigned long long pl[3][64][3];
+    SearchLds q;
+};
+
+struct Bounds {
+    uint64_t rlo[32], rhi[32], glo[64], ghi[64], blo[32], bhi[32];
+    uint64_t base;       // sum of weight x |colour|^2
+};
+
+// Store of the size classes whose texel count never exceeds the colour
+// capacity.  The unique-colour pass sorts (colour, texel index) pairs in a
+// buffer that overlays the search's tables (dead until the search starts):
+// 13, 15, 24 and 49 KiB.
 template <uint32_t MaxU>
 struct LdsS {
-    static constexpr uint32_t kCapU = MaxU;
-    static constexpr uint32_t kSearch = MaxU + 8 * (3 * 64 * 3) + 8 * (32 + 32 + 64 + 64 + 32 + 32);
+    static constexpr uint32_t kSearch = MaxU + sizeof(PlanesOrSearch) + sizeof(Bounds);
     static constexpr uint32_t kSort = 6 * MaxU;   // u32 colours + u16 texel indices
-    uint32_t col[MaxU];
+    uint32_t col[MaxU];      // r | g << 8 | b << 16
     uint16_t w[MaxU];
-    uint16_t tmap[MaxU];                 // texel -> unique colour
     uint32_t fbits[MaxU / 32];           // first texel of each colour
     uint32_t fbase[MaxU / 32];           // first texels before each word of fbits
+    uint32_t nuniq, nopaque;
+    int scan[8];                         // per wave
     uint8_t sel[MaxU];                   // from here on: the sort buffers' space
-    unsigned long long pl[3][64][3];
-    uint64_t rlo[32], rhi[32], glo[64], ghi[64], blo[32], bhi[32];
+    PlanesOrSearch u;
+    Bounds b;
     uint8_t pad[kSort > kSearch ? kSort - kSearch : 4];
+};
+
+// Store of clusters of more texels but at most MaxU distinct colours: a colour
+// hash with the first texel and the count of each colour, whose space the
+// search takes over (128 KiB).
+template <uint32_t MaxU>
+struct LdsT {
+    static constexpr uint32_t kCapH = 2 * MaxU;    // colour hash slots (power of two)
+    uint32_t col[MaxU];          // during the unique-colour pass: first texels ...
+    uint32_t w[MaxU];            // ... and hash slots (u16) being sorted
+    uint32_t nuniq, nopaque, nsort, pad;
+    union {
+        struct {
+            uint32_t hkey[kCapH];        // colour | 0xFF000000, 0 = empty
+            uint32_t hval[kCapH];        // first texel
+            uint32_t hcnt[kCapH];
+        };
+        struct {
+            uint8_t sel[MaxU];
+            PlanesOrSearch u;
+            Bounds b;
+        };
+    };
 };
 
 // A colour store tagged with the evaluator: kUber -- evaluate_solution_uber
 // with both block types (3-colour blocks allowed); else the hc evaluators.
 template <class Base, bool U>
 struct LdsU : Base {
+    using Base::Base;
     static constexpr bool kUber = U;
 };
 
@@ -99,6 +185,7 @@ struct St {
     int perceptual;
     int have_alpha;      // DXT1A: texels below the alpha threshold are transparent (3-colour blocks only)
     uint32_t nu, total_w;
+    uint64_t base;       // sum of weight x |colour|^2
     float mean[3], meanw[3], pw[3], axis[3];
     Best best;
     bool sel_valid;      // L.sel holds the selectors of the current best solution
@@ -107,14 +194,39 @@ struct St {
 
 __device__ inline uint32_t lane_id() { return threadIdx.x & 63u; }
 
+__device__ inline uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ inline uint64_t uni64(uint64_t v) { return (uint64_t)uni((uint32_t)v) | ((uint64_t)uni((uint32_t)(v >> 32)) << 32); }
+__device__ inline bool unib(bool v) { return uni(v ? 1u : 0u) != 0; }
+__device__ inline float unif(float v) { return __builtin_bit_cast(float, uni(__builtin_bit_cast(uint32_t, v))); }
+__device__ inline uint32_t lane_u32(uint32_t v, uint32_t l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l); }
+__device__ inline uint64_t lane_u64(uint64_t v, uint32_t l)
+{
+    return (uint64_t)lane_u32((uint32_t)v, l) | ((uint64_t)lane_u32((uint32_t)(v >> 32), l) << 32);
+}
+__device__ inline float lane_f32(float v, uint32_t l) { return __builtin_bit_cast(float, lane_u32(__builtin_bit_cast(uint32_t, v), l)); }
+__device__ inline double lane_f64(double v, uint32_t l) { return __builtin_bit_cast(double, lane_u64(__builtin_bit_cast(uint64_t, v), l)); }
+
+template <int Ctrl, int RowMask>
+__device__ inline uint64_t dpp_add(uint64_t v)
+{
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, Ctrl, RowMask, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), Ctrl, RowMask, 0xF, false);
+    return v + ((uint64_t)lo | ((uint64_t)hi << 32));
+}
+
+// Sums over each half of the wave, in lanes 31 and 63.
+__device__ inline uint64_t half_sums(uint64_t v)
+{
+    v = dpp_add<0x111, 0xF>(v);   // row_shr 1, 2, 4, 8
+    v = dpp_add<0x112, 0xF>(v);
+    v = dpp_add<0x114, 0xF>(v);
+    v = dpp_add<0x118, 0xF>(v);
+    return dpp_add<0x142, 0xA>(v);   // row_bcast15 into rows 1 and 3
+}
+
 __device__ inline uint64_t wave_sum(uint64_t v)
 {
-    for (int off = 32; off > 0; off >>= 1) {
-        const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)v, off);
-        const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(v >> 32), off);
-        v += ((uint64_t)hi << 32) | lo;
-    }
-    return v;
+    return lane_u64(dpp_add<0x143, 0xC>(half_sums(v)), 63);   // row_bcast31 into rows 2 and 3
 }
 
 __device__ inline uint32_t hash32(uint32_t x)
@@ -156,11 +268,9 @@ __device__ inline uint32_t pack565(int r, int g, int b, int scaled)
 
 __device__ inline void canon(uint32_t& lo, uint32_t& hi)
 {
-    if (lo < hi) {
-        const uint32_t t = lo;
-        lo = hi;
-        hi = t;
-    }
+    const uint32_t a = max(lo, hi), b = min(lo, hi);
+    lo = a;
+    hi = b;
 }
 
 __device__ inline uint32_t cdist(int perceptual, uint32_t px, int r, int g, int b)
@@ -168,10 +278,6 @@ __device__ inline uint32_t cdist(int perceptual, uint32_t px, int r, int g, int 
     const int dr = (int)(px & 255u) - r, dg = (int)((px >> 8) & 255u) - g, db = (int)((px >> 16) & 255u) - b;
     return perceptual ? (uint32_t)(dr * dr * 8 + dg * dg * 25 + db * db) : (uint32_t)(dr * dr + dg * dg + db * db);
 }
-
-struct Pal {
-    int r[4], g[4], b[4];
-};
 
 __device__ inline Pal palette4(uint32_t lo, uint32_t hi, int alt)
 {
@@ -200,163 +306,384 @@ __device__ inline Pal palette3(uint32_t lo, uint32_t hi, int alt)
     return p;
 }
 
-// evaluate_solution_hc (crn_dxt1.cpp:1759-1835): sum over colours of the
-// weighted distance to the nearest of the four colours.
-template <class Lds>
-__device__ bool eval_hc(St& s, const Lds& L, uint32_t lo, uint32_t hi, int alt)
+// ------------------------------------------------------------- scoring
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// Two integers of at most 8 significant bits (times a power of two) as bfloat16.
+__device__ inline uint32_t bf2(float a, float b)
 {
-    const Pal p = palette4(lo, hi, alt);
-    uint64_t err = 0;
-    for (uint32_t i = lane_id(); i < s.nu; i += 64) {
-        const uint32_t px = L.col[i];
-        const uint32_t e0 = cdist(s.perceptual, px, p.r[0], p.g[0], p.b[0]);
-        const uint32_t e1 = cdist(s.perceptual, px, p.r[1], p.g[1], p.b[1]);
-        const uint32_t e2 = cdist(s.perceptual, px, p.r[2], p.g[2], p.b[2]);
-        const uint32_t e3 = cdist(s.perceptual, px, p.r[3], p.g[3], p.b[3]);
-        err += (uint64_t)min(min(e0, e1), min(e2, e3)) * L.w[i];
-    }
-    err = wave_sum(err);
-    if (err >= s.best.err) return false;
-    s.best.lo = lo;
-    s.best.hi = hi;
-    s.best.err = err;
-    s.best.alt = alt;
-    s.best.enforce = lo == hi;
-    if (s.best.enforce) {
-        if ((s.best.lo & 31) != 31) {
-            s.best.lo++;
-            s.best.enforced = 1;
-        } else {
-            s.best.hi--;
-            s.best.enforced = 0;
-        }
-    }
-    s.sel_valid = false;
-    return true;
+    return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xFFFF0000u);
 }
 
-// evaluate_solution_uber (crn_dxt1.cpp:1370-1592), both block types: the
-// 4-colour error, then (alpha blocks allowed) the 3-colour error, each
-// kept when below the best so far (exact integer sums over the colours);
-// a 4-colour pair with equal endpoints enforces one selector.  The selectors
-// of the kept type are recomputed on demand (compute_selectors).
-template <class Lds>
-__device__ bool eval_uber(St& s, const Lds& L, uint32_t lo, uint32_t hi, int alt)
+// Row `row` (palette row / 4, entry row % 4) of the palettes' operand.
+template <bool Uber>
+__device__ inline bf16x8 palette_row(const SearchLds& q, uint32_t pal, uint32_t entry, uint32_t n, int alt,
+                                     int perceptual)
 {
-    const Pal p4 = palette4(lo, hi, alt), p3 = palette3(lo, hi, alt);
-    uint64_t e4 = 0, e3 = 0;
-    for (uint32_t i = lane_id(); i < s.nu; i += 64) {
-        const uint32_t px = L.col[i];
-        const uint32_t d0 = cdist(s.perceptual, px, p4.r[0], p4.g[0], p4.b[0]);
-        const uint32_t d1 = cdist(s.perceptual, px, p4.r[1], p4.g[1], p4.b[1]);
-        const uint32_t d2 = cdist(s.perceptual, px, p4.r[2], p4.g[2], p4.b[2]);
-        const uint32_t d3 = cdist(s.perceptual, px, p4.r[3], p4.g[3], p4.b[3]);
-        e4 += (uint64_t)min(min(d0, d1), min(d2, d3)) * L.w[i];
-        {
-            const uint32_t t2 = cdist(s.perceptual, px, p3.r[2], p3.g[2], p3.b[2]);
-            e3 += (uint64_t)min(min(d0, d1), t2) * L.w[i];
-        }
+    const uint32_t cand = Uber ? pal >> 1 : pal;
+    const bool three = Uber && (pal & 1u);
+    const uint32_t c = q.cand[min(cand, n - 1)];
+    int a[3], b[3], p[3];
+    unpack565(c & 0xFFFFu, 1, a[0], a[1], a[2]);
+    unpack565(c >> 16, 1, b[0], b[1], b[2]);
+    for (int k = 0; k < 3; k++) {
+        const int far = entry == 2 ? a[k] : b[k], near = entry == 2 ? b[k] : a[k];
+        const int mid = three ? (a[k] + b[k] + alt) >> 1 : (far * 2 + near + alt) / 3;
+        p[k] = entry == 0 ? a[k] : entry == 1 ? b[k] : mid;
     }
-    e4 = wave_sum(e4);
-    e3 = wave_sum(e3);
-    uint64_t terr = s.best.err;
-    int talpha = 0;
+    const float r = (float)p[0], g = (float)p[1], bl = (float)p[2];
+    const uint32_t K = perceptual ? (uint32_t)(8 * p[0] * p[0] + 25 * p[1] * p[1] + p[2] * p[2])
+                                  : (uint32_t)(p[0] * p[0] + p[1] * p[1] + p[2] * p[2]);
+    u32x4 v;
+    v.x = perceptual ? bf2(-16.0f * r, -32.0f * g) : bf2(-2.0f * r, -2.0f * g);
+    v.y = perceptual ? bf2(-16.0f * g, -2.0f * g) : 0u;
+    v.z = bf2(-2.0f * bl, (float)(K & 0xFF0000u));
+    v.w = bf2((float)(K & 0xFF00u), (float)(K & 0xFFu));
+    return __builtin_bit_cast(bf16x8, v);
+}
+
+// Sums of weight x smallest distance for the batch's palettes, groups of
+// eight dealt to the W waves; Lds::kUber scores two palettes per candidate.
+template <class Lds, uint32_t W>
+__device__ void score(Lds& L, SearchLds& q, uint32_t nu, uint64_t base, int perceptual, uint32_t n, int alt,
+                      uint32_t wave)
+{
+    constexpr uint32_t kPer = Lds::kUber ? 2 : 1;
+    constexpr uint32_t kShare = kBatchOf<W> * kPer / 8 / W;
+    constexpr uint32_t G = kShare >= 2 ? 2 : 1;   // groups that share a pass over the colours
+    const uint32_t groups = (n * kPer + 7) / 8;
+    const uint32_t col = lane_id() & 31u, half = lane_id() >> 5;
+    for (uint32_t g0 = wave * G; g0 < groups; g0 += W * G) {
+        bf16x8 A[G];
+        double acc[G][4];
+#pragma unroll
+        for (uint32_t t = 0; t < G; t++) {
+            A[t] = palette_row<Lds::kUber>(q, 8 * (g0 + t) + (col >> 2), col & 3u, n, alt, perceptual);
+            if (half) A[t] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[t][j] = 0.0;
+        }
+        for (uint32_t i0 = 0; i0 < nu; i0 += 32) {
+            const uint32_t i = min(i0 + col, nu - 1);
+            const uint32_t px = L.col[i];
+            const double w = i0 + col < nu ? (double)L.w[i] : 0.0;
+            const float r = (float)(px & 255u), g = (float)((px >> 8) & 255u), b = (float)((px >> 16) & 255u);
+            const u32x4 v = {bf2(r, g), bf2(g, g), bf2(b, 1.0f), bf2(1.0f, 1.0f)};
+            const bf16x8 B = __builtin_bit_cast(bf16x8, v);
+#pragma unroll
+            for (uint32_t t = 0; t < G; t++) {
+                const f32x16 zero = {0};
+                const f32x16 d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[t], B, zero, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float m = fminf(fminf(d[4 * j], d[4 * j + 1]), fminf(d[4 * j + 2], d[4 * j + 3]));
+                    acc[t][j] = __builtin_fma(w, (double)m, acc[t][j]);
+                }
+            }
+        }
+#pragma unroll
+        for (uint32_t t = 0; t < G; t++)
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++) {
+                const uint64_t e = base + half_sums((uint64_t)(int64_t)acc[t][j]);
+                const uint32_t pal = 8 * (g0 + t) + 2 * j + half;
+                if (col == 31u && pal < kPer * n) q.err[pal] = e;
+            }
+    }
+}
+
+// The waves beside wave 0: score their share of each batch until the search ends.
+template <class Lds, uint32_t W>
+__device__ void score_loop(Lds& L, uint32_t nu, uint64_t base, int perceptual, uint32_t wave)
+{
+    SearchLds& q = L.u.q;
+    for (;;) {
+        __syncthreads();
+        const uint32_t cmd = uni(q.cmd);
+        if (!cmd) return;
+        score<Lds, W>(L, q, nu, base, perceptual, cmd & 0xFFu, (int)(cmd >> 8), wave);
+        __syncthreads();
+    }
+}
+
+// evaluate_solution's plane lower bound (crn_dxt1.cpp:1312-1340)
+__device__ inline uint64_t plane_bound(const Bounds& B, uint32_t lo, uint32_t hi)
+{
+    int ar, ag, ab, br, bg, bb;
+    unpack565(lo, 0, ar, ag, ab);
+    unpack565(hi, 0, br, bg, bb);
+    return B.rlo[min(ar, br)] + B.rhi[max(ar, br)] + B.glo[min(ag, bg)] + B.ghi[max(ag, bg)] + B.blo[min(ab, bb)] +
+           B.bhi[max(ab, bb)];
+}
+
+__device__ inline int clampi(int v, int hi) { return v < 0 ? 0 : (v > hi ? hi : v); }
+
+// ------------------------------------------------------------ candidate lists
+enum ListKind : uint32_t {
+    kListPair,      // list[0][0..3]: the six pairs of four colours, canonical order
+    kListRefine,    // refine_solution level 1: 27 moves of either endpoint
+    kListSweep,     // list[0] x list[1], canonical order; index low * 32 + high
+    kListAdj0,      // 26 neighbours of the low / high end (the other end is the current best's)
+    kListAdj1,
+    kListAxis0,     // +-2 on each component of the low / high end
+    kListAxis1,
+    kListSolid,     // the average colour (list[0][0]) and each colour as a solid block
+    kListComb,      // list[0][i], list[0][j], i < j < fixed[0][0]; index i * 64 + j
+    kListComp0,     // optimize_endpoint_comps, one component: c0 * 64 + c1
+    kListComp1,
+    kListComp2,
+};
+
+__device__ inline uint32_t expand_comp(int comp, uint32_t c)
+{
+    return comp == 1 ? (((c << 2) | (c >> 4)) & 0xFF) : (((c << 3) | (c >> 2)) & 0xFF);
+}
+
+// Candidate `i` of the list; false: the list has none there.
+template <class Lds>
+__device__ inline bool list_candidate(const St& s, const Lds& L, const SearchLds& q, uint32_t kind, uint32_t i,
+                                      uint32_t from, uint32_t& lo, uint32_t& hi)
+{
+    switch (kind) {
+    case kListPair: {
+        const uint32_t a = i < 3 ? 0 : i < 5 ? 1 : 2, b = i < 3 ? i + 1 : i < 5 ? i - 1 : 3;
+        lo = q.list[0][a];
+        hi = q.list[0][b];
+        canon(lo, hi);
+        return true;
+    }
+    case kListRefine: {
+        const uint32_t e = i >= 27 ? 1 : 0, m = i - 27 * e;
+        uint32_t c[2];
+        for (uint32_t k = 0; k < 2; k++) {
+            const int d = e == k ? 1 : 0;
+            c[k] = pack565(clampi(q.fixed[k][0] + d * ((int)(m / 9) - 1), 31),
+                           clampi(q.fixed[k][1] + d * ((int)(m / 3 % 3) - 1), 63),
+                           clampi(q.fixed[k][2] + d * ((int)(m % 3) - 1), 31), 0);
+        }
+        lo = c[0];
+        hi = c[1];
+        canon(lo, hi);
+        return true;
+    }
+    case kListSweep:
+        if ((i & 31u) >= (uint32_t)q.fixed[0][0]) return false;
+        lo = q.list[0][i >> 5];
+        hi = q.list[1][i & 31u];
+        canon(lo, hi);
+        return true;
+    case kListAdj0:
+    case kListAdj1:
+    case kListAxis0:
+    case kListAxis1: {
+        int c[3];
+        unpack565(from, 0, c[0], c[1], c[2]);
+        if (kind <= kListAdj1) {
+            for (int k = 0; k < 3; k++) c[k] += c_adj[min(i, 25u)][k];
+        } else {
+            const int d = (i & 1u) ? 2 : -2;
+            for (uint32_t k = 0; k < 3; k++) c[k] += i >> 1 == k ? d : 0;
+        }
+        if (c[0] < 0 || c[0] > 31 || c[1] < 0 || c[1] > 63 || c[2] < 0 || c[2] > 31) return false;
+        lo = pack565(c[0], c[1], c[2], 0);
+        hi = kind == kListAdj0 || kind == kListAxis0 ? s.best.hi : s.best.lo;
+        canon(lo, hi);
+        return true;
+    }
+    case kListSolid: {
+        const uint32_t k = Lds::kUber ? i >> 1 : i;
+        const uint32_t avg = q.list[0][0];
+        const uint32_t c = k ? L.col[min(k, s.nu) - 1] : avg;
+        if (k && c == avg) return false;
+        const uint32_t r = c & 255u, g = (c >> 8) & 255u, b = (c >> 16) & 255u;
+        const uint8_t(*o5)[2] = Lds::kUber && (i & 1u) ? g_c_om5_3 : g_c_om5;
+        const uint8_t(*o6)[2] = Lds::kUber && (i & 1u) ? g_c_om6_3 : g_c_om6;
+        lo = ((uint32_t)o5[r][0] << 11) | ((uint32_t)o6[g][0] << 5) | o5[b][0];
+        hi = ((uint32_t)o5[r][1] << 11) | ((uint32_t)o6[g][1] << 5) | o5[b][1];
+        return true;
+    }
+    case kListComb:
+        if ((i & 63u) <= i >> 6 || (i & 63u) >= (uint32_t)q.fixed[0][0]) return false;
+        lo = q.list[0][i >> 6];
+        hi = q.list[0][i & 63u];
+        return true;
+    default: {
+        // optimize_endpoint_comps (crn_dxt1.cpp:420-486), one component
+        const int comp = (int)(kind - kListComp0);
+        const uint32_t c0 = i >> 6, c1 = i & 63u, lim = comp == 1 ? 64 : 32;
+        if (c1 >= lim) return false;
+        const uint32_t p0 = expand_comp(comp, c0), p1 = expand_comp(comp, c1);
+        const uint64_t best = q.qbest, e0 = q.q.at(0, p0);
+        if (e0 + q.brem[1] >= best) return false;
+        uint64_t e = e0 + q.q.at(1, p1);
+        if (e + q.brem[2] >= best) return false;
+        e += q.q.at(2, (p0 * 2 + p1) / 3);
+        if (e + q.brem[3] >= best) return false;
+        e += q.q.at(3, (p0 + p1 * 2) / 3);
+        if (e >= best) return false;
+        int a[3], b[3];
+        for (int k = 0; k < 3; k++) {
+            a[k] = k == comp ? (int)c0 : q.fixed[0][k];
+            b[k] = k == comp ? (int)c1 : q.fixed[1][k];
+        }
+        lo = pack565(a[0], a[1], a[2], 0);
+        hi = pack565(b[0], b[1], b[2], 0);
+        return true;
+    }
+    }
+}
+
+// Tries the list's candidates [first, n) in order from `first`: gathers a
+// batch, scores it, takes what the reference takes.  With `again`, returns at
+// the first candidate taken (first: the place after it).  True: one was taken.
+template <class Lds, uint32_t W>
+__device__ bool try_list(St& s, Lds& L, uint32_t kind, uint32_t n, int alt, bool again, uint32_t from, uint32_t& first)
+{
+    constexpr uint32_t kBatch = kBatchOf<W>;
+    SearchLds& q = L.u.q;
+    const uint32_t lane = lane_id();
     bool took = false;
-    if (!s.have_alpha && e4 < terr) {
-        terr = e4;
-        took = true;
-    }
-    if (e3 < terr) {
-        terr = e3;
-        talpha = 1;
-        took = true;
-    }
-    if (!took || terr >= s.best.err) return false;
-    s.best.lo = lo;
-    s.best.hi = hi;
-    s.best.err = terr;
-    s.best.alpha = talpha;
-    s.best.alt = alt;
-    s.best.enforce = !talpha && lo == hi;
-    if (s.best.enforce) {
-        if ((s.best.lo & 31) != 31) {
-            s.best.lo++;
-            s.best.enforced = 1;
+    while (first < n && s.best.err) {
+        uint32_t cnt = 0, next = first;
+        while (next < n && cnt < kBatch) {
+            const uint32_t i = next + lane;
+            uint32_t lo = 0, hi = 0;
+            bool ok = i < n && list_candidate(s, L, q, kind, i, from, lo, hi);
+            uint64_t b = 0;
+            if (ok) {
+                b = plane_bound(L.b, lo, hi);
+                ok = b < s.best.err;
+            }
+            const uint64_t mask = __ballot(ok);
+            const uint32_t at = cnt + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+            if (ok && at < kBatch) {
+                q.cand[at] = lo | (hi << 16);
+                q.cidx[at] = i;
+                q.bnd[at] = b;
+            }
+            cnt += (uint32_t)__popcll(mask);
+            next += 64;
+        }
+        if (!cnt) {
+            first = n;
+            break;
+        }
+        if (cnt > kBatch) cnt = kBatch;
+        if (lane == 0) q.cmd = cnt | ((uint32_t)alt << 8);
+        __builtin_amdgcn_wave_barrier();
+        if (cnt == kBatch) next = uni(q.cidx[kBatch - 1]) + 1;
+        if constexpr (W > 1) __syncthreads();
+        score<Lds, W>(L, q, s.nu, s.base, s.perceptual, cnt, alt, 0);
+        if constexpr (W > 1) __syncthreads();
+        else __builtin_amdgcn_wave_barrier();
+        // lane k: candidate k's error, block type and the larger of error and bound
+        const uint32_t k = min(lane, cnt - 1);
+        uint64_t e;
+        uint32_t alpha = 0;
+        if constexpr (Lds::kUber) {
+            const uint64_t e4 = q.err[2 * k], e3 = q.err[2 * k + 1];
+            alpha = s.have_alpha || e3 < e4 ? 1u : 0u;
+            e = alpha ? e3 : e4;
         } else {
-            s.best.hi--;
-            s.best.enforced = 0;
+            e = q.err[k];
+        }
+        const uint64_t bk = q.bnd[k];
+        const uint64_t m = e > bk ? e : bk;
+        const uint32_t c = q.cand[k];
+        uint64_t left = ~0ull;
+        first = next;
+        for (;;) {
+            const uint64_t mask = __ballot(lane < cnt && m < s.best.err) & left;
+            if (!mask) break;
+            const uint32_t t = (uint32_t)__builtin_ctzll(mask);
+            const uint32_t lh = lane_u32(c, t);
+            s.best.lo = lh & 0xFFFFu;
+            s.best.hi = lh >> 16;
+            s.best.err = lane_u64(e, t);
+            s.best.alt = alt;
+            s.best.alpha = Lds::kUber ? (int)lane_u32(alpha, t) : 0;
+            s.best.enforce = !s.best.alpha && s.best.lo == s.best.hi;
+            if (s.best.enforce) {
+                if ((s.best.lo & 31) != 31) {
+                    s.best.lo++;
+                    s.best.enforced = 1;
+                } else {
+                    s.best.hi--;
+                    s.best.enforced = 0;
+                }
+            }
+            s.sel_valid = false;
+            if (Lds::kUber) s.sel_nonempty = true;
+            took = true;
+            if (again) {
+                first = uni(q.cidx[t]) + 1;
+                return true;
+            }
+            left = t == 63 ? 0ull : ~0ull << (t + 1);
         }
     }
-    s.sel_valid = false;
-    s.sel_nonempty = true;
-    return true;
+    return took;
 }
 
-// compute_selectors_hc (crn_dxt1.cpp:1837-1869)
+// The selector of a colour: compute_selectors_hc (crn_dxt1.cpp:1837-1869), or
+// with `three` the 3-colour palette's first nearest entry (evaluate_solution_uber).
+__device__ inline uint32_t nearest(const Pal& p, int perceptual, bool three, uint32_t px)
+{
+    const uint32_t e0 = cdist(perceptual, px, p.r[0], p.g[0], p.b[0]);
+    const uint32_t e1 = cdist(perceptual, px, p.r[1], p.g[1], p.b[1]);
+    const uint32_t e2 = cdist(perceptual, px, p.r[2], p.g[2], p.b[2]);
+    if (three) return e1 < e0 ? (e2 < e1 ? 2 : 1) : (e2 < e0 ? 2 : 0);
+    const uint32_t e3 = cdist(perceptual, px, p.r[3], p.g[3], p.b[3]);
+    const uint32_t e01 = min(e0, e1), e23 = min(e2, e3);
+    return e01 <= e23 ? (e01 == e0 ? 0 : 1) : (e23 == e2 ? 2 : 3);
+}
+
+// The best solution's selectors of the unique colours.
 template <class Lds>
 __device__ void compute_selectors(St& s, Lds& L)
 {
     if (s.sel_valid) return;
-    if (s.best.enforce) {
-        for (uint32_t i = lane_id(); i < s.nu; i += 64) L.sel[i] = (uint8_t)s.best.enforced;
-    } else if (Lds::kUber && s.best.alpha) {
-        // the 3-colour palette's first nearest entry (evaluate_solution_uber)
-        const Pal p = palette3(s.best.lo, s.best.hi, s.best.alt);
-        for (uint32_t i = lane_id(); i < s.nu; i += 64) {
-            const uint32_t px = L.col[i];
-            const uint32_t e0 = cdist(s.perceptual, px, p.r[0], p.g[0], p.b[0]);
-            const uint32_t e1 = cdist(s.perceptual, px, p.r[1], p.g[1], p.b[1]);
-            const uint32_t e2 = cdist(s.perceptual, px, p.r[2], p.g[2], p.b[2]);
-            L.sel[i] = (uint8_t)(e1 < e0 ? (e2 < e1 ? 2 : 1) : (e2 < e0 ? 2 : 0));
-        }
-    } else {
-        const Pal p = palette4(s.best.lo, s.best.hi, s.best.alt);
-        for (uint32_t i = lane_id(); i < s.nu; i += 64) {
-            const uint32_t px = L.col[i];
-            const uint32_t e0 = cdist(s.perceptual, px, p.r[0], p.g[0], p.b[0]);
-            const uint32_t e1 = cdist(s.perceptual, px, p.r[1], p.g[1], p.b[1]);
-            const uint32_t e2 = cdist(s.perceptual, px, p.r[2], p.g[2], p.b[2]);
-            const uint32_t e3 = cdist(s.perceptual, px, p.r[3], p.g[3], p.b[3]);
-            const uint32_t e01 = min(e0, e1), e23 = min(e2, e3);
-            L.sel[i] = (uint8_t)(e01 <= e23 ? (e01 == e0 ? 0 : 1) : (e23 == e2 ? 2 : 3));
-        }
-    }
+    const bool three = Lds::kUber && s.best.alpha;
+    const Pal p = three ? palette3(s.best.lo, s.best.hi, s.best.alt) : palette4(s.best.lo, s.best.hi, s.best.alt);
+    for (uint32_t i = lane_id(); i < s.nu; i += 64)
+        L.sel[i] = (uint8_t)(s.best.enforce ? (uint32_t)s.best.enforced : nearest(p, s.perceptual, three, L.col[i]));
     __builtin_amdgcn_wave_barrier();
     s.sel_valid = true;
     s.sel_nonempty = true;
 }
 
-// evaluate_solution with the plane lower bound (crn_dxt1.cpp:1312-1340); the
-// bound only skips candidates that cannot win.
-template <class Lds>
-__device__ bool evaluate(St& s, Lds& L, uint32_t lo, uint32_t hi, int alt)
+// --------------------------------------------------- sequential float sums
+// Lane k < K adds row k's 64 staged terms to its sum, one after another.
+__device__ inline float add_row(const float* row, float a)
 {
-    int ar, ag, ab, br, bg, bb;
-    unpack565(lo, 0, ar, ag, ab);
-    unpack565(hi, 0, br, bg, bb);
-    const uint64_t re = ar < br ? L.rlo[ar] + L.rhi[br] : L.rhi[ar] + L.rlo[br];
-    const uint64_t ge = ag < bg ? L.glo[ag] + L.ghi[bg] : L.ghi[ag] + L.glo[bg];
-    const uint64_t be = ab < bb ? L.blo[ab] + L.bhi[bb] : L.bhi[ab] + L.blo[bb];
-    if (re + ge + be >= s.best.err) return false;
-    if constexpr (Lds::kUber) return eval_uber(s, L, lo, hi, alt);
-    else return eval_hc(s, L, lo, hi, alt);
+#pragma unroll
+    for (uint32_t j = 0; j < 64; j += 4) {
+        const float4 v = *reinterpret_cast<const float4*>(row + j);
+        a += v.x;
+        a += v.y;
+        a += v.z;
+        a += v.w;
+    }
+    return a;
 }
 
-template <class Lds>
-__device__ inline bool eval_canon(St& s, Lds& L, uint32_t lo, uint32_t hi)
+__device__ inline double add_row(const double* row, double a)
 {
-    canon(lo, hi);
-    return evaluate(s, L, lo, hi, 0);
+#pragma unroll
+    for (uint32_t j = 0; j < 64; j += 2) {
+        const double2 v = *reinterpret_cast<const double2*>(row + j);
+        a += v.x;
+        a += v.y;
+    }
+    return a;
 }
 
-__device__ inline int clampi(int v, int hi) { return v < 0 ? 0 : (v > hi ? hi : v); }
-
-// normalised (and perceptually weighted) colour i minus the mean, as
+// normalised (and perceptually weighted) colour minus the mean, as
 // compute_vectors stores it (crn_dxt1.cpp:155-189)
-template <class Lds>
-__device__ inline void norm_of(const St& s, const Lds& L, uint32_t i, float* n, float* nw)
+__device__ inline void norm_of(const St& s, uint32_t c, float* n, float* nw)
 {
-    const uint32_t c = L.col[i];
     for (int k = 0; k < 3; k++) {
         const float v = (float)((c >> (8 * k)) & 255u) * 1.0f / 255.0f;
         n[k] = v - s.mean[k];
@@ -365,45 +692,59 @@ __device__ inline void norm_of(const St& s, const Lds& L, uint32_t i, float* n, 
 }
 
 template <class Lds>
-__device__ void compute_vectors(St& s, const Lds& L)
+__device__ void compute_vectors(St& s, Lds& L)
 {
-    for (int k = 0; k < 3; k++) s.mean[k] = s.meanw[k] = 0.0f;
-    for (uint32_t i = 0; i < s.nu; i++) {
-        const uint32_t c = L.col[i];
+    const uint32_t lane = lane_id();
+    float(*f)[kRow] = L.u.q.stage.f;
+    float acc = 0.0f;
+    for (uint32_t i0 = 0; i0 < s.nu; i0 += 64) {
+        const uint32_t i = min(i0 + lane, s.nu - 1), c = L.col[i];
+        const bool in = i0 + lane < s.nu;
         const float w = (float)L.w[i];
         for (int k = 0; k < 3; k++) {
             const float v = (float)((c >> (8 * k)) & 255u) * 1.0f / 255.0f;
-            s.mean[k] += v * w;
-            s.meanw[k] += (s.pw[k] * v) * w;
+            f[k][lane] = in ? v * w : 0.0f;
+            f[3 + k][lane] = in ? (s.pw[k] * v) * w : 0.0f;
         }
+        __builtin_amdgcn_wave_barrier();
+        acc = add_row(f[min(lane, 5u)], acc);
+        __builtin_amdgcn_wave_barrier();
+    }
+    for (uint32_t k = 0; k < 3; k++) {
+        s.mean[k] = lane_f32(acc, k);
+        s.meanw[k] = lane_f32(acc, 3 + k);
     }
     if (s.total_w) {
         const float inv = 1.0f / (float)s.total_w;
         for (int k = 0; k < 3; k++) {
-            s.mean[k] *= inv;
-            s.meanw[k] *= inv;
+            s.mean[k] = unif(s.mean[k] * inv);
+            s.meanw[k] = unif(s.meanw[k] * inv);
         }
     }
 }
 
 // compute_pca (crn_dxt1.cpp:192-256) over the weighted vectors
 template <class Lds>
-__device__ void compute_pca(St& s, const Lds& L, float* axis)
+__device__ void compute_pca(St& s, Lds& L, float* axis)
 {
-    double cov[6] = {0, 0, 0, 0, 0, 0};
-    for (uint32_t i = 0; i < s.nu; i++) {
+    const uint32_t lane = lane_id();
+    double(*d)[kRowD] = L.u.q.stage.d;
+    double acc = 0.0;
+    for (uint32_t i0 = 0; i0 < s.nu; i0 += 64) {
+        const uint32_t i = min(i0 + lane, s.nu - 1), wi = L.w[i];
+        const bool in = i0 + lane < s.nu;
         float n[3], nw[3];
-        norm_of(s, L, i, n, nw);
+        norm_of(s, L.col[i], n, nw);
         const float r = nw[0], g = nw[1], b = nw[2];
-        if (L.w[i] > 1) {
-            const double w = L.w[i];
-            cov[0] += r * r * w; cov[1] += r * g * w; cov[2] += r * b * w;
-            cov[3] += g * g * w; cov[4] += g * b * w; cov[5] += b * b * w;
-        } else {
-            cov[0] += r * r; cov[1] += r * g; cov[2] += r * b;
-            cov[3] += g * g; cov[4] += g * b; cov[5] += b * b;
-        }
+        const float t[6] = {r * r, r * g, r * b, g * g, g * b, b * b};
+        const double w = (double)wi;
+        for (int k = 0; k < 6; k++) d[k][lane] = !in ? 0.0 : wi > 1 ? t[k] * w : (double)t[k];
+        __builtin_amdgcn_wave_barrier();
+        acc = add_row(d[min(lane, 5u)], acc);
+        __builtin_amdgcn_wave_barrier();
     }
+    double cov[6];
+    for (uint32_t k = 0; k < 6; k++) cov[k] = lane_f64(acc, k);
     double vr = .9f, vg = 1.0f, vb = .7f;
     for (int it = 0; it < 8; it++) {
         double r = vr * cov[0] + vg * cov[1] + vb * cov[2];
@@ -418,11 +759,11 @@ __device__ void compute_pca(St& s, const Lds& L, float* axis)
             g *= m;
             b *= m;
         }
-        const double d = (vr - r) * (vr - r) + (vg - g) * (vg - g) + (vb - b) * (vb - b);
+        const double dd = (vr - r) * (vr - r) + (vg - g) * (vg - g) + (vb - b) * (vb - b);
         vr = r;
         vg = g;
         vb = b;
-        if (it > 2 && d < 1e-8) break;
+        if (it > 2 && dd < 1e-8) break;
     }
     double len = vr * vr + vg * vg + vb * vb;
     if (len < 1e-10) {
@@ -444,6 +785,7 @@ __device__ bool ray_unit_box(float* coord, const float* org, const float* dir)
     int quad[3];
     float cand[3], maxt[3];
     for (int i = 0; i < 3; i++) {
+        cand[i] = 0.0f;
         if (org[i] < 0.0f) { quad[i] = 1; cand[i] = 0.0f; inside = false; }
         else if (org[i] > 1.0f) { quad[i] = 0; cand[i] = 1.0f; inside = false; }
         else quad[i] = 2;
@@ -451,13 +793,17 @@ __device__ bool ray_unit_box(float* coord, const float* org, const float* dir)
     if (inside) return false;
     for (int i = 0; i < 3; i++) maxt[i] = (quad[i] != 2 && dir[i] != 0.0f) ? (cand[i] - org[i]) / dir[i] : -1.0f;
     int wp = 0;
+    float wt = maxt[0];
     for (int i = 1; i < 3; i++)
-        if (maxt[wp] < maxt[i]) wp = i;
-    if (maxt[wp] < 0.0f) return false;
+        if (wt < maxt[i]) {
+            wp = i;
+            wt = maxt[i];
+        }
+    if (wt < 0.0f) return false;
     float c[3];
     for (int i = 0; i < 3; i++) {
         if (i != wp) {
-            c[i] = org[i] + maxt[wp] * dir[i];
+            c[i] = org[i] + wt * dir[i];
             if (c[i] < 0.0f || c[i] > 1.0f) return false;
         } else {
             c[i] = cand[i];
@@ -467,11 +813,12 @@ __device__ bool ray_unit_box(float* coord, const float* org, const float* dir)
     return true;
 }
 
-// refine_solution (crn_dxt1.cpp:525-698), levels 0 and 1.  The sums are of
-// integers times integer weights (exact in double), so a lane-split sum is
+// refine_solution's least squares (crn_dxt1.cpp:525-600): the rounded
+// endpoints into q.fixed; false when the system has no solution.  The sums are
+// of integers times integer weights (exact in double), so a lane-split sum is
 // the reference's value.
 template <class Lds>
-__device__ bool refine(St& s, Lds& L, int level)
+__device__ bool refine_fit(St& s, Lds& L)
 {
     compute_selectors(s, L);
     uint64_t A0 = 0, A1 = 0, A2 = 0, T1[3] = {0, 0, 0}, T2[3] = {0, 0, 0};
@@ -502,7 +849,7 @@ __device__ bool refine(St& s, Lds& L, int level)
     }
     const double xx = (double)A2, yy = (double)A1, xy = (double)A0;
     const double t = xx * yy - xy * xy;
-    if (!yy || !xx || fabs(t) < (double).0000125f) return false;
+    if (unib(!yy || !xx || fabs(t) < (double).0000125f)) return false;
     const double frb = (double)(3.0f * 31.0f / 255.0f) / t;
     const double fg = frb * (double)(63.0f / 31.0f);
     int e0[3], e1[3];
@@ -512,24 +859,13 @@ __device__ bool refine(St& s, Lds& L, int level)
     e1[0] = clampi((int)((t2[0] * xx - t1[0] * xy) * frb + (double)0.5f), 31);
     e1[1] = clampi((int)((t2[1] * xx - t1[1] * xy) * fg + (double)0.5f), 63);
     e1[2] = clampi((int)((t2[2] * xx - t1[2] * xy) * frb + (double)0.5f), 31);
-    bool improved = false;
-    if (level == 0) {
-        improved |= eval_canon(s, L, (uint32_t)((e1[0] << 11) | (e1[1] << 5) | e1[2]),
-                               (uint32_t)((e0[0] << 11) | (e0[1] << 5) | e0[2]));
-    } else {
-        for (int i = 0; i < 2; i++)
-            for (int rr = -1; rr <= 1; rr++)
-                for (int gr = -1; gr <= 1; gr++)
-                    for (int br = -1; br <= 1; br++) {
-                        int c0[3] = {e0[0], e0[1], e0[2]}, c1[3] = {e1[0], e1[1], e1[2]};
-                        int* c = i ? c1 : c0;
-                        c[0] = clampi(c[0] + rr, 31);
-                        c[1] = clampi(c[1] + gr, 63);
-                        c[2] = clampi(c[2] + br, 31);
-                        improved |= eval_canon(s, L, pack565(c0[0], c0[1], c0[2], 0), pack565(c1[0], c1[1], c1[2], 0));
-                    }
-    }
-    return improved;
+    if (lane_id() == 0)
+        for (int k = 0; k < 3; k++) {
+            L.u.q.fixed[0][k] = e0[k];
+            L.u.q.fixed[1][k] = e1[k];
+        }
+    __builtin_amdgcn_wave_barrier();
+    return true;
 }
 
 // fast_random (crn_rand.cpp:310-405)
@@ -551,16 +887,19 @@ struct FastRandom {
     }
 };
 
-// try_median4 (crn_dxt1.cpp:1181-1308): 4-means over the colours (sequential
-// float sums), then the six pairs of means and refine_solution.
+// try_median4's means (crn_dxt1.cpp:1181-1290): 4-means over the colours with
+// sequential float sums (lane 4 j + k: mean j's component k, k = 3 its weight;
+// lane 16: the total distance); the four means as 5:6:5 colours into q.list.
 template <class Lds>
-__device__ bool try_median4(St& s, Lds& L, const float* lo, const float* hi)
+__device__ void median4(St& s, Lds& L, const float* lo, const float* hi)
 {
+    const uint32_t lane = lane_id();
+    SearchLds& q = L.u.q;
     float means[4][3];
     if (s.nu <= 4) {
-        for (int i = 0; i < 4; i++) {
+        for (uint32_t i = 0; i < 4; i++) {
             float n[3], nw[3];
-            norm_of(s, L, (uint32_t)i < s.nu - 1 ? (uint32_t)i : s.nu - 1, n, nw);
+            norm_of(s, L.col[min(i, s.nu - 1)], n, nw);
             for (int k = 0; k < 3; k++) means[i][k] = n[k];
         }
     } else {
@@ -575,19 +914,23 @@ __device__ bool try_median4(St& s, Lds& L, const float* lo, const float* hi)
         FastRandom rm;
         uint32_t rover = 0;
         float prev = 1.0e+37f;
+        float(*f)[kRow] = q.stage.f;
         for (uint32_t it = 0; it < 8; it++) {
-            float nm[4][3] = {}, nwt[4] = {0, 0, 0, 0};
-            float total = 0;
-            for (uint32_t i = 0; i < s.nu; i++) {
+            float acc = 0.0f;
+            const uint32_t mine = min(lane >> 2, 4u);
+            const float* row = f[lane < 16 ? lane & 3u : 4u];
+            for (uint32_t i0 = 0; i0 < s.nu; i0 += 64) {
+                const uint32_t i = min(i0 + lane, s.nu - 1);
+                const bool in = i0 + lane < s.nu;
                 float v[3], vw[3];
-                norm_of(s, L, i, v, vw);
+                norm_of(s, L.col[i], v, vw);
                 float bd = 0;
                 for (int k = 0; k < 3; k++) {
                     const float d = means[0][k] - v[k];
                     bd += d * d;
                 }
-                int bi = 0;
-                for (int jj = 1; jj < 4; jj++) {
+                uint32_t bi = 0;
+                for (uint32_t jj = 1; jj < 4; jj++) {
                     float dd = 0;
                     for (int k = 0; k < 3; k++) {
                         const float d = means[jj][k] - v[k];
@@ -598,56 +941,68 @@ __device__ bool try_median4(St& s, Lds& L, const float* lo, const float* hi)
                         bi = jj;
                     }
                 }
-                total += bd;
                 const float w = (float)L.w[i];
-                for (int k = 0; k < 3; k++) nm[bi][k] += v[k] * w;
-                nwt[bi] += w;
+                for (int k = 0; k < 3; k++) f[k][lane] = v[k] * w;
+                f[3][lane] = w;
+                f[4][lane] = in ? bd : 0.0f;
+                f[5][lane] = __builtin_bit_cast(float, in ? bi : 7u);
+                __builtin_amdgcn_wave_barrier();
+                // a term of another mean adds +0, which changes no sum (none is -0)
+#pragma unroll 4
+                for (uint32_t j = 0; j < 64; j += 4) {
+                    const float4 x = *reinterpret_cast<const float4*>(row + j);
+                    const uint4 b = *reinterpret_cast<const uint4*>(&f[5][j]);
+                    const bool all = mine == 4u;
+                    acc += all || b.x == mine ? x.x : 0.0f;
+                    acc += all || b.y == mine ? x.y : 0.0f;
+                    acc += all || b.z == mine ? x.z : 0.0f;
+                    acc += all || b.w == mine ? x.w : 0.0f;
+                }
+                __builtin_amdgcn_wave_barrier();
             }
+            const float total = lane_f32(acc, 16);
             uint32_t hidx = 0;
             float hw = 0;
             bool empty = false;
-            for (int jj = 0; jj < 4; jj++) {
+            float nwt[4];
+            for (uint32_t jj = 0; jj < 4; jj++) {
+                nwt[jj] = lane_f32(acc, 4 * jj + 3);
                 if (nwt[jj] > 0.0f) {
-                    for (int k = 0; k < 3; k++) means[jj][k] = nm[jj][k] / nwt[jj];
+                    for (uint32_t k = 0; k < 3; k++) means[jj][k] = lane_f32(acc, 4 * jj + k) / nwt[jj];
                     if (nwt[jj] > hw) {
                         hw = nwt[jj];
-                        hidx = (uint32_t)jj;
+                        hidx = jj;
                     }
                 } else {
                     empty = true;
                 }
             }
             if (!empty) {
-                if (fabsf(total - prev) < .00001f) break;
+                if (unib(fabsf(total - prev) < .00001f)) break;
                 prev = total;
             } else {
                 prev = 1.0e+37f;
             }
-            if (empty && it != 7) {
+            if (unib(empty) && it != 7) {
                 const uint32_t ri = (hidx + rover) & 3u;
                 rover++;
-                for (int jj = 0; jj < 4; jj++)
+                for (uint32_t jj = 0; jj < 4; jj++)
                     if (nwt[jj] == 0.0f)
-                        for (int k = 0; k < 3; k++) means[jj][k] = means[ri][k] + rm.frand(-.00196f, .00196f);
+                        for (int k = 0; k < 3; k++) {
+                            const float src = ri == 0 ? means[0][k] : ri == 1 ? means[1][k] : ri == 2 ? means[2][k] : means[3][k];
+                            means[jj][k] = src + rm.frand(-.00196f, .00196f);
+                        }
             }
         }
     }
-    bool improved = false;
-    for (int i = 0; i < 3; i++)
-        for (int jj = i + 1; jj < 4; jj++) {
-            float a[3], b[3];
-            for (int k = 0; k < 3; k++) {
-                a[k] = means[i][k] + s.mean[k];
-                b[k] = means[jj][k] + s.mean[k];
-            }
-            uint32_t lo2 = pack565((int)floorf(.5f + a[0] * 31.0f), (int)floorf(.5f + a[1] * 63.0f),
+    if (lane == 0)
+        for (int i = 0; i < 4; i++) {
+            float a[3];
+            for (int k = 0; k < 3; k++) a[k] = means[i][k] + s.mean[k];
+            q.list[0][i] = pack565((int)floorf(.5f + a[0] * 31.0f), (int)floorf(.5f + a[1] * 63.0f),
                                    (int)floorf(.5f + a[2] * 31.0f), 0);
-            uint32_t hi2 = pack565((int)floorf(.5f + b[0] * 31.0f), (int)floorf(.5f + b[1] * 63.0f),
-                                   (int)floorf(.5f + b[2] * 31.0f), 0);
-            improved |= eval_canon(s, L, lo2, hi2);
         }
-    improved |= refine(s, L, 1);
-    return improved;
+    __builtin_amdgcn_wave_barrier();
 }
 
 // are_selectors_all_equal (crn_dxt1.h:300-316) on the best solution's
@@ -658,14 +1013,14 @@ template <class Lds>
 __device__ bool sel_all_equal(const St& s, const Lds& L)
 {
     if (!s.sel_nonempty) return false;
-    uint32_t diff = 0;
+    bool diff = false;
     for (uint32_t i = lane_id(); i < s.nu; i += 64) diff |= L.sel[i] != L.sel[0];
-    return wave_sum(diff) == 0;
+    return __ballot(diff) == 0;
 }
 
-// try_average_block_as_solid (crn_dxt1.cpp:93-153), uber branch
+// The average colour of try_average_block_as_solid (crn_dxt1.cpp:93-153)
 template <class Lds>
-__device__ bool try_average_solid(St& s, Lds& L)
+__device__ uint32_t average_colour(St& s, Lds& L)
 {
     uint64_t tr = 0, tg = 0, tb = 0, tw = 0;
     for (uint32_t i = lane_id(); i < s.nu; i += 64) {
@@ -681,53 +1036,28 @@ __device__ bool try_average_solid(St& s, Lds& L)
     tg = wave_sum(tg);
     tb = wave_sum(tb);
     const uint64_t half = tw >> 1;
-    const uint32_t ar = (uint32_t)((tr + half) / tw), ag = (uint32_t)((tg + half) / tw), ab = (uint32_t)((tb + half) / tw);
-    bool improved = evaluate(s, L, (g_c_om5[ar][0] << 11) | (g_c_om6[ag][0] << 5) | g_c_om5[ab][0],
-                             (g_c_om5[ar][1] << 11) | (g_c_om6[ag][1] << 5) | g_c_om5[ab][1], 0);
-    if (Lds::kUber && s.best.err)
-        improved |= evaluate(s, L, (g_c_om5_3[ar][0] << 11) | (g_c_om6_3[ag][0] << 5) | g_c_om5_3[ab][0],
-                             (g_c_om5_3[ar][1] << 11) | (g_c_om6_3[ag][1] << 5) | g_c_om5_3[ab][1], 0);
-    for (uint32_t i = 0; i < s.nu; i++) {
-        const uint32_t c = L.col[i];
-        const uint32_t r = c & 255u, g = (c >> 8) & 255u, b = (c >> 16) & 255u;
-        if (r == ar && g == ag && b == ab) continue;
-        improved |= evaluate(s, L, (g_c_om5[r][0] << 11) | (g_c_om6[g][0] << 5) | g_c_om5[b][0],
-                             (g_c_om5[r][1] << 11) | (g_c_om6[g][1] << 5) | g_c_om5[b][1], 0);
-        if (Lds::kUber && s.best.err)
-            improved |= evaluate(s, L, (g_c_om5_3[r][0] << 11) | (g_c_om6_3[g][0] << 5) | g_c_om5_3[b][0],
-                                 (g_c_om5_3[r][1] << 11) | (g_c_om6_3[g][1] << 5) | g_c_om5_3[b][1], 0);
-    }
-    return improved;
+    return (uint32_t)((tr + half) / tw) | (uint32_t)((tg + half) / tw) << 8 | (uint32_t)((tb + half) / tw) << 16;
 }
 
 // compute_endpoint_component_errors (crn_dxt1.cpp:369-418)
-// Per-channel error of one selector class as a function of the class's value
-// p: W p^2 - WP2 p + WPP (the reference's compute_endpoint_component_errors
-// tables, crn_dxt1.cpp:369-418, evaluated where they are read).
-struct QErr {
-    uint64_t W[4], WP2[4], WPP[4];
-    __device__ inline uint64_t at(int sl, uint64_t p) const { return W[sl] * p * p - WP2[sl] * p + WPP[sl]; }
-};
-
-__device__ inline uint32_t expand_comp(int comp, uint32_t c)
-{
-    return comp == 1 ? (((c << 2) | (c >> 4)) & 0xFF) : (((c << 3) | (c >> 2)) & 0xFF);
-}
-
 template <class Lds>
-__device__ void comp_errors(St& s, Lds& L, int comp, QErr& q, uint64_t* brem)
+__device__ void comp_errors(St& s, Lds& L, int comp)
 {
+    SearchLds& sq = L.u.q;
+    QErr q;
     uint64_t W[4] = {0, 0, 0, 0}, WP2[4] = {0, 0, 0, 0}, WPP[4] = {0, 0, 0, 0};
     for (uint32_t i = lane_id(); i < s.nu; i += 64) {
-        const uint64_t p = (L.col[i] >> (8 * comp)) & 255u;
-        const uint64_t w = L.w[i];
+        const uint32_t p = (L.col[i] >> (8 * comp)) & 255u;
+        const uint32_t w = L.w[i];
         const uint32_t sl = L.sel[i];
-        for (uint32_t k = 0; k < 4; k++)
-            if (k == sl) {
-                W[k] += w;
-                WP2[k] += w * p * 2;
-                WPP[k] += w * p * p;
-            }
+        const uint64_t w2 = (uint64_t)w * (2 * p), wpp = (uint64_t)w * (p * p);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) {
+            const bool on = k == sl;
+            W[k] += on ? w : 0u;
+            WP2[k] += on ? w2 : 0ull;
+            WPP[k] += on ? wpp : 0ull;
+        }
     }
     for (int k = 0; k < 4; k++) {
         q.W[k] = wave_sum(W[k]);
@@ -736,6 +1066,7 @@ __device__ void comp_errors(St& s, Lds& L, int comp, QErr& q, uint64_t* brem)
     }
     const uint32_t lane = lane_id();
     const uint32_t lim = comp == 1 ? 64 : 32;
+    uint64_t brem[4];
     for (int sl = 0; sl < 4; sl++) {
         const uint32_t n = sl < 2 ? lim : 256;
         uint64_t m = ~0ull;
@@ -745,243 +1076,133 @@ __device__ void comp_errors(St& s, Lds& L, int comp, QErr& q, uint64_t* brem)
             const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(m >> 32), off);
             m = min(m, ((uint64_t)hi << 32) | lo);
         }
-        brem[sl] = m;
+        brem[sl] = uni64(m);
     }
     for (int sl = 3; sl; sl--) brem[sl - 1] += brem[sl];
-}
-
-// optimize_endpoint_comps (crn_dxt1.cpp:420-486)
-template <class Lds>
-__device__ void optimize_comps(St& s, Lds& L)
-{
-    compute_selectors(s, L);
-    if (s.best.alpha || !s.best.err) return;
-    int slo[3], shi[3];
-    unpack565(s.best.lo, 1, slo[0], slo[1], slo[2]);
-    unpack565(s.best.hi, 1, shi[0], shi[1], shi[2]);
-    uint64_t brem[4];
-    QErr q;
-    for (int comp = 0; comp < 3; comp++) {
-        uint32_t p0 = (uint32_t)slo[comp], p1 = (uint32_t)shi[comp];
-        int low[3], high[3];
-        unpack565(s.best.lo, 0, low[0], low[1], low[2]);
-        unpack565(s.best.hi, 0, high[0], high[1], high[2]);
-        comp_errors(s, L, comp, q, brem);
-        uint64_t best = q.at(0, p0) + q.at(1, p1) + q.at(2, (p0 * 2 + p1) / 3) + q.at(3, (p0 + p1 * 2) / 3);
-        if (brem[0] >= best) continue;
-        const uint32_t lim = comp == 1 ? 64 : 32;
-        for (uint32_t c0 = 0; c0 < lim; c0++) {
-            p0 = expand_comp(comp, c0);
-            uint64_t e0 = q.at(0, p0);
-            if (e0 + brem[1] >= best) continue;
-            low[comp] = (int)c0;
-            const uint32_t plow = pack565(low[0], low[1], low[2], 0);
-            for (uint32_t c1 = 0; c1 < lim; c1++) {
-                p1 = expand_comp(comp, c1);
-                uint64_t e = e0 + q.at(1, p1);
-                if (e + brem[2] >= best) continue;
-                e += q.at(2, (p0 * 2 + p1) / 3);
-                if (e + brem[3] >= best) continue;
-                e += q.at(3, (p0 + p1 * 2) / 3);
-                if (e >= best) continue;
-                high[comp] = (int)c1;
-                if (!evaluate(s, L, plow, pack565(high[0], high[1], high[2], 0), 0)) continue;
-                if (!s.best.err) return;
-                compute_selectors(s, L);
-                comp_errors(s, L, comp, q, brem);
-                best = q.at(0, p0) + q.at(1, p1) + q.at(2, (p0 * 2 + p1) / 3) + q.at(3, (p0 + p1 * 2) / 3);
-                e0 = q.at(0, p0);
-                if (e0 + brem[1] >= best) break;
-            }
-        }
+    if (lane == 0) {
+        sq.q = q;
+        for (int sl = 0; sl < 4; sl++) sq.brem[sl] = brem[sl];
     }
+    __builtin_amdgcn_wave_barrier();
 }
 
-__device__ inline void lerp_color(int ar, int ag, int ab, int br, int bg, int bb, float f, int rounding, int& r,
-                                  int& g, int& b)
+// The component errors' sum at (p0, p1) into q.qbest.
+template <class Lds>
+__device__ void comp_best(Lds& L, uint32_t p0, uint32_t p1)
+{
+    SearchLds& q = L.u.q;
+    const uint64_t best = q.q.at(0, p0) + q.q.at(1, p1) + q.q.at(2, (p0 * 2 + p1) / 3) + q.q.at(3, (p0 + p1 * 2) / 3);
+    __builtin_amdgcn_wave_barrier();
+    if (lane_id() == 0) q.qbest = best;
+    __builtin_amdgcn_wave_barrier();
+}
+
+__device__ inline uint32_t lerp_color(uint32_t a, uint32_t b, float f, int rounding)
 {
     const float rr = rounding ? 1.0f : 0.0f;
-    r = clampi((int)(rr + ((float)ar + ((float)br - (float)ar) * f)), 255);
-    g = clampi((int)(rr + ((float)ag + ((float)bg - (float)ag) * f)), 255);
-    b = clampi((int)(rr + ((float)ab + ((float)bb - (float)ab) * f)), 255);
-}
-
-// try_combinatorial_encoding (crn_dxt1.cpp:1886-1997): 2 to 4 colours only
-template <class Lds>
-__device__ void try_combinatorial(St& s, Lds& L)
-{
-    if (s.nu < 2 || s.nu > 4) return;
-    int tr[52], tg[52], tb[52];
-    uint32_t n = 0;
-    for (uint32_t i = 0; i < s.nu; i++) {
-        const uint32_t c = L.col[i];
-        tr[n] = (int)(c & 255u);
-        tg[n] = (int)((c >> 8) & 255u);
-        tb[n] = (int)((c >> 16) & 255u);
-        n++;
-    }
-    if (s.nu == 2) {
-        const float fs[10] = {2.0f, 3.0f, .5f, 1.5f, -1.0f, 2.0f, -.5f, .5f, -2.0f, -1.0f};
-        for (int k = 0; k < 2; k++)
-            for (int q = 0; q < 2; q++) {
-                const int r = q ^ 1;
-                for (int f = 0; f < 10; f++) {
-                    lerp_color(tr[q], tg[q], tb[q], tr[r], tg[r], tb[r], fs[f], k, tr[n], tg[n], tb[n]);
-                    n++;
-                }
-            }
-    } else if (s.nu == 3) {
-        const float fs[4] = {1.5f, 2.0f / 3.0f, 1.0f / 3.0f, -.5f};
-        for (int i = 0; i <= 2; i++)
-            for (int jj = 0; jj <= 2; jj++) {
-                if (i == jj) continue;
-                for (int f = 0; f < 4; f++) {
-                    lerp_color(tr[i], tg[i], tb[i], tr[jj], tg[jj], tb[jj], fs[f], 1, tr[n], tg[n], tb[n]);
-                    n++;
-                }
-            }
-    }
-    uint32_t packed[64];
-    uint32_t np = 0;
-    for (uint32_t i = 0; i < n; i++) {
-        const uint32_t p = pack565(tr[i], tg[i], tb[i], 1);
-        bool dup = false;
-        for (uint32_t k = 0; k < np; k++)
-            if (packed[k] == p) dup = true;
-        if (!dup) packed[np++] = p;
-    }
-    for (uint32_t i = 0; s.best.err && i + 1 < np; i++)
-        for (uint32_t jj = i + 1; s.best.err && jj < np; jj++) evaluate(s, L, packed[i], packed[jj], 0);
-    const uint64_t err = s.best.err;
-    if (err) s.best.err = 1;
-    for (uint32_t i = 0; s.best.err && i + 1 < np; i++)
-        for (uint32_t jj = i + 1; s.best.err && jj < np; jj++) evaluate(s, L, packed[i], packed[jj], 1);
-    if (s.best.err) s.best.err = err;
-}
-
-__device__ uint32_t sweep(uint32_t range, const float* base, const float (*axis2)[3], uint32_t* out)
-{
-    int prev[2] = {-1, -1};
-    uint32_t n = 0;
-    const float init[3] = {base[0] + .5f, base[1] + .5f, base[2] + .5f};
-    for (uint32_t i = 0; i < range; i++) {
-        const int ls = i ? 0 : 1;
-        const int x = c_uber_probe[i];
-        for (int sg = ls; sg < 2; sg++) {
-            const float pr = init[0] + axis2[sg][0] * (float)x;
-            const float pg = init[1] + axis2[sg][1] * (float)x;
-            const float pb = init[2] + axis2[sg][2] * (float)x;
-            const int r = clampi((int)floorf(pr), 31), g = clampi((int)floorf(pg), 63), b = clampi((int)floorf(pb), 31);
-            const int packed = b | (g << 5) | (r << 11);
-            if (packed != prev[sg]) {
-                out[n++] = (uint32_t)packed;
-                prev[sg] = packed;
-            }
-        }
-    }
-    return n;
-}
-
-template <class Lds>
-__device__ void lattice(St& s, Lds& L, int which)
-{
-    int lr, lg, lb;
-    unpack565(which ? s.best.hi : s.best.lo, 0, lr, lg, lb);
-    for (int i = 0; i < 26; i++) {
-        const int r = lr + c_adj[i][0];
-        if (r < 0 || r > 31) continue;
-        const int g = lg + c_adj[i][1];
-        if (g < 0 || g > 63) continue;
-        const int b = lb + c_adj[i][2];
-        if (b < 0 || b > 31) continue;
-        const uint32_t c = pack565(r, g, b, 0);
-        if (which) eval_canon(s, L, s.best.lo, c);
-        else eval_canon(s, L, c, s.best.hi);
-    }
-    unpack565(which ? s.best.hi : s.best.lo, 0, lr, lg, lb);
-    for (int a = 0; a < 3; a++) {
-        const int limit = a == 1 ? 63 : 31;
-        for (int sg = -2; sg <= 2; sg += 4) {
-            int comp[3] = {lr, lg, lb};
-            const int q = comp[a] + sg;
-            if (q < 0 || q > limit) continue;
-            comp[a] = q;
-            const uint32_t c = pack565(comp[0], comp[1], comp[2], 0);
-            if (which) eval_canon(s, L, s.best.lo, c);
-            else eval_canon(s, L, c, s.best.hi);
-        }
-    }
-}
-
-// optimize_endpoints (crn_dxt1.cpp:703-1067), uber quality
-template <class Lds>
-__device__ void optimize_endpoints(St& s, Lds& L, float* lo, float* hi)
-{
-    const float olo[3] = {lo[0], lo[1], lo[2]}, ohi[3] = {hi[0], hi[1], hi[2]};
-    const uint32_t range = 15, passes = 4;
-    const float dist = .015625f;
-    try_median4(s, L, olo, ohi);
-    float ax[2][3];
-    for (int k = 0; k < 3; k++) ax[1][k] = s.axis[k] * dist;
-    ax[1][0] *= 31.0f;
-    ax[1][1] *= 63.0f;
-    ax[1][2] *= 31.0f;
-    for (int k = 0; k < 3; k++) ax[0][k] = -ax[1][k];
-    const float lim[3] = {31.0f, 63.0f, 31.0f};
+    int o[3];
     for (int k = 0; k < 3; k++) {
-        const float a = lo[k] * lim[k];
-        lo[k] = a < 0.0f ? 0.0f : (a > lim[k] ? lim[k] : a);
-        const float b = hi[k] * lim[k];
-        hi[k] = b < 0.0f ? 0.0f : (b > lim[k] ? lim[k] : b);
+        const float x = (float)((a >> (8 * k)) & 255u), y = (float)((b >> (8 * k)) & 255u);
+        o[k] = clampi((int)(rr + (x + (y - x) * f)), 255);
     }
-    uint32_t plow[31], phigh[31];
-    for (uint32_t pass = 0; pass < passes; pass++) {
-        if (pass) {
-            int r, g, b;
-            unpack565(s.best.lo, 0, r, g, b);
-            lo[0] = (float)r; lo[1] = (float)g; lo[2] = (float)b;
-            unpack565(s.best.hi, 0, r, g, b);
-            hi[0] = (float)r; hi[1] = (float)g; hi[2] = (float)b;
-        }
-        const uint64_t prev = s.best.err;
-        if (!prev) break;
-        const uint32_t nl = sweep(range, lo, ax, plow);
-        const uint32_t nh = sweep(range, hi, ax, phigh);
-        for (uint32_t i = 0; i < nl; i++)
-            for (uint32_t jj = 0; jj < nh; jj++) eval_canon(s, L, plow[i], phigh[jj]);
-        lattice(s, L, 0);
-        lattice(s, L, 1);
-        if (!s.best.err || (pass && s.best.err == prev)) break;
-        refine(s, L, 1);
-    }
-    if (s.best.err && !s.have_alpha) {
-        bool solid = false;
-        // the uber evaluator keeps the best solution's selectors current
-        if (Lds::kUber && s.sel_nonempty) compute_selectors(s, L);
-        if (sel_all_equal(s, L)) solid = try_average_solid(s, L);
-        if (!solid) optimize_comps(s, L);
-    }
-    if (s.best.err) try_combinatorial(s, L);
+    return pack565(o[0], o[1], o[2], 1);
 }
 
-// handle_multicolor_block (crn_dxt1.cpp:1069-1178)
+// The distinct packed colours of try_combinatorial_encoding (crn_dxt1.cpp:
+// 1886-1950) for 2 to 4 colours into q.list[0], in the reference's order (the
+// colours, then the interpolations; one per lane): their number.
 template <class Lds>
-__device__ void handle_multicolor(St& s, Lds& L)
+__device__ uint32_t combinatorial_colours(St& s, Lds& L)
 {
+    SearchLds& q = L.u.q;
+    const uint32_t lane = lane_id(), nu = s.nu;
+    uint32_t n = nu, p = 0;
+    if (lane < nu) {
+        const uint32_t c = L.col[lane];
+        p = pack565((int)(c & 255u), (int)((c >> 8) & 255u), (int)((c >> 16) & 255u), 1);
+    }
+    if (nu == 2) {
+        // rounding (2) x start (2) x ten factors
+        n += 40;
+        if (lane >= nu && lane < n) {
+            const uint32_t i = lane - nu, k = i / 20, a = i / 10 % 2, f = i % 10;
+            const float fs[10] = {2.0f, 3.0f, .5f, 1.5f, -1.0f, 2.0f, -.5f, .5f, -2.0f, -1.0f};
+            float v = fs[0];
+            for (uint32_t t = 1; t < 10; t++) v = t == f ? fs[t] : v;
+            p = lerp_color(L.col[a], L.col[a ^ 1u], v, (int)k);
+        }
+    } else if (nu == 3) {
+        // ordered pairs (6) x four factors
+        n += 24;
+        if (lane >= nu && lane < n) {
+            const uint32_t i = lane - nu, pr = i / 4, f = i % 4, a = pr / 2, b0 = pr % 2, b = b0 >= a ? b0 + 1 : b0;
+            const float v = f == 0 ? 1.5f : f == 1 ? 2.0f / 3.0f : f == 2 ? 1.0f / 3.0f : -.5f;
+            p = lerp_color(L.col[a], L.col[b], v, 1);
+        }
+    }
+    bool dup = lane >= n;
+    for (uint32_t k = 0; k + 1 < n; k++) dup |= k < lane && lane_u32(p, k) == p;
+    const uint64_t mask = __ballot(!dup);
+    if (!dup) q.list[0][__popcll(mask & ((1ull << lane) - 1ull))] = p;
+    const uint32_t np = (uint32_t)__popcll(mask);
+    if (lane == 0) q.fixed[0][0] = (int)np;
+    __builtin_amdgcn_wave_barrier();
+    return np;
+}
+
+// One end of a probe sweep into `out`: probe i's two signs in order, each
+// dropped when it packs as the sign's probe before it did (one probe and sign
+// per lane); their number.
+__device__ uint32_t sweep(const float* base, const float (*axis2)[3], uint32_t* out)
+{
+    const uint32_t lane = lane_id();
+    uint32_t packed[2] = {0, 0};
+    const uint32_t sg = (lane + 1) & 1u;       // lane 0: probe 0, sign 1; lane 2 i - 1, 2 i: probe i, signs 0, 1
+    const uint32_t i = (lane + 1) >> 1;
+    for (int back = 0; back < 2; back++) {
+        const int x = c_uber_probe[min(i - (uint32_t)(back && i ? 1 : 0), 14u)];
+        const float a0 = sg ? axis2[1][0] : axis2[0][0], a1 = sg ? axis2[1][1] : axis2[0][1],
+                    a2 = sg ? axis2[1][2] : axis2[0][2];
+        const float pr = (base[0] + .5f) + a0 * (float)x;
+        const float pg = (base[1] + .5f) + a1 * (float)x;
+        const float pb = (base[2] + .5f) + a2 * (float)x;
+        packed[back] = (uint32_t)(clampi((int)floorf(pb), 31) | (clampi((int)floorf(pg), 63) << 5) |
+                                  (clampi((int)floorf(pr), 31) << 11));
+    }
+    // probe 0 has sign 1 only: nothing lies before it, nor before probe 1 of sign 0
+    const bool first = sg ? i == 0 : i == 1;
+    const bool keep = lane < 29 && (first || packed[0] != packed[1]);
+    const uint64_t mask = __ballot(keep);
+    if (keep) out[__popcll(mask & ((1ull << lane) - 1ull))] = packed[0];
+    return (uint32_t)__popcll(mask);
+}
+
+// handle_multicolor_block up to optimize_endpoints (crn_dxt1.cpp:1069-1178):
+// weights, means, axis, and the two ends of the colours' extent on the axis.
+template <class Lds>
+__device__ void multicolor_ends(St& s, Lds& L, float* lo, float* hi)
+{
+    const uint32_t lane = lane_id();
     uint32_t npass = 1;
     s.pw[0] = s.pw[1] = s.pw[2] = 1.0f;
     if (s.perceptual) {
-        float red = 0, blue = 0, al = 0;
-        for (uint32_t i = 0; i < s.nu; i++) {
-            const uint32_t c = L.col[i];
+        float(*f)[kRow] = L.u.q.stage.f;
+        float acc = 0.0f;
+        for (uint32_t i0 = 0; i0 < s.nu; i0 += 64) {
+            const uint32_t i = min(i0 + lane, s.nu - 1), c = L.col[i];
+            const bool in = i0 + lane < s.nu;
             const int r = (int)(c & 255u), g = (int)((c >> 8) & 255u), b = (int)((c >> 16) & 255u);
             const int l = (r + g + b + 1) / 3;
             const float lf = (float)l;
             const float scale = (float)L.w[i] / (lf > 1.0f ? lf : 1.0f);
-            red += scale * r;
-            blue += scale * b;
-            al += l;
+            f[0][lane] = in ? scale * r : 0.0f;
+            f[1][lane] = in ? scale * b : 0.0f;
+            f[2][lane] = in ? lf : 0.0f;
+            __builtin_amdgcn_wave_barrier();
+            acc = add_row(f[min(lane, 2u)], acc);
+            __builtin_amdgcn_wave_barrier();
         }
+        float red = lane_f32(acc, 0), blue = lane_f32(acc, 1), al = lane_f32(acc, 2);
         red /= s.total_w;
         blue /= s.total_w;
         al /= s.total_w;
@@ -990,13 +1211,13 @@ __device__ void handle_multicolor(St& s, Lds& L)
         const float m = red > blue ? red : blue;
         float sat = m * 1.0f / 3.0f;
         sat = sat < 0.0f ? 0.0f : (sat > 1.0f ? 1.0f : sat);
-        const float p = al * powf(sat, 2.75f);
+        const float p = unif(al * powf(sat, 2.75f));
         if (p >= 1.0f) {
             npass = 1;
         } else {
             npass = 2;
             const float lum[3] = {.212f, .72f, .072f};
-            for (int k = 0; k < 3; k++) s.pw[k] = lum[k] + (s.pw[k] - lum[k]) * p;
+            for (int k = 0; k < 3; k++) s.pw[k] = unif(lum[k] + (s.pw[k] - lum[k]) * p);
         }
     }
     for (uint32_t pass = 0; pass < npass; pass++) {
@@ -1012,6 +1233,7 @@ __device__ void handle_multicolor(St& s, Lds& L)
             const float k = (float)(1.0f / sqrt(n));
             for (int i = 0; i < 3; i++) s.axis[i] *= k;
         }
+        for (int i = 0; i < 3; i++) s.axis[i] = unif(s.axis[i]);
         if (npass > 1) {
             if (fabsf(s.axis[0]) >= .795f) {
                 s.pw[0] = .424f; s.pw[1] = .6f; s.pw[2] = .072f;
@@ -1023,16 +1245,22 @@ __device__ void handle_multicolor(St& s, Lds& L)
         }
     }
     float l = 1e+9f, h = -1e+9f;
-    for (uint32_t i = 0; i < s.nu; i++) {
+    for (uint32_t i = lane; i < s.nu; i += 64) {
         float n[3], nw[3];
-        norm_of(s, L, i, n, nw);
+        norm_of(s, L.col[i], n, nw);
         float d = n[0] * s.axis[0];
         d += n[1] * s.axis[1];
         d += n[2] * s.axis[2];
         l = d < l ? d : l;
         h = h < d ? d : h;
     }
-    float lo[3], hi[3];
+    for (int off = 32; off > 0; off >>= 1) {
+        const float l2 = __shfl_xor(l, off), h2 = __shfl_xor(h, off);
+        l = l2 < l ? l2 : l;
+        h = h < h2 ? h2 : h;
+    }
+    l = unif(l);
+    h = unif(h);
     for (int k = 0; k < 3; k++) {
         lo[k] = s.mean[k] + l * s.axis[k];
         hi[k] = s.mean[k] + h * s.axis[k];
@@ -1052,7 +1280,205 @@ __device__ void handle_multicolor(St& s, Lds& L)
         const float nd[3] = {-s.axis[0], -s.axis[1], -s.axis[2]};
         if (ray_unit_box(c, hi, nd)) { hi[0] = c[0]; hi[1] = c[1]; hi[2] = c[2]; }
     }
-    optimize_endpoints(s, L, lo, hi);
+}
+
+// The search over the cluster's colours (crn_dxt1.cpp:703-1178, 2207-2232):
+// the one-colour shortcut, or handle_multicolor_block and optimize_endpoints
+// at uber quality.  Every step prepares a list of candidates; one loop tries
+// them, so that gathering, scoring and taking exist once.
+enum Step : uint32_t {
+    kStepOne,         // a single colour
+    kStepMedian,      // try_median4: the pairs of means ...
+    kStepMedianFit,   // ... and refine_solution
+    kStepSweep,       // a pass: probe sweeps, lattice moves of either end, refine_solution
+    kStepAdj0,
+    kStepAxis0,
+    kStepAdj1,
+    kStepAxis1,
+    kStepPassEnd,
+    kStepSolid,       // all selectors equal: solid tries
+    kStepComps,       // optimize_endpoint_comps, one component at a time
+    kStepCombFirst,   // 2 to 4 colours: try_combinatorial_encoding
+    kStepComb,
+    kStepCombAlt,
+};
+
+template <class Lds, uint32_t W>
+__device__ void search(St& s, Lds& L)
+{
+    SearchLds& q = L.u.q;
+    const uint32_t lane = lane_id();
+    float lo[3], hi[3], ax[2][3];
+    uint32_t step = kStepOne, pass = 0;
+    uint64_t prev = 0, comb_err = 0;
+    int slo[3] = {0, 0, 0}, shi[3] = {0, 0, 0}, comp = 0;
+    if (!(s.nu == 1 && !s.have_alpha)) {
+        multicolor_ends(s, L, lo, hi);
+        median4(s, L, lo, hi);
+        const float dist = .015625f;
+        for (int k = 0; k < 3; k++) ax[1][k] = s.axis[k] * dist;
+        ax[1][0] *= 31.0f;
+        ax[1][1] *= 63.0f;
+        ax[1][2] *= 31.0f;
+        for (int k = 0; k < 3; k++) ax[0][k] = -ax[1][k];
+        const float lim[3] = {31.0f, 63.0f, 31.0f};
+        for (int k = 0; k < 3; k++) {
+            const float a = lo[k] * lim[k];
+            lo[k] = a < 0.0f ? 0.0f : (a > lim[k] ? lim[k] : a);
+            const float b = hi[k] * lim[k];
+            hi[k] = b < 0.0f ? 0.0f : (b > lim[k] ? lim[k] : b);
+        }
+        step = kStepMedian;
+    }
+    for (;;) {
+        uint32_t kind = 0, n = 0, from = 0;
+        int alt = 0;
+        bool again = false;
+        switch (step) {
+        case kStepOne:
+            // evaluated as the average of one colour
+            if (lane == 0) q.list[0][0] = L.col[0];
+            __builtin_amdgcn_wave_barrier();
+            kind = kListSolid;
+            n = Lds::kUber ? 2 : 1;
+            break;
+        case kStepMedian:
+            kind = kListPair;
+            n = 6;
+            break;
+        case kStepMedianFit:
+        case kStepPassEnd:
+            if (refine_fit(s, L)) {
+                kind = kListRefine;
+                n = 54;
+            }
+            break;
+        case kStepSweep: {
+            if (pass == 4 || !s.best.err) {
+                step = kStepSolid;
+                continue;
+            }
+            if (pass) {
+                int r, g, b;
+                unpack565(s.best.lo, 0, r, g, b);
+                lo[0] = (float)r; lo[1] = (float)g; lo[2] = (float)b;
+                unpack565(s.best.hi, 0, r, g, b);
+                hi[0] = (float)r; hi[1] = (float)g; hi[2] = (float)b;
+            }
+            prev = s.best.err;
+            const uint32_t nl = sweep(lo, ax, q.list[0]);
+            const uint32_t nh = sweep(hi, ax, q.list[1]);
+            if (lane == 0) q.fixed[0][0] = (int)nh;
+            __builtin_amdgcn_wave_barrier();
+            kind = kListSweep;
+            n = nl * 32;
+            break;
+        }
+        case kStepAdj0:
+        case kStepAdj1:
+            kind = step == kStepAdj0 ? kListAdj0 : kListAdj1;
+            from = step == kStepAdj0 ? s.best.lo : s.best.hi;
+            n = 26;
+            again = true;
+            break;
+        case kStepAxis0:
+        case kStepAxis1:
+            kind = step == kStepAxis0 ? kListAxis0 : kListAxis1;
+            from = step == kStepAxis0 ? s.best.lo : s.best.hi;
+            n = 6;
+            again = true;
+            break;
+        case kStepSolid:
+            if (!s.best.err || s.have_alpha) {
+                step = kStepCombFirst;
+                continue;
+            }
+            // the uber evaluator keeps the best solution's selectors current
+            if (Lds::kUber && s.sel_nonempty) compute_selectors(s, L);
+            if (sel_all_equal(s, L)) {
+                const uint32_t avg = average_colour(s, L);
+                if (lane == 0) q.list[0][0] = avg;
+                __builtin_amdgcn_wave_barrier();
+                kind = kListSolid;
+                n = (s.nu + 1) * (Lds::kUber ? 2 : 1);
+            }
+            break;
+        case kStepComps: {
+            if (comp == 0) {
+                // the starting values stay those of the solution found so far
+                compute_selectors(s, L);
+                unpack565(s.best.lo, 1, slo[0], slo[1], slo[2]);
+                unpack565(s.best.hi, 1, shi[0], shi[1], shi[2]);
+            }
+            if (!s.best.err || comp == 3 || (comp == 0 && s.best.alpha)) {
+                step = kStepCombFirst;
+                continue;
+            }
+            int a[3], b[3];
+            unpack565(s.best.lo, 0, a[0], a[1], a[2]);
+            unpack565(s.best.hi, 0, b[0], b[1], b[2]);
+            if (lane == 0)
+                for (int k = 0; k < 3; k++) {
+                    q.fixed[0][k] = a[k];
+                    q.fixed[1][k] = b[k];
+                }
+            compute_selectors(s, L);
+            comp_errors(s, L, comp);
+            comp_best(L, (uint32_t)(comp == 0 ? slo[0] : comp == 1 ? slo[1] : slo[2]),
+                      (uint32_t)(comp == 0 ? shi[0] : comp == 1 ? shi[1] : shi[2]));
+            if (uni64(q.brem[0]) < uni64(q.qbest)) {
+                kind = kListComp0 + (uint32_t)comp;
+                n = (comp == 1 ? 64u : 32u) * 64;
+                again = true;
+            }
+            break;
+        }
+        case kStepCombFirst:
+            if (!s.best.err || s.nu < 2 || s.nu > 4) return;
+            combinatorial_colours(s, L);
+            step = kStepComb;
+            continue;
+        case kStepComb:
+        case kStepCombAlt:
+            kind = kListComb;
+            alt = step == kStepCombAlt ? 1 : 0;
+            n = uni((uint32_t)q.fixed[0][0]) * 64;
+            break;
+        }
+        bool improved = false;
+        uint32_t first = 0;
+        while (first < n && try_list<Lds, W>(s, L, kind, n, alt, again, from, first)) {
+            improved = true;
+            if (kind >= kListComp0 && s.best.err) {
+                // the tables and the best of the new solution's selectors
+                const uint32_t i = first - 1;
+                compute_selectors(s, L);
+                comp_errors(s, L, comp);
+                comp_best(L, expand_comp(comp, i >> 6), expand_comp(comp, i & 63u));
+            }
+        }
+        switch (step) {
+        case kStepOne: return;
+        case kStepAxis1:
+            step = !s.best.err || (pass && s.best.err == prev) ? (uint32_t)kStepSolid : (uint32_t)kStepPassEnd;
+            break;
+        case kStepPassEnd:
+            pass++;
+            step = kStepSweep;
+            break;
+        case kStepSolid: step = improved ? (uint32_t)kStepCombFirst : (uint32_t)kStepComps; break;
+        case kStepComps: comp++; break;
+        case kStepComb:
+            comb_err = s.best.err;
+            if (comb_err) s.best.err = 1;
+            step = kStepCombAlt;
+            break;
+        case kStepCombAlt:
+            if (s.best.err) s.best.err = comb_err;
+            return;
+        default: step++; break;   // kStepMedian, kStepMedianFit, kStepSweep, kStepAdj0, kStepAxis0, kStepAdj1
+        }
+    }
 }
 
 struct ClusterOut {
@@ -1064,77 +1490,25 @@ struct ClusterOut {
 };
 constexpr uint32_t kNotEncoded = 1u << 8;
 
-// Open-addressing colour hash over L.kCapH slots (a power of two in LDS, any
+// Open-addressing colour hash over `cap` slots (a power of two in LDS, any
 // size in the global store): first slot and linear probe.
-template <class Lds>
-__device__ inline uint32_t hash_slot(const Lds& L, uint32_t key)
+__device__ inline uint32_t hash_next(uint32_t cap, uint32_t h) { return h + 1 == cap ? 0 : h + 1; }
+
+__device__ inline uint32_t hash_find(const uint32_t* hkey, uint32_t cap, uint32_t key)
 {
-    return hash32(key) % L.kCapH;
+    uint32_t h = hash32(key) % cap;
+    while (hkey[h] != key) h = hash_next(cap, h);
+    return h;
 }
 
-template <class Lds>
-__device__ inline uint32_t hash_next(const Lds& L, uint32_t h)
+// Ascending bitonic sort of P (a power of two) pairs by (key, idx), T threads.
+template <uint32_t T>
+__device__ inline void sort_pairs(uint32_t* key, uint16_t* idx, uint32_t P)
 {
-    return h + 1 == L.kCapH ? 0 : h + 1;
-}
-
-template <class Lds>
-__device__ inline int hash_find(const Lds& L, uint32_t key)
-{
-    uint32_t h = hash_slot(L, key);
-    while (L.hkey[h]) {
-        if (L.hkey[h] == key) return (int)L.hval[h];
-        h = hash_next(L, h);
-    }
-    return -1;
-}
-
-// Unique-colour index of texel i (key = its colour | 0xFF000000).
-template <uint32_t MaxU>
-__device__ inline uint32_t unique_index(const LdsT<MaxU>& L, uint32_t, uint32_t key)
-{
-    return (uint32_t)hash_find(L, key);
-}
-
-template <uint32_t MaxU>
-__device__ inline uint32_t unique_index(const LdsS<MaxU>& L, uint32_t i, uint32_t)
-{
-    return L.tmap[i];
-}
-
-// Unique colours of a cluster of n <= MaxU texels in first-appearance order
-// with their texel counts, and every texel's unique index, without a hash:
-// bitonic sort of (colour, texel index) pairs, the first texel of each run
-// of equal colours marked in a bitmap, a colour's rank = the number of marked
-// texels before its first one.  One wave; the block is the wave.
-template <uint32_t MaxU>
-__device__ uint32_t unique_sorted(LdsS<MaxU>& L, const uint32_t* __restrict__ px, uint32_t p0, uint32_t n,
-                              uint32_t thresh, uint32_t& opaque)
-{
-    uint32_t* key = reinterpret_cast<uint32_t*>(L.sel);
-    uint16_t* idx = reinterpret_cast<uint16_t*>(key + MaxU);
-    const uint32_t lane = lane_id();
-    uint32_t P = 64;
-    while (P < n) P <<= 1;   // n <= MaxU, a power of two
-    uint32_t nop = 0;
-    for (uint32_t i = lane; i < P; i += 64) {
-        // transparent texels (DXT1A) sort after every colour, before the padding
-        const uint32_t p = i < n ? px[p0 + i] : 0u;
-        const bool tr = i < n && (p >> 24) < thresh;
-        key[i] = i < n ? (tr ? 0xFFFFFFFEu : (p & 0x00FFFFFFu)) : 0xFFFFFFFFu;
-        idx[i] = (uint16_t)i;
-        nop += (i < n && !tr) ? 1u : 0u;
-    }
-    for (int off = 32; off; off >>= 1) nop += (uint32_t)__shfl_xor((int)nop, off);
-    opaque = nop;
-    const uint32_t nsrc = n;
-    n = nop;
-    for (uint32_t i = lane; i < MaxU / 32; i += 64) L.fbits[i] = 0;
-    __syncthreads();
     for (uint32_t k = 2; k <= P; k <<= 1)
         for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            for (uint32_t t = lane; t < P / 2; t += 64) {
-                const uint32_t a = 2 * j * (t / j) + (t % j), b = a + j;
+            for (uint32_t t = threadIdx.x; t < P / 2; t += T) {
+                const uint32_t a = ((t & ~(j - 1)) << 1) | (t & (j - 1)), b = a + j;
                 const uint32_t ka = key[a], kb = key[b];
                 const uint32_t ia = idx[a], ib = idx[b];
                 const bool gt = ka > kb || (ka == kb && ia > ib);
@@ -1147,28 +1521,181 @@ __device__ uint32_t unique_sorted(LdsS<MaxU>& L, const uint32_t* __restrict__ px
             }
             __syncthreads();
         }
+}
+
+// Unique colours of a cluster of n <= MaxU texels in first-appearance order
+// with their texel counts, without a hash: sorted (colour, texel index) pairs, the first texel of each run of equal
+// colours marked in a bitmap, a colour's rank = the number of marked texels
+// before its first one.  Each of the T threads then walks its stretch of the
+// sorted pairs from the run that reaches into it.
+template <uint32_t MaxU, uint32_t T>
+__device__ uint32_t unique_sorted(LdsS<MaxU>& L, const uint32_t* __restrict__ px, uint32_t p0, uint32_t n,
+                                  uint32_t thresh, uint32_t& opaque)
+{
+    uint32_t* key = reinterpret_cast<uint32_t*>(L.sel);
+    uint16_t* idx = reinterpret_cast<uint16_t*>(key + MaxU);
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = uni(tid >> 6);
+    uint32_t P = 64;
+    while (P < n) P <<= 1;   // n <= MaxU, a power of two
+    if (tid == 0) L.nopaque = 0;
+    __syncthreads();
+    for (uint32_t i0 = 0; i0 < P; i0 += T) {
+        // transparent texels (DXT1A) sort after every colour, before the padding
+        const uint32_t i = i0 + tid;
+        const uint32_t p = i < n ? px[p0 + i] : 0u;
+        const bool tr = i < n && (p >> 24) < thresh;
+        if (i < P) {
+            key[i] = i < n ? (tr ? 0xFFFFFFFEu : (p & 0x00FFFFFFu)) : 0xFFFFFFFFu;
+            idx[i] = (uint16_t)i;
+        }
+        const uint64_t mask = __ballot(i < n && !tr);
+        if (lane == 0) atomicAdd(&L.nopaque, (uint32_t)__popcll(mask));
+    }
+    for (uint32_t i = tid; i < MaxU / 32; i += T) L.fbits[i] = 0;
+    __syncthreads();
+    const uint32_t nop = opaque = uni(L.nopaque);
+    sort_pairs<T>(key, idx, P);
     // runs of equal colours (the padding sorts past the n real texels)
-    for (uint32_t j = lane; j < n; j += 64)
+    for (uint32_t j = tid; j < nop; j += T)
         if (j == 0 || key[j] != key[j - 1]) atomicOr(&L.fbits[idx[j] >> 5], 1u << (idx[j] & 31u));
     __syncthreads();
-    const uint32_t nw = (nsrc + 31) / 32;   // first-texel bits of all texels: at most 64 words, one per lane
-    const uint32_t cnt = lane < nw ? (uint32_t)__popc(L.fbits[lane]) : 0u;
-    uint32_t incl = cnt;
-    for (uint32_t off = 1; off < 64; off <<= 1) {
-        const uint32_t v = (uint32_t)__shfl_up((int)incl, off);
-        if (lane >= off) incl += v;
+    if (wave == 0) {
+        uint32_t base = 0;
+        for (uint32_t w0 = 0; w0 < MaxU / 32; w0 += 64) {
+            const uint32_t w = w0 + lane;
+            const uint32_t cnt = w < MaxU / 32 ? (uint32_t)__popc(L.fbits[w]) : 0u;
+            uint32_t incl = cnt;
+            for (uint32_t off = 1; off < 64; off <<= 1) {
+                const uint32_t v = (uint32_t)__shfl_up((int)incl, off);
+                if (lane >= off) incl += v;
+            }
+            if (w < MaxU / 32) L.fbase[w] = base + incl - cnt;
+            base += lane_u32(incl, 63);
+        }
+        if (lane == 0) L.nuniq = base;
     }
-    if (lane < nw) L.fbase[lane] = incl - cnt;
-    const uint32_t nu = (uint32_t)__shfl((int)incl, 63);
+    // the last run start in each thread's stretch, and by a scan the one before it
+    const uint32_t E = P > T ? P / T : 1u, j0 = min(tid * E, nop), j1 = min(j0 + E, nop);
+    int head = -1;
+    for (uint32_t j = j0; j < j1; j++)
+        if (j == 0 || key[j] != key[j - 1]) head = (int)j;
+    int incl = head;
+    for (uint32_t off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(incl, off);
+        if (lane >= off) incl = max(incl, v);
+    }
+    if (lane == 63) L.scan[wave] = incl;
+    int before = __shfl_up(incl, 1);
+    if (lane == 0) before = -1;
     __syncthreads();
-    for (uint32_t j = lane; j < n; j += 64) {
-        if (j != 0 && key[j] == key[j - 1]) continue;
+    for (uint32_t w = 0; w < wave; w++) before = max(before, L.scan[w]);
+    auto rank = [&](uint32_t j) {
         const uint32_t f = idx[j];   // the colour's first texel
-        const uint32_t r = L.fbase[f >> 5] + (uint32_t)__popc(L.fbits[f >> 5] & ((1u << (f & 31u)) - 1u));
-        uint32_t e = j;
-        for (; e < n && key[e] == key[j]; e++) L.tmap[idx[e]] = (uint16_t)r;
-        L.col[r] = key[j];
-        L.w[r] = (uint16_t)(e - j);
+        return L.fbase[f >> 5] + (uint32_t)__popc(L.fbits[f >> 5] & ((1u << (f & 31u)) - 1u));
+    };
+    if (j0 < j1) {
+        int h = before;
+        uint32_t r = h >= 0 ? rank((uint32_t)h) : 0u;
+        for (uint32_t j = j0; j < j1; j++) {
+            if (j == 0 || key[j] != key[j - 1]) {
+                if (h >= 0) L.w[r] = (uint16_t)(j - (uint32_t)h);
+                h = (int)j;
+                r = rank(j);
+                L.col[r] = key[j];
+            }
+        }
+        if (j1 == nop) L.w[r] = (uint16_t)(nop - (uint32_t)h);
+    }
+    __syncthreads();
+    return uni(L.nuniq);
+}
+
+// The same for a cluster of any number of texels, through a colour hash in
+// LDS that keeps each colour's first texel and count; a colour's rank follows
+// from sorting the first texels.  More than MaxU colours: returns MaxU + 1.
+template <uint32_t MaxU, uint32_t T>
+__device__ uint32_t unique_hashed(LdsT<MaxU>& L, const uint32_t* __restrict__ px, uint32_t p0, uint32_t n,
+                                  uint32_t thresh, uint32_t& opaque)
+{
+    constexpr uint32_t kCap = LdsT<MaxU>::kCapH, kPer = MaxU / T;
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t i = tid; i < kCap; i += T) {
+        L.hkey[i] = 0;
+        L.hval[i] = 0xFFFFFFFFu;
+        L.hcnt[i] = 0;
+    }
+    if (tid == 0) L.nuniq = L.nopaque = L.nsort = 0;
+    __syncthreads();
+    uint32_t nop = 0;
+    // the table is half empty at MaxU colours and each thread adds at most one
+    // more once the count has passed it, so a probe always ends
+    static_assert(MaxU + T < kCap, "hash load");
+    auto insert = [&](uint32_t key, uint32_t first, uint32_t count) {
+        if (__hip_atomic_load(&L.nuniq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > MaxU) return;
+        uint32_t h = hash32(key) % kCap;
+        for (;;) {
+            const uint32_t prev = atomicCAS(&L.hkey[h], 0u, key);
+            if (prev == 0u) atomicAdd(&L.nuniq, 1u);
+            if (prev == 0u || prev == key) {
+                atomicMin(&L.hval[h], first);
+                atomicAdd(&L.hcnt[h], count);
+                return;
+            }
+            h = hash_next(kCap, h);
+        }
+    };
+    // four texels per thread at a time; equal neighbours are added at once
+    for (uint32_t i = 4 * tid; i < n; i += 4 * T) {
+        uint32_t p[4], run = 0, first = 0, key = 0;
+        const uint32_t m = min(4u, n - i);
+        for (uint32_t k = 0; k < 4; k++) p[k] = px[p0 + i + min(k, m - 1)];
+        for (uint32_t k = 0; k < m; k++) {
+            if ((p[k] >> 24) < thresh) continue;   // transparent (DXT1A)
+            const uint32_t c = (p[k] & 0x00FFFFFFu) | 0xFF000000u;
+            nop++;
+            if (run && c == key) {
+                run++;
+                continue;
+            }
+            if (run) insert(key, first, run);
+            key = c;
+            first = i + k;
+            run = 1;
+        }
+        if (run) insert(key, first, run);
+    }
+    atomicAdd(&L.nopaque, nop);
+    __syncthreads();
+    opaque = uni(L.nopaque);
+    const uint32_t nu = uni(L.nuniq);
+    if (nu > MaxU) return MaxU + 1;
+    uint32_t* first = L.col;
+    uint16_t* slot = reinterpret_cast<uint16_t*>(L.w);
+    uint32_t P = 64;
+    while (P < nu) P <<= 1;
+    for (uint32_t h = tid; h < kCap; h += T)
+        if (L.hkey[h]) {
+            const uint32_t at = atomicAdd(&L.nsort, 1u);
+            first[at] = L.hval[h];
+            slot[at] = (uint16_t)h;
+        }
+    for (uint32_t i = nu + tid; i < P; i += T) {
+        first[i] = 0xFFFFFFFFu;
+        slot[i] = 0xFFFFu;
+    }
+    __syncthreads();
+    sort_pairs<T>(first, slot, P);
+    uint32_t mine[kPer];
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; k++) mine[k] = tid + k * T < nu ? slot[tid + k * T] : 0u;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; k++) {
+        const uint32_t r = tid + k * T;
+        if (r < nu) {
+            L.col[r] = L.hkey[mine[k]] & 0x00FFFFFFu;
+            L.w[r] = L.hcnt[mine[k]];
+        }
     }
     __syncthreads();
     return nu;
@@ -1176,34 +1703,29 @@ __device__ uint32_t unique_sorted(LdsS<MaxU>& L, const uint32_t* __restrict__ px
 
 // The colour set of a cluster with more distinct colours than the LDS store
 // holds: colours, weights, selectors and the hash in global memory (a scratch
-// region the cluster owns, sized by its texel count), the per-channel tables
-// in LDS.  Members mirror LdsT's so every search step reads either store.
-struct GStore {
-    uint32_t kCapU, kCapH;
-    uint32_t* col;
-    uint32_t* w;
-    uint8_t* sel;
-    uint32_t* hkey;
-    uint32_t* hval;
-    uint32_t* hcnt;
-    uint32_t* mark;
-    unsigned long long (*pl)[64][3];
-    uint64_t *rlo, *rhi, *glo, *ghi, *blo, *bhi;
-};
-
-__device__ inline uint32_t unique_index(const GStore& L, uint32_t, uint32_t key)
-{
-    return (uint32_t)hash_find(L, key);
-}
-
-
+// region the cluster owns, sized by its texel count), the search's working
+// set and tables in LDS.
 struct GTables {
-    unsigned long long pl[3][64][3];
-    uint64_t rlo[32], rhi[32], glo[64], ghi[64], blo[32], bhi[32];
+    PlanesOrSearch u;
+    Bounds b;
+    uint32_t nopaque;
+    uint32_t scan[8];    // per wave
 };
 
-// Clusters by texel count into the four LDS sizes (any order within a class:
-// each cluster's result depends only on its own texels).
+struct GStore {
+    PlanesOrSearch& u;
+    Bounds& b;
+    uint32_t kCapH = 0;
+    uint32_t* col = nullptr;
+    uint32_t* w = nullptr;
+    uint8_t* sel = nullptr;
+    uint32_t* hkey = nullptr;
+    uint32_t* hval = nullptr;
+    __device__ explicit GStore(GTables& t) : u(t.u), b(t.b) {}
+};
+
+// Clusters by texel count into the five classes (any order within a class: each
+// cluster's result depends only on its own texels).
 __global__ void __launch_bounds__(256) dxt1_cluster_classes_kernel(const uint32_t* __restrict__ ofs,
                                                                   uint32_t nclusters, uint32_t* __restrict__ count,
                                                                   uint32_t* __restrict__ list)
@@ -1211,216 +1733,225 @@ __global__ void __launch_bounds__(256) dxt1_cluster_classes_kernel(const uint32_
     const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nclusters) return;
     const uint32_t n = ofs[c + 1] - ofs[c];
-    const uint32_t k = n <= 512 ? 0 : n <= 1024 ? 1 : n <= 2048 ? 2 : 3;
-    list[(size_t)k * nclusters + atomicAdd(&count[k], 1u)] = c;
+    const uint32_t k = n <= 512 ? 0 : n <= 1024 ? 1 : n <= 2048 ? 2 : n <= 4096 ? 3 : 4;
+    // the last two classes share an array of nclusters entries, filled from its two ends
+    const uint32_t at = atomicAdd(&count[k], 1u);
+    if (k < 4) list[(size_t)k * nclusters + at] = c;
+    else list[4 * (size_t)nclusters - 1 - at] = c;
+}
+
+// One channel's bounds: prefix sums of its planes, one value per lane.
+__device__ inline uint64_t channel_bounds(const unsigned long long (*pl)[3], uint32_t lim, uint64_t scale, uint64_t* lo,
+                                          uint64_t* hi)
+{
+    const uint32_t lane = lane_id();
+    uint64_t p[3];
+    for (int k = 0; k < 3; k++) {
+        p[k] = lane < lim ? pl[lane][k] * scale : 0ull;
+        for (uint32_t off = 1; off < 64; off <<= 1) {
+            const uint32_t a = (uint32_t)__shfl_up((int)(uint32_t)p[k], off), b = (uint32_t)__shfl_up((int)(p[k] >> 32), off);
+            if (lane >= off) p[k] += (uint64_t)a | ((uint64_t)b << 32);
+        }
+    }
+    const uint64_t C = lim == 64 ? (uint8_t)((lane << 2) | (lane >> 4)) : (uint8_t)((lane << 3) | (lane >> 2));
+    const uint64_t t0 = lane_u64(p[0], 63), t1 = lane_u64(p[1], 63), t2 = lane_u64(p[2], 63);
+    const uint64_t l = p[2] + C * C * p[0] - 2 * C * p[1];
+    if (lane < lim) {
+        lo[lane] = l;
+        hi[lane] = t2 + C * C * t0 - 2 * C * t1 - l;
+    }
+    return t2;
 }
 
 // Everything after the unique colours: error planes (crn_dxt1.cpp:2134-2203),
-// the 1-colour shortcut or handle_multicolor_block, selectors and
-// return_solution, for either colour store.
-template <class Lds>
+// the search, selectors and return_solution, for any colour store.  The
+// planes have been cleared.
+template <class Lds, uint32_t W>
 __device__ void cluster_search(St& s, Lds& L, const uint32_t* __restrict__ px, uint32_t p0, uint32_t n,
                                int flags, uint32_t cl, ClusterOut* __restrict__ out,
                                uint8_t* __restrict__ selectors)
 {
-    const uint32_t lane = lane_id();
+    constexpr uint32_t T = 64 * W;
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = uni(tid >> 6);
     ClusterOut o{};
     const uint32_t thresh = s.have_alpha ? ((uint32_t)flags >> 8) & 255u : 0u;
     if (!s.nu) {
         // no opaque texel (compute_internal, crn_dxt1.cpp:2207-2212): a 3-colour
         // block of zero endpoints, every selector transparent (error 0 here)
         if (selectors)
-            for (uint32_t i = lane; i < n; i += 64) selectors[p0 + i] = 3;
-        if (lane == 0) {
+            for (uint32_t i = tid; i < n; i += T) selectors[p0 + i] = 3;
+        if (tid == 0) {
             o.flags = 2;
             out[cl] = o;
         }
         return;
     }
-    for (uint32_t i = lane; i < s.nu; i += 64) {
+    for (uint32_t i = tid; i < s.nu; i += T) {
         const uint32_t c = L.col[i];
         const unsigned long long w = L.w[i];
         const uint32_t R = c & 255u, G = (c >> 8) & 255u, B = (c >> 16) & 255u;
         const uint32_t r = (R >> 3) + (((R & 7) > (R >> 5)) ? 1 : 0);
         const uint32_t g = (G >> 2) + (((G & 3) > (G >> 6)) ? 1 : 0);
         const uint32_t b = (B >> 3) + (((B & 7) > (B >> 5)) ? 1 : 0);
-        atomicAdd(&L.pl[0][r][0], w); atomicAdd(&L.pl[0][r][1], w * R); atomicAdd(&L.pl[0][r][2], w * R * R);
-        atomicAdd(&L.pl[1][g][0], w); atomicAdd(&L.pl[1][g][1], w * G); atomicAdd(&L.pl[1][g][2], w * G * G);
-        atomicAdd(&L.pl[2][b][0], w); atomicAdd(&L.pl[2][b][1], w * B); atomicAdd(&L.pl[2][b][2], w * B * B);
+        auto& pl = L.u.pl;
+        atomicAdd(&pl[0][r][0], w); atomicAdd(&pl[0][r][1], w * R); atomicAdd(&pl[0][r][2], w * R * R);
+        atomicAdd(&pl[1][g][0], w); atomicAdd(&pl[1][g][1], w * G); atomicAdd(&pl[1][g][2], w * G * G);
+        atomicAdd(&pl[2][b][0], w); atomicAdd(&pl[2][b][1], w * B); atomicAdd(&pl[2][b][2], w * B * B);
     }
     __syncthreads();
-    if (lane == 0) {
-        const uint64_t sc[3] = {s.perceptual ? 8u : 1u, s.perceptual ? 25u : 1u, 1u};
-        for (int ch = 0; ch < 3; ch++) {
-            const int lim = ch == 1 ? 64 : 32;
-            for (int c = 0; c < lim; c++)
-                for (int k = 0; k < 3; k++) {
-                    L.pl[ch][c][k] *= sc[ch];
-                    if (c) L.pl[ch][c][k] += L.pl[ch][c - 1][k];
-                }
-        }
-        for (uint32_t c = 0; c < 32; c++) {
-            const uint64_t C = (uint8_t)((c << 3) | (c >> 2));
-            L.rlo[c] = L.pl[0][c][2] + C * C * L.pl[0][c][0] - 2 * C * L.pl[0][c][1];
-            L.rhi[c] = L.pl[0][31][2] + C * C * L.pl[0][31][0] - 2 * C * L.pl[0][31][1] - L.rlo[c];
-            L.blo[c] = L.pl[2][c][2] + C * C * L.pl[2][c][0] - 2 * C * L.pl[2][c][1];
-            L.bhi[c] = L.pl[2][31][2] + C * C * L.pl[2][31][0] - 2 * C * L.pl[2][31][1] - L.blo[c];
-        }
-        for (uint32_t c = 0; c < 64; c++) {
-            const uint64_t C = (uint8_t)((c << 2) | (c >> 4));
-            L.glo[c] = L.pl[1][c][2] + C * C * L.pl[1][c][0] - 2 * C * L.pl[1][c][1];
-            L.ghi[c] = L.pl[1][63][2] + C * C * L.pl[1][63][0] - 2 * C * L.pl[1][63][1] - L.glo[c];
-        }
+    if (wave == 0) {
+        const uint64_t base = channel_bounds(L.u.pl[0], 32, s.perceptual ? 8u : 1u, L.b.rlo, L.b.rhi) +
+                              channel_bounds(L.u.pl[1], 64, s.perceptual ? 25u : 1u, L.b.glo, L.b.ghi) +
+                              channel_bounds(L.u.pl[2], 32, 1u, L.b.blo, L.b.bhi);
+        if (lane == 0) L.b.base = base;
     }
     __syncthreads();
-    s.best.lo = s.best.hi = 0;
-    s.best.err = ~0ull;
-    s.best.alt = s.best.enforce = s.best.enforced = s.best.alpha = 0;
-    s.sel_valid = false;
-    s.sel_nonempty = false;
-    if (s.nu == 1 && !s.have_alpha) {
-        const uint32_t c = L.col[0];
-        const uint32_t r = c & 255u, g = (c >> 8) & 255u, b = (c >> 16) & 255u;
-        evaluate(s, L, (g_c_om5[r][0] << 11) | (g_c_om6[g][0] << 5) | g_c_om5[b][0],
-                 (g_c_om5[r][1] << 11) | (g_c_om6[g][1] << 5) | g_c_om5[b][1], 0);
-        if (Lds::kUber && s.best.err)
-            evaluate(s, L, (g_c_om5_3[r][0] << 11) | (g_c_om6_3[g][0] << 5) | g_c_om5_3[b][0],
-                     (g_c_om5_3[r][1] << 11) | (g_c_om6_3[g][1] << 5) | g_c_om5_3[b][1], 0);
-    } else {
-        handle_multicolor(s, L);
-    }
-    compute_selectors(s, L);
-    // return_solution (crn_dxt1.cpp:263-365): four-colour blocks keep low >
-    // high (selectors through {1, 0, 3, 2}), 3-colour blocks low <= high
-    // (through {1, 0, 2, 3})
-    const bool inv = s.best.alpha ? s.best.lo > s.best.hi : s.best.lo < s.best.hi;
-    const uint32_t lo = inv ? s.best.hi : s.best.lo, hi = inv ? s.best.lo : s.best.hi;
-    if (selectors) {
-        for (uint32_t i = lane; i < n; i += 64) {
-            if ((px[p0 + i] >> 24) < thresh) {
-                selectors[p0 + i] = 3;   // transparent (return_solution, crn_dxt1.cpp:300-343)
-                continue;
-            }
-            const uint32_t key = (px[p0 + i] & 0x00FFFFFFu) | 0xFF000000u;
-            uint32_t v = L.sel[unique_index(L, i, key)];
-            if (inv) v = s.best.alpha ? (v < 2 ? v ^ 1u : v) : (v ^ 1u);
-            selectors[p0 + i] = (uint8_t)v;
+    s.base = uni64(L.b.base);
+    if (wave == 0) {
+        s.best.lo = s.best.hi = 0;
+        s.best.err = ~0ull;
+        s.best.alt = s.best.enforce = s.best.enforced = s.best.alpha = 0;
+        s.sel_valid = false;
+        s.sel_nonempty = false;
+        search<Lds, W>(s, L);
+        // return_solution (crn_dxt1.cpp:263-365): four-colour blocks keep low >
+        // high (selectors through {1, 0, 3, 2}), 3-colour blocks low <= high
+        // (through {1, 0, 2, 3})
+        const bool inv = s.best.alpha ? s.best.lo > s.best.hi : s.best.lo < s.best.hi;
+        if (lane == 0) {
+            const uint32_t lo = inv ? s.best.hi : s.best.lo, hi = inv ? s.best.lo : s.best.hi;
+            o.error = s.best.err;
+            o.lo_hi = lo | (hi << 16);
+            o.nunique = s.nu;
+            o.flags = (uint32_t)inv | ((uint32_t)s.best.alpha << 1) | ((uint32_t)s.best.alt << 2) |
+                      ((uint32_t)s.best.enforce << 3) | ((uint32_t)s.best.enforced << 4);
+            out[cl] = o;
+            L.u.q.end_pal = s.best.alpha ? palette3(s.best.lo, s.best.hi, s.best.alt)
+                                         : palette4(s.best.lo, s.best.hi, s.best.alt);
+            L.u.q.end_alpha = (uint32_t)s.best.alpha;
+            L.u.q.end_inv = inv ? 1u : 0u;
+            L.u.q.end_enforce = (uint32_t)s.best.enforce;
+            L.u.q.end_enforced = (uint32_t)s.best.enforced;
+            L.u.q.cmd = 0;
         }
+    } else if constexpr (W > 1) {
+        score_loop<Lds, W>(L, s.nu, s.base, s.perceptual, wave);
+        __syncthreads();
     }
-    if (lane == 0) {
-        o.error = s.best.err;
-        o.lo_hi = lo | (hi << 16);
-        o.nunique = s.nu;
-        o.flags = (uint32_t)inv | ((uint32_t)s.best.alpha << 1) | ((uint32_t)s.best.alt << 2) |
-                  ((uint32_t)s.best.enforce << 3) | ((uint32_t)s.best.enforced << 4);
-        out[cl] = o;
+    if (wave == 0) {
+        __syncthreads();   // ends the other waves' loop
+        if constexpr (W > 1) __syncthreads();
+    }
+    if (!selectors) return;
+    const SearchLds& q = L.u.q;
+    const bool alpha = uni(q.end_alpha) != 0, inv = uni(q.end_inv) != 0, enforce = uni(q.end_enforce) != 0;
+    const Pal pal = q.end_pal;
+    for (uint32_t i = tid; i < n; i += T) {
+        const uint32_t p = px[p0 + i];
+        uint32_t v = 3;   // transparent (return_solution, crn_dxt1.cpp:300-343)
+        if ((p >> 24) >= thresh) {
+            v = enforce ? q.end_enforced : nearest(pal, s.perceptual, alpha, p);
+            if (inv) v = alpha ? (v < 2 ? v ^ 1u : v) : (v ^ 1u);
+        }
+        selectors[p0 + i] = (uint8_t)v;
     }
 }
 
-template <uint32_t MaxU, bool Uber>
-__global__ void __launch_bounds__(64) dxt1_cluster_kernel(const uint32_t* __restrict__ px,
-                                                          const uint32_t* __restrict__ ofs,
-                                                          const uint32_t* __restrict__ list,
-                                                          const uint32_t* __restrict__ count, int perceptual,
-                                                          ClusterOut* __restrict__ out,
-                                                          uint8_t* __restrict__ selectors)
+// Waves per cluster: the search of one cluster is a chain of lists, so a large
+// cluster is shared by several waves (each list's candidates dealt to them)
+// and a small one, of which there are thousands, is left to one.  Eight waves
+// and batches of 64 serve the last class, whose workgroups have a CU alone.
+template <uint32_t Class>
+constexpr uint32_t kWavesOf = Class == 0 ? 1 : Class == 1 ? 2 : Class == 4 ? 8 : 4;
+constexpr uint32_t kBigWaves = 8;
+
+template <uint32_t Class>
+using StoreOf = std::conditional_t<Class == 4, LdsT<kMaxU>, LdsS<(Class < 3 ? 512u << Class : kMaxU)>>;
+
+template <uint32_t Class, bool Uber>
+__device__ void cluster_of_class(LdsU<StoreOf<Class>, Uber>& L, const uint32_t* __restrict__ px,
+                                 const uint32_t* __restrict__ ofs, uint32_t cl, int flags,
+                                 ClusterOut* __restrict__ out, uint8_t* __restrict__ selectors)
 {
-    typedef LdsU<std::conditional_t<(MaxU < kMaxU), LdsS<MaxU>, LdsT<MaxU>>, Uber> Lds;
-    extern __shared__ __align__(16) uint8_t lds_raw[];
-    Lds& L = *reinterpret_cast<Lds*>(lds_raw);
-    if (blockIdx.x >= *count) return;
-    const uint32_t cl = list[blockIdx.x];
-    const uint32_t lane = lane_id();
+    constexpr uint32_t W = kWavesOf<Class>, T = 64 * W;
+    const uint32_t tid = threadIdx.x;
     const uint32_t p0 = ofs[cl], p1 = ofs[cl + 1];
     const uint32_t n = p1 - p0;
     // DXT1A (qdxt1 with 3-colour blocks): texels with alpha below this are transparent
-    const uint32_t thresh = Uber ? ((uint32_t)perceptual >> 8) & 255u : 0u;
+    const uint32_t thresh = Uber ? ((uint32_t)flags >> 8) & 255u : 0u;
     ClusterOut o{};
     if (!n) {
-        if (lane == 0) out[cl] = o;
+        if (tid == 0) out[cl] = o;
         return;
     }
-    if constexpr (MaxU < kMaxU) {
-        // this class holds at most MaxU texels (dxt1_cluster_classes_kernel)
-        St s;
-        s.perceptual = perceptual & 1;
-        uint32_t opaque = n;
-        s.nu = unique_sorted(L, px, p0, n, thresh, opaque);
-        s.total_w = opaque;
-        s.have_alpha = opaque != n;
-        for (uint32_t i = lane; i < 3 * 64 * 3; i += 64) (&L.pl[0][0][0])[i] = 0;   // over the sort buffers
-        __syncthreads();
-        cluster_search(s, L, px, p0, n, perceptual, cl, out, selectors);
-        return;
-    }
-    else {
-    constexpr uint32_t kHashCap = LdsT<MaxU>::kCapH;
-    for (uint32_t i = lane; i < kHashCap; i += 64) L.hkey[i] = 0;
-    for (uint32_t i = lane; i < 3 * 64 * 3; i += 64) (&L.pl[0][0][0])[i] = 0;
-    __builtin_amdgcn_wave_barrier();
-    // unique colours in first-appearance order (one lane; the order fixes the float sums)
     St s;
-    s.perceptual = perceptual & 1;
-    s.nu = 0;
-    uint32_t opaque = 0;
-    bool overflow = false;
-    if (lane == 0) {
-        for (uint32_t i = 0; i < n; i++) {
-            if ((px[p0 + i] >> 24) < thresh) continue;   // transparent (DXT1A)
-            opaque++;
-            const uint32_t key = (px[p0 + i] & 0x00FFFFFFu) | 0xFF000000u;
-            uint32_t h = hash_slot(L, key);
-            while (L.hkey[h] && L.hkey[h] != key) h = hash_next(L, h);
-            if (L.hkey[h] == key) {
-                L.w[L.hval[h]]++;
-            } else if (s.nu < Lds::kCapU) {
-                L.hkey[h] = key;
-                L.hval[h] = (uint16_t)s.nu;
-                L.col[s.nu] = key & 0x00FFFFFFu;
-                L.w[s.nu] = 1;
-                s.nu++;
-            } else {
-                overflow = true;
-                break;
-            }
+    s.perceptual = flags & 1;
+    uint32_t opaque = n;
+    if constexpr (Class < 4) {
+        // the class's texel count is at most its colour capacity
+        s.nu = unique_sorted<(Class < 3 ? 512u << Class : kMaxU), T>(L, px, p0, n, thresh, opaque);
+    } else {
+        s.nu = unique_hashed<kMaxU, T>(L, px, p0, n, thresh, opaque);
+        if (s.nu > kMaxU) {
+            // more distinct colours than this store holds: left to dxt1_cluster_big_kernel
+            o.flags = kNotEncoded;
+            if (tid == 0) out[cl] = o;
+            return;
         }
     }
-    __builtin_amdgcn_wave_barrier();
-    s.nu = (uint32_t)__shfl((int)s.nu, 0);
-    s.total_w = (uint32_t)__shfl((int)opaque, 0);
-    s.have_alpha = s.total_w != n;
-    overflow = __shfl((int)overflow, 0) != 0;
-    if (overflow) {
-        // more distinct colours than this store holds: left to dxt1_cluster_big_kernel
-        o.flags = kNotEncoded;
-        if (lane == 0) out[cl] = o;
-        return;
-    }
-    cluster_search(s, L, px, p0, n, perceptual, cl, out, selectors);
+    s.total_w = opaque;
+    s.have_alpha = opaque != n;
+    for (uint32_t i = tid; i < 3 * 64 * 3; i += T) (&L.u.pl[0][0][0])[i] = 0;   // over the sort buffers or the hash
+    __syncthreads();
+    cluster_search<LdsU<StoreOf<Class>, Uber>, W>(s, L, px, p0, n, flags, cl, out, selectors);
+}
+
+template <uint32_t Class, bool Uber>
+__global__ void __launch_bounds__(64 * kWavesOf<Class>, 4) dxt1_cluster_kernel(const uint32_t* __restrict__ px,
+                                                                               const uint32_t* __restrict__ ofs,
+                                                                               const uint32_t* __restrict__ list,
+                                                                               const uint32_t* __restrict__ count,
+                                                                               int flags,
+                                                                               ClusterOut* __restrict__ out,
+                                                                               uint8_t* __restrict__ selectors)
+{
+    extern __shared__ __align__(16) uint8_t lds_raw[];
+    LdsU<StoreOf<Class>, Uber>& L = *reinterpret_cast<LdsU<StoreOf<Class>, Uber>*>(lds_raw);
+    if constexpr (Class < 4) {
+        if (blockIdx.x >= *count) return;
+        cluster_of_class<Class, Uber>(L, px, ofs, list[blockIdx.x], flags, out, selectors);
+    } else {
+        // (its list runs downwards)
+        const uint32_t num = *count;
+        for (uint32_t b = blockIdx.x; b < num; b += gridDim.x) {
+            cluster_of_class<Class, Uber>(L, px, ofs, *(list - b), flags, out, selectors);
+            __syncthreads();   // the last reads of L
+        }
     }
 }
 
-// Clusters the LDS pass flagged (more than 4,096 distinct colours), one wave
-// each, with the colour set in global scratch: the cluster's texels own
-// scratch entries [p0, p1) of the texel-sized arrays and [2 p0, 2 p1) of the
-// hash.  The first-appearance order is found in parallel: every texel inserts
-// its colour with compare-and-swap and keeps the smallest texel index and
-// the count per slot, the first texel of each colour is marked, and a prefix
-// count over the marks gives each colour its rank.
+// Clusters the LDS pass flagged (more than 4,096 distinct colours), one
+// workgroup each, with the colour set in global scratch: the cluster's texels
+// own scratch entries [p0, p1) of the texel-sized arrays and [2 p0, 2 p1) of
+// the hash.  The first-appearance order is found in parallel: every texel
+// inserts its colour with compare-and-swap and keeps the smallest texel index
+// and the count per slot, the first texel of each colour is marked, and a
+// prefix count over the marks gives each colour its rank.
 template <bool Uber>
-__global__ void __launch_bounds__(64) dxt1_cluster_big_kernel(const uint32_t* __restrict__ px,
-                                                              const uint32_t* __restrict__ ofs, uint32_t nclusters,
-                                                              int perceptual, ClusterOut* __restrict__ out,
-                                                              uint8_t* __restrict__ selectors,
-                                                              uint8_t* __restrict__ work)
+__global__ void __launch_bounds__(64 * kBigWaves) dxt1_cluster_big_kernel(const uint32_t* __restrict__ px,
+                                                                         const uint32_t* __restrict__ ofs,
+                                                                         uint32_t nclusters, int perceptual,
+                                                                         ClusterOut* __restrict__ out,
+                                                                         uint8_t* __restrict__ selectors,
+                                                                         uint8_t* __restrict__ work)
 {
-    __shared__ GTables T;
+    constexpr uint32_t W = kBigWaves, T = 64 * W;
+    __shared__ GTables G;
     const uint32_t cl = blockIdx.x;
     if (cl >= nclusters || !(out[cl].flags & kNotEncoded)) return;
-    const uint32_t lane = lane_id();
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = uni(tid >> 6);
     const uint32_t p0 = ofs[cl], p1 = ofs[cl + 1], n = p1 - p0, total = ofs[nclusters];
-    LdsU<GStore, Uber> L;
-    L.kCapU = n;
+    LdsU<GStore, Uber> L(G);
     L.kCapH = 2 * n;
     // scratch layout, 37 bytes per texel of all clusters (`total`): u32
     // arrays col, w, mark of `total` entries, hkey, hval, hcnt of 2 * total,
@@ -1428,76 +1959,76 @@ __global__ void __launch_bounds__(64) dxt1_cluster_big_kernel(const uint32_t* __
     uint32_t* base = reinterpret_cast<uint32_t*>(work);
     L.col = base + p0;
     L.w = base + (size_t)total + p0;
-    L.mark = base + 2 * (size_t)total + p0;
+    uint32_t* mark = base + 2 * (size_t)total + p0;
     L.hkey = base + 3 * (size_t)total + 2 * (size_t)p0;
     L.hval = base + 5 * (size_t)total + 2 * (size_t)p0;
-    L.hcnt = base + 7 * (size_t)total + 2 * (size_t)p0;
+    uint32_t* hcnt = base + 7 * (size_t)total + 2 * (size_t)p0;
     L.sel = work + 36 * (size_t)total + p0;
-    L.pl = T.pl;
-    L.rlo = T.rlo;
-    L.rhi = T.rhi;
-    L.glo = T.glo;
-    L.ghi = T.ghi;
-    L.blo = T.blo;
-    L.bhi = T.bhi;
-    for (uint32_t i = lane; i < L.kCapH; i += 64) {
+    for (uint32_t i = tid; i < L.kCapH; i += T) {
         L.hkey[i] = 0;
         L.hval[i] = 0xFFFFFFFFu;
-        L.hcnt[i] = 0;
+        hcnt[i] = 0;
     }
-    for (uint32_t i = lane; i < n; i += 64) L.mark[i] = 0;
-    for (uint32_t i = lane; i < 3 * 64 * 3; i += 64) (&T.pl[0][0][0])[i] = 0;
+    for (uint32_t i = tid; i < n; i += T) mark[i] = 0;
+    for (uint32_t i = tid; i < 3 * 64 * 3; i += T) (&G.u.pl[0][0][0])[i] = 0;
+    if (tid == 0) G.nopaque = 0;
     __threadfence();
     __syncthreads();
     const uint32_t thresh = Uber ? ((uint32_t)perceptual >> 8) & 255u : 0u;
-    uint32_t opaque = 0;
-    for (uint32_t i = lane; i < n; i += 64) {
+    uint32_t nop = 0;
+    for (uint32_t i = tid; i < n; i += T) {
         if ((px[p0 + i] >> 24) < thresh) continue;   // transparent (DXT1A)
-        opaque++;
+        nop++;
         const uint32_t key = (px[p0 + i] & 0x00FFFFFFu) | 0xFF000000u;
-        uint32_t h = hash_slot(L, key);
+        uint32_t h = hash32(key) % L.kCapH;
         for (;;) {
             const uint32_t prev = atomicCAS(&L.hkey[h], 0u, key);
             if (prev == 0u || prev == key) {
                 atomicMin(&L.hval[h], i);
-                atomicAdd(&L.hcnt[h], 1u);
+                atomicAdd(&hcnt[h], 1u);
                 break;
             }
-            h = hash_next(L, h);
+            h = hash_next(L.kCapH, h);
         }
     }
+    atomicAdd(&G.nopaque, nop);
     __threadfence();
     __syncthreads();
-    for (uint32_t h = lane; h < L.kCapH; h += 64)
-        if (L.hkey[h]) L.mark[L.hval[h]] = 1;
+    for (uint32_t h = tid; h < L.kCapH; h += T)
+        if (L.hkey[h]) mark[L.hval[h]] = 1;
     __threadfence();
     __syncthreads();
-    // ranks in texel order: a running count over the marks, 64 texels per step
+    // ranks in texel order: a running count over the marks, T texels per step
     uint32_t base_rank = 0;
-    for (uint32_t i0 = 0; i0 < n; i0 += 64) {
-        const uint32_t i = i0 + lane;
-        const bool m = i < n && L.mark[i];
+    for (uint32_t i0 = 0; i0 < n; i0 += T) {
+        const uint32_t i = i0 + tid;
+        const bool m = i < n && mark[i];
         const uint64_t bal = __ballot(m);
-        const uint32_t r = base_rank + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
-        if (m) {
-            const uint32_t key = (px[p0 + i] & 0x00FFFFFFu) | 0xFF000000u;
-            uint32_t h = hash_slot(L, key);
-            while (L.hkey[h] != key) h = hash_next(L, h);
-            L.col[r] = key & 0x00FFFFFFu;
-            L.w[r] = L.hcnt[h];
-            L.hval[h] = r;
+        if (lane == 0) G.scan[wave] = (uint32_t)__popcll(bal);
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+        for (uint32_t w = 0; w < W; w++) {
+            before += w < wave ? G.scan[w] : 0u;
+            all += G.scan[w];
         }
-        base_rank += (uint32_t)__popcll(bal);
+        if (m) {
+            const uint32_t r = base_rank + before + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
+            const uint32_t key = (px[p0 + i] & 0x00FFFFFFu) | 0xFF000000u;
+            const uint32_t h = hash_find(L.hkey, L.kCapH, key);
+            L.col[r] = key & 0x00FFFFFFu;
+            L.w[r] = hcnt[h];
+        }
+        base_rank += all;
+        __syncthreads();
     }
     __threadfence();
     __syncthreads();
-    for (int off = 32; off; off >>= 1) opaque += (uint32_t)__shfl_xor((int)opaque, off);
     St s;
     s.perceptual = perceptual & 1;
-    s.nu = base_rank;
-    s.total_w = opaque;
-    s.have_alpha = opaque != n;
-    cluster_search(s, L, px, p0, n, perceptual, cl, out, selectors);
+    s.nu = uni(base_rank);
+    s.total_w = uni(G.nopaque);
+    s.have_alpha = s.total_w != n;
+    cluster_search<LdsU<GStore, Uber>, W>(s, L, px, p0, n, perceptual, cl, out, selectors);
 }
 
 }  // namespace
@@ -1537,17 +2068,18 @@ int side_streams(hipStream_t* side, hipEvent_t* fork, hipEvent_t* join)
 }  // namespace
 
 namespace {
-// Scratch of crn2_dxt1_clusters_noalloc_device: four class counters, then four
-// lists of at most kNoAllocMaxClusters cluster indices (1 MiB + 16 B on every
+// Scratch of crn2_dxt1_clusters_noalloc_device: the class counters, then four
+// lists of at most kNoAllocMaxClusters cluster indices (1 MiB + 32 B on every
 // GPU the library runs on, held until the process ends).  Host code never
 // passes the array's name to a kernel: it takes the device address from
 // hipGetSymbolAddress once per device (noalloc_scratch below).
 constexpr uint32_t kNoAllocMaxClusters = 65536;
-__device__ __align__(256) uint32_t scratch[4 + 4 * kNoAllocMaxClusters];
+constexpr uint32_t kCountWords = 8;   // class counters, before the lists
+__device__ __align__(256) uint32_t scratch[kCountWords + 4 * kNoAllocMaxClusters];
 
 __global__ void clear_class_counts_kernel(uint32_t* __restrict__ count)
 {
-    if (threadIdx.x < 4) count[threadIdx.x] = 0;
+    if (threadIdx.x < kCountWords) count[threadIdx.x] = 0;
 }
 
 constexpr int kMaxDevices = 64;
@@ -1558,17 +2090,20 @@ uint32_t* g_noalloc_scratch[kMaxDevices];
 // Per-device set-up: the single-colour tables in device memory, the kernels'
 // LDS limits and the device address of `scratch`.  Idempotent; runs on the
 // device that is current.
+template <uint32_t Class, bool Uber>
+int set_lds_of()
+{
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(&dxt1_cluster_kernel<Class, Uber>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(StoreOf<Class>)) == hipSuccess
+               ? CRN2_OK
+               : CRN2_EHIP;
+}
+
 template <bool Uber>
 int set_lds()
 {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&dxt1_cluster_kernel<512, Uber>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(LdsS<512>)) != hipSuccess ||
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&dxt1_cluster_kernel<1024, Uber>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(LdsS<1024>)) != hipSuccess ||
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&dxt1_cluster_kernel<2048, Uber>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(LdsS<2048>)) != hipSuccess ||
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&dxt1_cluster_kernel<kMaxU, Uber>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(LdsT<kMaxU>)) != hipSuccess)
+    if (set_lds_of<0, Uber>() != CRN2_OK || set_lds_of<1, Uber>() != CRN2_OK || set_lds_of<2, Uber>() != CRN2_OK ||
+        set_lds_of<3, Uber>() != CRN2_OK || set_lds_of<4, Uber>() != CRN2_OK)
         return CRN2_EHIP;
     return CRN2_OK;
 }
@@ -1619,28 +2154,39 @@ int clusters_init(int* dev_out)
     return CRN2_OK;
 }
 
+// One class's launch: a workgroup per cluster of the call, those past the
+// class's count ending at once.  The last class has few clusters and nearly a
+// CU's LDS per workgroup, so idle ones would hold the other classes up: one
+// workgroup per CU takes its clusters in turn.
+template <uint32_t Class, bool Uber>
+void launch_class(const uint32_t* px, const uint32_t* offsets, uint32_t nclusters, const uint32_t* list,
+                  const uint32_t* count, int flags, ClusterOut* o, uint8_t* selectors, hipStream_t st)
+{
+    const uint32_t grid = Class < 4 ? nclusters : std::min(nclusters, 256u);
+    hipLaunchKernelGGL((dxt1_cluster_kernel<Class, Uber>), dim3(grid), dim3(64 * kWavesOf<Class>),
+                       sizeof(StoreOf<Class>), st, px, offsets, list, count + Class, flags, o, selectors);
+}
+
 template <bool Uber>
 void launch_classes(const uint32_t* px, const uint32_t* offsets, uint32_t nclusters, const uint32_t* list,
                     const uint32_t* work, int perceptual, ClusterOut* o, uint8_t* selectors, const hipStream_t* cls)
 {
-    hipLaunchKernelGGL((dxt1_cluster_kernel<kMaxU, Uber>), dim3(nclusters), dim3(64), sizeof(LdsT<kMaxU>), cls[3], px,
-                       offsets, list + 3 * (size_t)nclusters, work + 3, perceptual, o, selectors);
-    hipLaunchKernelGGL((dxt1_cluster_kernel<2048, Uber>), dim3(nclusters), dim3(64), sizeof(LdsS<2048>), cls[2], px,
-                       offsets, list + 2 * (size_t)nclusters, work + 2, perceptual, o, selectors);
-    hipLaunchKernelGGL((dxt1_cluster_kernel<1024, Uber>), dim3(nclusters), dim3(64), sizeof(LdsS<1024>), cls[1], px,
-                       offsets, list + (size_t)nclusters, work + 1, perceptual, o, selectors);
-    hipLaunchKernelGGL((dxt1_cluster_kernel<512, Uber>), dim3(nclusters), dim3(64), sizeof(LdsS<512>), cls[0], px,
-                       offsets, list, work, perceptual, o, selectors);
+    const size_t n = nclusters;
+    launch_class<4, Uber>(px, offsets, nclusters, list + 4 * n - 1, work, perceptual, o, selectors, cls[3]);
+    launch_class<3, Uber>(px, offsets, nclusters, list + 3 * n, work, perceptual, o, selectors, cls[3]);
+    launch_class<2, Uber>(px, offsets, nclusters, list + 2 * n, work, perceptual, o, selectors, cls[2]);
+    launch_class<1, Uber>(px, offsets, nclusters, list + n, work, perceptual, o, selectors, cls[1]);
+    launch_class<0, Uber>(px, offsets, nclusters, list, work, perceptual, o, selectors, cls[0]);
 }
 
-// The search proper.  work: 4 class counters + 4 lists of nclusters entries
-// (device memory).  fork: run the four size classes side by side on helper
+// The search proper.  work: kCountWords class counters + 4 lists of nclusters
+// entries (device memory).  fork: run the classes side by side on helper
 // streams; else every class runs on `st`, in turn (identical results).
 int clusters_run(const void* rgba, const uint32_t* offsets, uint32_t nclusters, int flags, void* out,
                  uint8_t* selectors, hipStream_t st, uint32_t* work, bool fork)
 {
     hipLaunchKernelGGL(clear_class_counts_kernel, dim3(1), dim3(64), 0, st, work);
-    uint32_t* list = work + 4;
+    uint32_t* list = work + kCountWords;
     const uint32_t* px = static_cast<const uint32_t*>(rgba);
     ClusterOut* o = static_cast<ClusterOut*>(out);
     hipLaunchKernelGGL(dxt1_cluster_classes_kernel, dim3((nclusters + 255) / 256), dim3(256), 0, st, offsets,
@@ -1651,8 +2197,8 @@ int clusters_run(const void* rgba, const uint32_t* offsets, uint32_t nclusters, 
     std::unique_lock<std::mutex> lk(g_side_mu, std::defer_lock);
     int rc = CRN2_OK;
     if (fork) {
-        // The four classes run side by side: the large clusters are few and
-        // long, and alone would leave most CUs idle.  Three helper streams
+        // The classes run side by side: the large clusters are few and long, and
+        // alone would leave most CUs idle.  Three helper streams
         // (default priority, created once per device) fork from `st` and join
         // back into it.
         lk.lock();
@@ -1692,11 +2238,11 @@ int clusters_big_pass(const void* rgba, const uint32_t* offsets, uint32_t nclust
     uint8_t* big = nullptr;
     if (hipMallocAsync((void**)&big, 37 * (size_t)total, st) != hipSuccess) return CRN2_ENOMEM;
     if (flags & 2)
-        hipLaunchKernelGGL(dxt1_cluster_big_kernel<true>, dim3(nclusters), dim3(64), 0, st,
+        hipLaunchKernelGGL(dxt1_cluster_big_kernel<true>, dim3(nclusters), dim3(64 * kBigWaves), 0, st,
                            static_cast<const uint32_t*>(rgba), offsets, nclusters, flags & 0xFF01,
                            static_cast<ClusterOut*>(out), selectors, big);
     else
-        hipLaunchKernelGGL(dxt1_cluster_big_kernel<false>, dim3(nclusters), dim3(64), 0, st,
+        hipLaunchKernelGGL(dxt1_cluster_big_kernel<false>, dim3(nclusters), dim3(64 * kBigWaves), 0, st,
                            static_cast<const uint32_t*>(rgba), offsets, nclusters, flags & 1,
                            static_cast<ClusterOut*>(out), selectors, big);
     const int rc = hipGetLastError() == hipSuccess ? CRN2_OK : CRN2_EHIP;
@@ -1714,8 +2260,8 @@ extern "C" int crn2_dxt1_clusters_device(const void* rgba, const uint32_t* offse
     int rc = clusters_init(&dev);
     if (rc != CRN2_OK) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    uint32_t* work = nullptr;      // 4 class counts + 4 lists of nclusters
-    if (hipMallocAsync((void**)&work, (4 + 4 * (size_t)nclusters) * sizeof(uint32_t), st) != hipSuccess)
+    uint32_t* work = nullptr;      // class counts + 4 lists of nclusters
+    if (hipMallocAsync((void**)&work, (kCountWords + 4 * (size_t)nclusters) * sizeof(uint32_t), st) != hipSuccess)
         return CRN2_ENOMEM;
     rc = clusters_run(rgba, offsets, nclusters, flags, out, selectors, st, work, true);
     (void)hipFreeAsync(work, st);

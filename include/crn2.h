@@ -287,10 +287,10 @@ int crn2_dxt1_clusters_device(const void* rgba, const uint32_t* offsets, uint32_
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): crn2_dxt1_clusters_device with the same arguments and
- * results, bit for bit, that allocates nothing.  Its scratch (4 counters and
- * 4 lists of cluster indices) is a fixed array in device memory of 1 MiB per
- * GPU, held until the process ends, so nclusters is at most 65,536
- * (CRN2_EINVAL above).  The four cluster size classes run in turn on `stream`
+ * results, bit for bit, that allocates nothing.  Its scratch (the
+ * counters and lists of cluster indices) is a fixed array in device memory of
+ * 1 MiB per GPU, held until the process ends, so nclusters is at most 65,536
+ * (CRN2_EINVAL above).  The cluster size classes run in turn on `stream`
  * (no helper streams).  Every call on one GPU uses that GPU's one array:
  * calls that overlap on one GPU (other streams, other threads) race and must
  * be serialised by the caller. */

@@ -157,3 +157,38 @@ def test_clusters_with_transparent_texels_match_oracle(gpu):
         assert (lo, hi) == (ores.low, ores.high), c
         assert np.array_equal(sel[ofs[c]:ofs[c + 1]], osel), c
         assert ((int(r["flags"][c]) >> 1) & 1) == ores.alpha_block, c
+
+
+@pytest.mark.parametrize("uber", [False, True])
+@pytest.mark.parametrize("around", [512, 1024, 2048, 4096])
+def test_cluster_class_edges_match_oracle(gpu, around, uber):
+    """Texel counts on either side of each size class's limit, as runs of few
+    colours, as all-different colours and as one colour with an odd one out:
+    the sorted and the hashed colour sets, one to eight waves per cluster, and
+    colour counts off the 32-wide tiles of the scoring."""
+    rng = np.random.default_rng(around + uber)
+    parts = []
+    for n in (around - 1, around, around + 1, around + 33):
+        runs = np.repeat(rng.integers(0, 256, (n // 37 + 1, 4), dtype=np.uint8), 37, axis=0)[:n]
+        parts += [runs, rng.integers(96, 160, (n, 4), dtype=np.uint8)]
+        flat = np.repeat(runs[:1], n, axis=0)
+        flat[n // 2, 1] ^= 0x40
+        parts.append(flat)
+    if around == 4096:
+        few = rng.integers(0, 16, (30000, 4), dtype=np.uint8) * 16                  # every colour of a 16^3 cube
+        parts += [few, np.concatenate([few, np.full((1, 4), 7, np.uint8)])]         # 4,096 and 4,097 colours
+    px = np.concatenate(parts)
+    ofs = np.concatenate([[0], np.cumsum([len(p) for p in parts])]).astype(np.int32)
+    print("clusters around", around, "uber", uber, flush=True)
+    raw, sel = dxt1.encode_clusters_device(torch.from_numpy(px).cuda(), torch.from_numpy(ofs).cuda(), True,
+                                           alpha_blocks=uber)
+    torch.cuda.synchronize()
+    r = raw.cpu().numpy().view(dxt1.CLUSTER_DTYPE).reshape(-1)
+    sel = sel.cpu().numpy()
+    flags = oracle.DXT1_PERCEPTUAL | (oracle.DXT1_ALPHA_BLOCKS if uber else 0)
+    for c, p in enumerate(parts):
+        osel, ores = oracle.dxt1_cluster(p, 4, flags)
+        assert r["nunique"][c] == len(np.unique(p[:, :3], axis=0)), c
+        assert int(r["error"][c]) == ores.error, (c, len(p))
+        assert (int(r["lo_hi"][c] & 0xFFFF), int(r["lo_hi"][c] >> 16)) == (ores.low, ores.high), c
+        assert np.array_equal(sel[ofs[c]:ofs[c + 1]], osel), c
