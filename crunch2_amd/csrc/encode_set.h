@@ -43,6 +43,8 @@ int crn2_dxt1_set_prepare(void);
 // threads, each thread taking elements begin + tid, + grid * tb, ... (internal).
 int crn2_dxt1_set_launch(const crn2::SetJob* jobs, uint32_t njobs, uint64_t begin, uint64_t end, int quality,
                          uint32_t grid, uint32_t tb, hipStream_t stream);
+// The alpha kernel's waves take runs of `per` elements (crn2_dxt5a_set_per_wave).
+uint32_t crn2_dxt5a_set_per_wave(uint64_t elements);
 int crn2_dxt5a_set_launch(const crn2::SetJob* jobs, uint32_t njobs, uint64_t begin, uint64_t end, int quality,
-                          uint32_t grid, uint32_t tb, hipStream_t stream);
+                          uint32_t per, uint32_t grid, uint32_t tb, hipStream_t stream);
 }

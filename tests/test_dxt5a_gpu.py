@@ -38,3 +38,22 @@ def test_image_encode_matches_oracle(gpu, w, h, comp):
         (sel.astype(np.uint64) << shifts[None, :]).sum(1).astype(np.uint64) << np.uint64(16))
     assert np.array_equal(blocks, exp)
     assert np.array_equal(err.cpu().numpy().view(np.uint64), e)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 32768 * 2 + 1, 32768 * 3 + 3])
+@pytest.mark.parametrize("quality", [1, 4])
+def test_runs_of_blocks_match_oracle(gpu, n, quality):
+    """Block counts around the lengths of the runs that a wave takes, with
+    blocks of one, two, three and many values side by side."""
+    print("dxt5a runs", n, quality, flush=True)
+    rng = np.random.default_rng(n + quality)
+    few = rng.integers(0, 256, (n, 3))
+    kinds = rng.integers(1, 4, n) if n > 1000 else rng.integers(1, 5, n)
+    b = few[np.arange(n)[:, None], rng.integers(0, np.minimum(kinds, 3)[:, None], (n, 16))]
+    many = np.nonzero(kinds == 4)[0] if n <= 1000 else np.arange(0, n, 997)
+    b[many] = rng.integers(0, 256, (len(many), 16))
+    b = np.ascontiguousarray(b, np.uint8)
+    ref = oracle.dxt5a_blocks(b, quality, True)
+    got = dxt5a.compute_blocks(b, quality, True)
+    for k, name in enumerate(("selectors", "error", "first", "second", "type", "reordered")):
+        assert np.array_equal(np.asarray(got[k]), np.asarray(ref[k])), name
