@@ -9,14 +9,16 @@
 // (crn_dxt1.cpp:1370-1592, weights 8/25/1 from crn_color.h:724-726).
 //
 // Model: 57 -> 128 -> 128 -> 7, tanh-form GELU, weights and layer inputs in
-// bfloat16, sums in float32.  Training runs layer by layer through a strided
-// FP32 GEMM (bf16 rounding of the operands on load), bias/GELU kernels, the
-// loss kernel and Adam; inference is one fused kernel on
+// bfloat16, sums in float32.  Training is one fused kernel for the batch's loss
+// and gradient and Adam; the layer-by-layer pieces (a strided FP32 GEMM with
+// bf16 rounding of the operands on load, bias/GELU and loss kernels) stand as
+// entry points of their own; inference is one fused kernel on
 // v_mfma_f32_32x32x16_bf16 (a wave owns 32 blocks, weights staged in LDS).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstdint>
+#include <mutex>
 
 #include "crn2_internal.h"
 
@@ -200,6 +202,308 @@ __global__ void __launch_bounds__(256) mlp_loss_kernel(const float* __restrict__
     if (threadIdx.x == 0) atomicAdd(loss, red[0] / (float)rows);
 }
 
+// ------------------------------------------------- fused training gradient
+// Loss and gradient of a batch in one pass over its rows: a workgroup of four
+// waves takes R rows at a time through forward, loss and backward with every
+// layer in LDS or registers, keeps its part of the gradient in registers over
+// all its rows, and writes it once; mlp_grad_reduce_kernel adds the
+// workgroups' parts in a fixed order.
+//   forward: bfloat16 operands on v_mfma_f32_32x32x16_bf16; wave w computes
+//     columns 32 w .. of a layer and keeps gelu'(z) of its outputs;
+//   backward: float32 operands on v_mfma_f32_32x32x2_f32 (the gradients stay
+//     in float32, the bfloat16-rounded weights and activations are exact in
+//     it); the product's layout is that of the kept gelu'(z).
+// X carries a column of ones behind its 57 features (its weights are zero), so
+// that layer 1's bias gradient is a row of its weight gradient.
+// What bounds it: the float32 matrix products (64 cycles each) of the four
+// waves of each CU.  As 15 launches of a strided vector GEMM and elementwise
+// kernels 32,768 rows took 1,290 us, now 80 us (262,144 rows: 6,194, now 523).
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr uint32_t kInPad = 64;               // K of layer 1 (57 features + zeros)
+constexpr uint32_t kOutPad = 32;              // N of layer 3 (7 outputs + zeros)
+constexpr uint32_t kXs = kInPad + 8;          // LDS row strides (bf16 elements), padded against bank conflicts
+constexpr uint32_t kHs = kHid + 8;
+constexpr uint32_t kParams = kIn * kHid + kHid + kHid * kHid + kHid + kHid * kOut + kOut;
+constexpr uint32_t kPartial = kParams + 1;    // a workgroup's part: the gradient, then the loss
+constexpr uint32_t kDzs = kHid + 5;           // float row stride: an odd step between rows and columns alike
+constexpr uint32_t kMaxGradWgs = 256;
+
+__device__ inline bf16x8 lds_bf16x8(const uint8_t* lds, uint32_t byte_ofs)
+{
+    return *reinterpret_cast<const bf16x8*>(lds + byte_ofs);
+}
+
+__device__ inline __bf16 to_bf16(float x)
+{
+    const uint32_t u = __float_as_uint(bf16_round(x)) >> 16;
+    return __builtin_bit_cast(__bf16, (uint16_t)u);
+}
+
+__device__ inline float from_bf16(__bf16 x)
+{
+    return __uint_as_float((uint32_t)__builtin_bit_cast(uint16_t, x) << 16);
+}
+
+template <uint32_t R>
+struct GradLds {
+    __bf16 w1[kHid][kXs];       // W1 transposed: [n][k]
+    __bf16 w2[kHid][kHs];
+    __bf16 w3[kOutPad][kHs];
+    float bias[2 * kHid + 8];
+    __bf16 x[R][kXs];
+    __bf16 a1[R][kHs];
+    __bf16 a2[R][kHs];
+    float y[R][8];              // outputs, then their gradient
+    float dz[R][kDzs];
+};
+
+// gelu and its derivative from one tanh
+__device__ inline void gelu_both(float z, float& a, float& g)
+{
+    const float t = tanhf(kGeluC * (z + kGeluA * z * z * z));
+    const float du = kGeluC * (1.0f + 3.0f * kGeluA * z * z);
+    a = 0.5f * z * (1.0f + t);
+    g = 0.5f * (1.0f + t) + 0.5f * z * (1.0f - t * t) * du;
+}
+
+// One layer's columns c0 .. c0 + 31 of R rows: z = in W + b, its activation
+// into `out` and gelu'(z) into g (row 32 m + 8 (i / 4) + 4 half + i % 4 of
+// register i).
+template <uint32_t R, uint32_t KS>
+__device__ inline void grad_layer(const __bf16* in, uint32_t is, const __bf16* w, uint32_t ws, const float* bias,
+                                  uint32_t c0, __bf16 (*out)[kHs], float (*g)[16])
+{
+    const uint32_t lane = threadIdx.x & 63u, half = lane >> 5, col = lane & 31u;
+    f32x16 acc[R / 32];
+#pragma unroll
+    for (uint32_t m = 0; m < R / 32; m++) acc[m] = f32x16{0};
+#pragma unroll
+    for (uint32_t ks = 0; ks < KS; ks++) {
+        const uint32_t k = 16 * ks + 8 * half;
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(w + (c0 + col) * ws + k);
+#pragma unroll
+        for (uint32_t m = 0; m < R / 32; m++) {
+            const bf16x8 a = *reinterpret_cast<const bf16x8*>(in + (32 * m + col) * is + k);
+            acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[m], 0, 0, 0);
+        }
+    }
+    const float bc = bias[c0 + col];
+#pragma unroll
+    for (uint32_t m = 0; m < R / 32; m++)
+#pragma unroll
+        for (uint32_t i = 0; i < 16; i++) {
+            float act;
+            gelu_both(acc[m][i] + bc, act, g[m][i]);
+            out[32 * m + 8 * (i >> 2) + 4 * half + (i & 3)][c0 + col] = to_bf16(act);
+        }
+}
+
+template <uint32_t R>
+__global__ void __launch_bounds__(256) mlp_grad_kernel(const float* __restrict__ X, const float* __restrict__ T,
+                                                       const float* __restrict__ labels, uint32_t rows,
+                                                       const float* __restrict__ theta, float* __restrict__ part)
+{
+    extern __shared__ __align__(16) uint8_t lds[];
+    GradLds<R>& L = *reinterpret_cast<GradLds<R>*>(lds);
+    constexpr uint32_t M = R / 32;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, half = lane >> 5, col = lane & 31u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), c0 = 32 * wave;
+    const float* W1 = theta;
+    const float* b1 = W1 + kIn * kHid;
+    const float* W2 = b1 + kHid;
+    const float* b2 = W2 + kHid * kHid;
+    const float* W3 = b2 + kHid;
+    const float* b3 = W3 + kHid * kOut;
+    // weights (bf16, transposed so that a column is contiguous in K)
+#pragma unroll 8
+    for (uint32_t e = tid; e < kIn * kHid; e += 256) L.w1[e & 127u][e >> 7] = to_bf16(W1[e]);
+    for (uint32_t e = tid; e < (kXs - kIn) * kHid; e += 256) L.w1[e & 127u][kIn + (e >> 7)] = to_bf16(0.0f);
+#pragma unroll 8
+    for (uint32_t e = tid; e < kHid * kHid; e += 256) L.w2[e & 127u][e >> 7] = to_bf16(W2[e]);
+    for (uint32_t e = tid; e < kOutPad * kHs; e += 256) {
+        const uint32_t o = e / kHs, k = e % kHs;
+        L.w3[o][k] = to_bf16(k < kHid && o < kOut ? W3[k * kOut + o] : 0.0f);
+    }
+    for (uint32_t e = tid; e < 2 * kHid + 8; e += 256)
+        L.bias[e] = e < kHid ? b1[e] : e < 2 * kHid ? b2[e - kHid] : (e - 2 * kHid < kOut ? b3[e - 2 * kHid] : 0.0f);
+
+    f32x16 g1[2], g2[4], g3;     // gradient tiles: W1 (both k tiles) x columns c0, W2 k tile c0 x all, W3 k tile c0
+#pragma unroll
+    for (uint32_t t = 0; t < 2; t++) g1[t] = f32x16{0};
+#pragma unroll
+    for (uint32_t t = 0; t < 4; t++) g2[t] = f32x16{0};
+    g3 = f32x16{0};
+    float db2 = 0.0f, db3 = 0.0f, loss = 0.0f;
+    const float inv = 1.0f / (float)rows;
+    const uint32_t tiles = (rows + R - 1) / R;
+    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const uint32_t r0 = tile * R;
+        __syncthreads();   // the previous tile's last reads (and the weights)
+#pragma unroll 4
+        for (uint32_t e = tid; e < R * kInPad; e += 256) {
+            const uint32_t r = e >> 6, k = e & 63u;
+            const float v = k < kIn && r0 + r < rows ? X[(size_t)(r0 + r) * kIn + k] : (k == kIn ? 1.0f : 0.0f);
+            L.x[r][k] = to_bf16(v);
+        }
+        __syncthreads();
+        float p1[M][16], p2[M][16];
+        grad_layer<R, kInPad / 16>(&L.x[0][0], kXs, &L.w1[0][0], kXs, L.bias, c0, L.a1, p1);
+        __syncthreads();
+        grad_layer<R, kHid / 16>(&L.a1[0][0], kHs, &L.w2[0][0], kHs, L.bias + kHid, c0, L.a2, p2);
+        __syncthreads();
+        if (wave < M) {
+            f32x16 acc = {0};
+#pragma unroll
+            for (uint32_t ks = 0; ks < kHid / 16; ks++) {
+                const uint32_t k = 16 * ks + 8 * half;
+                const bf16x8 a = *reinterpret_cast<const bf16x8*>(&L.a2[32 * wave + col][k]);
+                const bf16x8 b = *reinterpret_cast<const bf16x8*>(&L.w3[col][k]);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+            }
+            if (col < 8) {
+                const float bc = L.bias[2 * kHid + col];
+#pragma unroll
+                for (uint32_t i = 0; i < 16; i++) L.y[32 * wave + 8 * (i >> 2) + 4 * half + (i & 3)][col] = acc[i] + bc;
+            }
+        }
+        __syncthreads();
+        // the loss and its gradient, one row per lane (mlp_loss_kernel's formulas)
+        if (tid < R) {
+            const uint32_t r = r0 + tid;
+            float dy[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            if (r < rows) {
+                const float scale[6] = {31, 63, 31, 31, 63, 31};
+                bool ok = true;
+                for (int k = 0; k < 6; k++) {
+                    const float y = L.y[tid][k], t = T[(size_t)r * 6 + k];
+                    const float d = y - t;
+                    loss += d * d;
+                    dy[k] = 2.0f * inv * d;
+                    const float q = fminf(fmaxf(rintf(y * scale[k]), 0.0f), scale[k]);
+                    ok &= fabsf(q - rintf(t * scale[k])) <= 1.0f;
+                }
+                const float lab = labels ? labels[r] : (ok ? 1.0f : 0.0f);
+                const float z = L.y[tid][6];
+                const float sg = 1.0f / (1.0f + expf(-z));
+                loss += kConfWeight * (fmaxf(z, 0.0f) + log1pf(expf(-fabsf(z))) - lab * z);
+                dy[6] = kConfWeight * inv * (sg - lab);
+            }
+            for (int k = 0; k < 8; k++) L.y[tid][k] = dy[k];
+        }
+        __syncthreads();
+        // dA2 = dY W3^T, dZ2 = dA2 gelu'(Z2)
+#pragma unroll
+        for (uint32_t m = 0; m < M; m++) {
+            f32x16 acc = {0};
+#pragma unroll
+            for (uint32_t o = 0; o < 8; o += 2)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(L.y[32 * m + col][o + half],
+                                                           from_bf16(L.w3[o + half][c0 + col]), acc, 0, 0, 0);
+#pragma unroll
+            for (uint32_t i = 0; i < 16; i++)
+                L.dz[32 * m + 8 * (i >> 2) + 4 * half + (i & 3)][c0 + col] = acc[i] * p2[m][i];
+        }
+        // dW3 and db3
+#pragma unroll 8
+        for (uint32_t r = 0; r < R; r += 2)
+            g3 = __builtin_amdgcn_mfma_f32_32x32x2f32(from_bf16(L.a2[r + half][c0 + col]),
+                                                      col < 8 ? L.y[r + half][col & 7u] : 0.0f, g3, 0, 0, 0);
+        if (tid >= 128 && tid < 128 + kOut)
+            for (uint32_t r = 0; r < R; r++) db3 += L.y[r][tid - 128];
+        __syncthreads();
+        // dW2 and db2
+#pragma unroll 4
+        for (uint32_t r = 0; r < R; r += 2) {
+            const float a = from_bf16(L.a1[r + half][c0 + col]);
+#pragma unroll
+            for (uint32_t t = 0; t < 4; t++)
+                g2[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, L.dz[r + half][32 * t + col], g2[t], 0, 0, 0);
+        }
+        if (tid < kHid)
+            for (uint32_t r = 0; r < R; r++) db2 += L.dz[r][tid];
+        // dA1 = dZ2 W2^T, dZ1 = dA1 gelu'(Z1)
+        {
+            f32x16 acc[M];
+#pragma unroll
+            for (uint32_t m = 0; m < M; m++) acc[m] = f32x16{0};
+#pragma unroll 8
+            for (uint32_t n = 0; n < kHid; n += 2) {
+                const float b = from_bf16(L.w2[n + half][c0 + col]);
+#pragma unroll
+                for (uint32_t m = 0; m < M; m++)
+                    acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(L.dz[32 * m + col][n + half], b, acc[m], 0, 0, 0);
+            }
+            __syncthreads();   // dZ2 has been read
+#pragma unroll
+            for (uint32_t m = 0; m < M; m++)
+#pragma unroll
+                for (uint32_t i = 0; i < 16; i++)
+                    L.dz[32 * m + 8 * (i >> 2) + 4 * half + (i & 3)][c0 + col] = acc[m][i] * p1[m][i];
+        }
+        __syncthreads();
+        // dW1, and db1 in row 57
+#pragma unroll 4
+        for (uint32_t r = 0; r < R; r += 2) {
+            const float b = L.dz[r + half][c0 + col];
+#pragma unroll
+            for (uint32_t t = 0; t < 2; t++)
+                g1[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(from_bf16(L.x[r + half][32 * t + col]), b, g1[t], 0, 0, 0);
+        }
+    }
+    // this workgroup's part, laid out as the parameters
+    float* P = part + (size_t)blockIdx.x * kPartial;
+#pragma unroll
+    for (uint32_t i = 0; i < 16; i++) {
+        const uint32_t row = 8 * (i >> 2) + 4 * half + (i & 3);
+#pragma unroll
+        for (uint32_t t = 0; t < 2; t++) {
+            const uint32_t k = 32 * t + row;
+            if (k <= kIn) P[k * kHid + c0 + col] = g1[t][i];   // row 57: b1 follows W1
+        }
+#pragma unroll
+        for (uint32_t t = 0; t < 4; t++) P[(kIn + 1) * kHid + (c0 + row) * kHid + 32 * t + col] = g2[t][i];
+        if (col < kOut) P[(kIn + 2 + kHid) * kHid + (c0 + row) * kOut + col] = g3[i];
+    }
+    if (tid < kHid) P[(kIn + 1 + kHid) * kHid + tid] = db2;
+    if (tid >= 128 && tid < 128 + kOut) P[kParams - kOut + tid - 128] = db3;
+    if (tid < 64) {
+        for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
+        if (tid == 0) P[kParams] = loss;
+    }
+}
+
+// Sums of the workgroups' parts, in order within each of four quarters; the
+// last sum is the loss over the batch.
+__global__ void __launch_bounds__(256) mlp_grad_reduce_kernel(const float* __restrict__ part, uint32_t n,
+                                                              float* __restrict__ g, float* __restrict__ loss,
+                                                              uint32_t rows)
+{
+    __shared__ float s[4][64];
+    const uint32_t q = threadIdx.x >> 6, lane = threadIdx.x & 63u, e = blockIdx.x * 64 + lane;
+    const uint32_t per = (n + 3) / 4, k0 = min(q * per, n), k1 = min(k0 + per, n);
+    float v = 0.0f;
+    if (e < kPartial) {
+#pragma unroll 8
+        for (uint32_t k = k0; k < k1; k++) v += part[(size_t)k * kPartial + e];
+    }
+    s[q][lane] = v;
+    __syncthreads();
+    if (q == 0 && e < kPartial) {
+        const float t = (s[0][lane] + s[1][lane]) + (s[2][lane] + s[3][lane]);
+        if (e < kParams) g[e] = t;
+        else *loss = t / (float)rows;
+    }
+}
+
+// Rows per workgroup step: 32 while that still leaves CUs without work at 64.
+inline uint32_t grad_rows(uint32_t n) { return n <= 32 * kMaxGradWgs ? 32u : 64u; }
+inline uint32_t grad_wgs(uint32_t n)
+{
+    return std::min<uint32_t>(kMaxGradWgs, (uint32_t)(((uint64_t)n + grad_rows(n) - 1) / grad_rows(n)));
+}
+
 __global__ void __launch_bounds__(256) adam_kernel(float* __restrict__ w, const float* __restrict__ g,
                                                    float* __restrict__ m, float* __restrict__ v, uint32_t n, float lr,
                                                    float b1, float b2, float eps, float c1, float c2)
@@ -215,13 +519,6 @@ __global__ void __launch_bounds__(256) adam_kernel(float* __restrict__ w, const 
 }
 
 // ------------------------------------------------- matrix-core inference
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-constexpr uint32_t kInPad = 64;               // K of layer 1 (57 features + zeros)
-constexpr uint32_t kOutPad = 32;              // N of layer 3 (7 outputs + zeros)
-constexpr uint32_t kXs = kInPad + 8;          // LDS row strides (bf16 elements), padded against bank conflicts
-constexpr uint32_t kHs = kHid + 8;
 constexpr uint32_t kInferWaves = 4;
 // LDS layout (bytes)
 constexpr uint32_t kW1Ofs = 0;                                    // [128][kXs]  W1 transposed (n-major, k contiguous)
@@ -231,17 +528,6 @@ constexpr uint32_t kBOfs = kW3Ofs + kOutPad * kHs * 2;            // biases: 128
 constexpr uint32_t kWaveOfs = kBOfs + (2 * kHid + kOutPad) * 4;   // per wave: two [32][kHs] buffers
 constexpr uint32_t kWaveBytes = 2 * 32 * kHs * 2;
 constexpr uint32_t kInferLds = kWaveOfs + kInferWaves * kWaveBytes;
-
-__device__ inline bf16x8 lds_bf16x8(const uint8_t* lds, uint32_t byte_ofs)
-{
-    return *reinterpret_cast<const bf16x8*>(lds + byte_ofs);
-}
-
-__device__ inline __bf16 to_bf16(float x)
-{
-    const uint32_t u = __float_as_uint(bf16_round(x)) >> 16;
-    return __builtin_bit_cast(__bf16, (uint16_t)u);
-}
 
 // One layer for the wave's 32 rows: in [32][ks] bf16 (row stride `is`), out
 // written as bf16(gelu(z)) into [32][os] or, for the last layer, z to `y`.
@@ -822,6 +1108,43 @@ int crn2_mlp_loss_device(const float* Y, const float* T, const float* labels, ui
     if (!rows) return CRN2_OK;
     hipLaunchKernelGGL(mlp_loss_kernel, dim3(grid1(rows, 256)), dim3(256), 0, static_cast<hipStream_t>(stream), Y, T,
                        labels, rows, dY, loss);
+    return hipGetLastError() == hipSuccess ? CRN2_OK : CRN2_EHIP;
+}
+
+uint64_t crn2_mlp_gradients_work(uint32_t rows) { return rows ? (uint64_t)grad_wgs(rows) * kPartial : 0; }
+
+int crn2_mlp_gradients_device(const float* X, const float* T, const float* labels, uint32_t rows, const float* theta,
+                              float* g, float* loss, float* work, uint64_t work_floats, void* stream)
+{
+    if (!theta || !g || !loss || (rows && (!X || !T || !work || work_floats < crn2_mlp_gradients_work(rows))))
+        return CRN2_EINVAL;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const uint32_t wgs = rows ? grad_wgs(rows) : 0;
+    if (rows) {
+        // the LDS limit is a property of the kernel on each device: set it once per device
+        static std::once_flag once[64];
+        static bool ready[64];
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return CRN2_EHIP;
+        std::call_once(once[dev], [&] {
+            ready[dev] = hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_grad_kernel<32>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)sizeof(GradLds<32>)) == hipSuccess &&
+                         hipFuncSetAttribute(reinterpret_cast<const void*>(&mlp_grad_kernel<64>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)sizeof(GradLds<64>)) == hipSuccess;
+        });
+        if (!ready[dev]) return CRN2_EHIP;
+        if (grad_rows(rows) == 32)
+            hipLaunchKernelGGL(mlp_grad_kernel<32>, dim3(wgs), dim3(256), sizeof(GradLds<32>), st, X, T, labels, rows,
+                               theta, work);
+        else
+            hipLaunchKernelGGL(mlp_grad_kernel<64>, dim3(wgs), dim3(256), sizeof(GradLds<64>), st, X, T, labels, rows,
+                               theta, work);
+        if (hipGetLastError() != hipSuccess) return CRN2_EHIP;
+    }
+    hipLaunchKernelGGL(mlp_grad_reduce_kernel, dim3((kPartial + 63) / 64), dim3(256), 0, st, work, wgs, g, loss,
+                       rows ? rows : 1u);
     return hipGetLastError() == hipSuccess ? CRN2_OK : CRN2_EHIP;
 }
 

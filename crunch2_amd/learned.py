@@ -75,7 +75,6 @@ class Trainer:
         self.v = torch.zeros_like(self.theta)
         self.g = torch.zeros_like(self.theta)
         self.loss = torch.zeros(1, dtype=torch.float32, device=self.dev)
-        self.ones = torch.ones(1, dtype=torch.float32, device=self.dev)
         self.lr = lr
         self.step_no = 0
         self._bufs = {}
@@ -91,41 +90,12 @@ class Trainer:
         """Loss and flat gradient of the batch (X: n x 57, T: n x 6 float32;
         labels: optional n float32 confidence labels)."""
         n = X.shape[0]
-        th, o = self.theta, OFFSETS
-        Z1, A1 = self._buf("Z1", (n, N_H)), self._buf("A1", (n, N_H))
-        Z2, A2 = self._buf("Z2", (n, N_H)), self._buf("A2", (n, N_H))
-        Y, dY = self._buf("Y", (n, N_OUT)), self._buf("dY", (n, N_OUT))
-        dA, dZ = self._buf("dA", (n, N_H)), self._buf("dZ", (n, N_H))
-        s = _s()
         L = lib()
-        # forward
-        gemm(n, N_H, N_IN, X, N_IN, 1, th, N_H, 1, Z1, N_H, round_a=True, round_b=True, b_ofs=o["W1"])
-        check(L.crn2_mlp_bias_act_device(_p(Z1), _p(A1), C.c_void_p(th.data_ptr() + 4 * o["b1"]), n, N_H, 1, s),
-              "bias_act")
-        gemm(n, N_H, N_H, A1, N_H, 1, th, N_H, 1, Z2, N_H, round_b=True, b_ofs=o["W2"])
-        check(L.crn2_mlp_bias_act_device(_p(Z2), _p(A2), C.c_void_p(th.data_ptr() + 4 * o["b2"]), n, N_H, 1, s),
-              "bias_act")
-        gemm(n, N_OUT, N_H, A2, N_H, 1, th, N_OUT, 1, Y, N_OUT, round_b=True, b_ofs=o["W3"])
-        check(L.crn2_mlp_bias_act_device(_p(Y), _p(Y), C.c_void_p(th.data_ptr() + 4 * o["b3"]), n, N_OUT, 0, s),
-              "bias_act")
-        self.loss.zero_()
-        lp = C.c_void_p(labels.data_ptr()) if labels is not None else C.c_void_p(0)
-        check(L.crn2_mlp_loss_device(_p(Y), _p(T), lp, n, _p(dY), _p(self.loss), s), "loss")
-        # backward
-        g = self.g
-        g.zero_()
-        ks = max(1, min(64, n // 1024))
-        gemm(N_H, N_OUT, n, A2, 1, N_H, dY, N_OUT, 1, g, N_OUT, ksplit=ks, c_ofs=o["W3"])
-        gemm(1, N_OUT, n, self.ones, 0, 0, dY, N_OUT, 1, g, N_OUT, ksplit=ks, c_ofs=o["b3"])
-        gemm(n, N_H, N_OUT, dY, N_OUT, 1, th, 1, N_OUT, dA, N_H, round_b=True, b_ofs=o["W3"])
-        check(L.crn2_mlp_gelu_back_device(_p(dA), _p(Z2), _p(dZ), n * N_H, s), "gelu_back")
-        gemm(N_H, N_H, n, A1, 1, N_H, dZ, N_H, 1, g, N_H, ksplit=ks, c_ofs=o["W2"])
-        gemm(1, N_H, n, self.ones, 0, 0, dZ, N_H, 1, g, N_H, ksplit=ks, c_ofs=o["b2"])
-        gemm(n, N_H, N_H, dZ, N_H, 1, th, 1, N_H, dA, N_H, round_b=True, b_ofs=o["W2"])
-        check(L.crn2_mlp_gelu_back_device(_p(dA), _p(Z1), _p(dZ), n * N_H, s), "gelu_back")
-        gemm(N_IN, N_H, n, X, 1, N_IN, dZ, N_H, 1, g, N_H, round_a=True, ksplit=ks, c_ofs=o["W1"])
-        gemm(1, N_H, n, self.ones, 0, 0, dZ, N_H, 1, g, N_H, ksplit=ks, c_ofs=o["b1"])
-        return self.loss, g
+        size = int(L.crn2_mlp_gradients_work(n))
+        work = self._buf("work", (size,)) if size else None
+        check(L.crn2_mlp_gradients_device(_p(X), _p(T), _p(labels), n, _p(self.theta), _p(self.g), _p(self.loss),
+                                          _p(work), size, _s()), "crn2_mlp_gradients_device")
+        return self.loss, self.g
 
     def step(self, X, T, labels=None):
         loss, g = self.gradients(X, T, labels)

@@ -536,6 +536,16 @@ int crn2_mlp_gelu_back_device(const float* dA, const float* Z, float* dZ, uint64
  * endpoint component within one step"; writes dY, adds the loss into *loss. */
 int crn2_mlp_loss_device(const float* Y, const float* T, const float* labels, uint32_t rows, float* dY, float* loss,
                          void* stream);
+/* Loss and gradient of one batch in two launches, without keeping the layers'
+ * values: X rows x 57 features, T rows x 6 targets, labels rows floats or NULL
+ * (as crn2_mlp_loss_device), theta the 24,839 parameters (W1, b1, W2, b2, W3,
+ * b3, row-major).  Writes the 24,839 gradients and the loss (both overwritten,
+ * sums in a fixed order).  work: device scratch of at least
+ * crn2_mlp_gradients_work(rows) floats (at most 25 MB), free again when the
+ * launches have run. */
+uint64_t crn2_mlp_gradients_work(uint32_t rows);
+int crn2_mlp_gradients_device(const float* X, const float* T, const float* labels, uint32_t rows, const float* theta,
+                              float* g, float* loss, float* work, uint64_t work_floats, void* stream);
 /* Adam step `step` (1-based) on n parameters. */
 int crn2_adam_device(float* w, const float* g, float* m, float* v, uint32_t n, float lr, float b1, float b2, float eps,
                      uint32_t step, void* stream);

@@ -82,6 +82,29 @@ def test_gradients_with_given_labels_match_oracle(gpu):
     assert abs(float(g2[-1].item()) - float(g[-1])) > 1e-6
 
 
+@pytest.mark.parametrize("n", [1, 31, 33, 63, 65, 8192, 8193, 16385])
+def test_gradients_at_tile_edges(gpu, n):
+    """Row counts around the 32- and 64-row steps, the switch between them and
+    the largest grid, against the oracle; the same batch twice gives the same
+    bits.  The error is that of activations that round to the other bfloat16
+    neighbour (2^-9 of one of 128 terms), so the bounds are those of the other
+    gradient tests."""
+    print("gradients", n, flush=True)
+    blocks = dxt1.image_blocks(texture.synth(520, 520, n, texture.RGB))[:n]
+    t = np.random.default_rng(n).random((n, 6)).astype(np.float32)
+    theta = omlp.init_params(n)
+    tr = learned.Trainer(dev(theta))
+    x = learned.features(dev(blocks))
+    loss, g = tr.gradients(x, dev(t))
+    one = (float(loss.item()), g.cpu().numpy().copy())
+    ref_loss, ref_g = omlp.loss_and_grads(theta, x.cpu().numpy(), t)
+    assert abs(one[0] - ref_loss) <= 1e-4 * max(1.0, abs(ref_loss))
+    cos = float(one[1] @ ref_g / (np.linalg.norm(one[1]) * np.linalg.norm(ref_g)))
+    assert cos > 0.99999 and np.abs(one[1] - ref_g).max() / np.abs(ref_g).max() < 1e-3
+    loss, g = tr.gradients(x, dev(t))
+    assert float(loss.item()) == one[0] and np.array_equal(g.cpu().numpy(), one[1])
+
+
 def test_inference_matches_oracle(gpu):
     blocks, _ = training_batch(700, 4)
     theta = omlp.init_params(11)
