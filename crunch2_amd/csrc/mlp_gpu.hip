@@ -800,43 +800,6 @@ __device__ inline uint32_t refine_from(const int (*px)[3], int (*e)[3], uint32_t
     return best;
 }
 
-// Best improving move among all 728 combinations of -1 / 0 / +1 on the six
-// endpoint components (refine_solution's both-ends lattice,
-// crnlib/crn_dxt1.cpp:601-643); false if none improves.
-__device__ inline bool box_step(const int (*px)[3], int (*e)[3], uint32_t& best)
-{
-    const int lim[3] = {31, 63, 31};
-    uint32_t cand = best;
-    int bm = -1;
-    for (int m = 0; m < 729; m++) {
-        if (m == 364) continue;   // all zero
-        int f[2][3];
-        int r = m;
-        bool ok = true;
-        for (int s = 0; s < 2; s++)
-            for (int k = 0; k < 3; k++) {
-                const int v = e[s][k] + (r % 3) - 1;
-                r /= 3;
-                ok &= v >= 0 && v <= lim[k];
-                f[s][k] = v;
-            }
-        if (!ok) continue;
-        const uint32_t er = pair_error_below(px, f[0], f[1], cand);
-        if (er < cand) {
-            cand = er;
-            bm = m;
-        }
-    }
-    if (bm < 0) return false;
-    for (int s = 0; s < 2; s++)
-        for (int k = 0; k < 3; k++) {
-            e[s][k] += (bm % 3) - 1;
-            bm /= 3;
-        }
-    best = cand;
-    return true;
-}
-
 // Principal-axis start: the extreme projections of the texels on the
 // dominant eigenvector of their covariance (power iteration).
 __device__ inline void pca_start(const int (*px)[3], int (*e)[3])
@@ -883,70 +846,48 @@ __device__ inline void pca_start(const int (*px)[3], int (*e)[3])
     }
 }
 
-// Sorts the 16 texels by falling error under endpoints e (a fixed sorting
-// network: the texels stay in registers); nibble i of *perm becomes the
-// original index of texel i.
-__device__ inline void order_texels(int (*px)[3], const int (*e)[3], uint64_t* perm)
+__device__ inline void net_start(const float* y, int (*e)[3])
 {
-    *perm = 0xFEDCBA9876543210ull;
-    uint32_t lo, hi;
-    {
-        const uint32_t ca = pack565(e[0]), cb = pack565(e[1]);
-        lo = ca > cb ? ca : cb;
-        hi = ca > cb ? cb : ca;
-    }
-    int p[4][3];
-    expand565(lo, p[0]);
-    expand565(hi, p[1]);
-    const bool four = lo > hi;
-    for (int k = 0; k < 3; k++) {
-        p[2][k] = four ? (2 * p[0][k] + p[1][k]) / 3 : (p[0][k] + p[1][k]) / 2;
-        p[3][k] = four ? (p[0][k] + 2 * p[1][k]) / 3 : 0;
-    }
-    uint32_t key[16];
+    const float lim[3] = {31.0f, 63.0f, 31.0f};
+    for (int s = 0; s < 2; s++)
+        for (int k = 0; k < 3; k++) e[s][k] = (int)fminf(fmaxf(rintf(y[3 * s + k] * lim[k]), 0.0f), lim[k]);
+}
+
+// Brightest and darkest texels (first extreme), kept by value so that the
+// texels are only ever indexed statically.
+__device__ inline void box_start(const int (*px)[3], int (*e)[3])
+{
+    int bl = -1, dl = 1 << 30, bc[3] = {0, 0, 0}, dc[3] = {0, 0, 0};
 #pragma unroll
     for (int i = 0; i < 16; i++) {
-        uint32_t best = 0xFFFFFFFFu;
-        for (int s = 0; s < 4; s++) {
-            const int dr = px[i][0] - p[s][0], dg = px[i][1] - p[s][1], db = px[i][2] - p[s][2];
-            best = min(best, (uint32_t)(8 * dr * dr + 25 * dg * dg + db * db));
+        const int l = 2 * px[i][0] + 4 * px[i][1] + px[i][2];
+        if (l > bl) {
+            bl = l;
+            for (int k = 0; k < 3; k++) bc[k] = px[i][k];
         }
-        key[i] = best;
+        if (l < dl) {
+            dl = l;
+            for (int k = 0; k < 3; k++) dc[k] = px[i][k];
+        }
     }
-    // Batcher's odd-even merge sort network for 16 elements, descending
-#pragma unroll
-    for (int pp = 1; pp < 16; pp <<= 1)
-#pragma unroll
-        for (int k = pp; k >= 1; k >>= 1)
-#pragma unroll
-            for (int j = k % pp; j + k < 16; j += 2 * k)
-#pragma unroll
-                for (int i = 0; i < k; i++)
-                    if (i + j + k < 16 && (i + j) / (2 * pp) == (i + j + k) / (2 * pp)) {
-                        const int a = i + j, b = i + j + k;
-                        if (key[a] < key[b]) {
-                            const uint32_t tk = key[a];
-                            key[a] = key[b];
-                            key[b] = tk;
-                            for (int c = 0; c < 3; c++) {
-                                const int tv = px[a][c];
-                                px[a][c] = px[b][c];
-                                px[b][c] = tv;
-                            }
-                            const uint64_t na = (*perm >> (4 * a)) & 15u, nb = (*perm >> (4 * b)) & 15u;
-                            *perm ^= ((na ^ nb) << (4 * a)) | ((na ^ nb) << (4 * b));
-                        }
-                    }
+    const float lim[3] = {31.0f, 63.0f, 31.0f};
+    for (int k = 0; k < 3; k++) {
+        e[0][k] = (int)rintf((float)bc[k] * lim[k] / 255.0f);
+        e[1][k] = (int)rintf((float)dc[k] * lim[k] / 255.0f);
+    }
 }
 
 // Start points, each refined, the lowest final error kept (earlier start on
 // ties): bit 0 of `starts` = the network's proposal y (8 floats per block,
 // components scaled to [0, 1]); bit 1 = the block's brightest and darkest
 // texels (luma 2r + 4g + b, first extreme); bit 2 = the principal axis.
-// Bit 3 adds the least-squares refit after each descent; bit 4 polishes the
-// kept result on the both-ends lattice.
+// Bit 3 adds the least-squares refit after each descent; with bit 4 (the
+// both-ends lattice, polish_kernel) the steps carry kSwapped when the second
+// endpoint packs higher.
 // out per block (16 bytes): u32 c0 | c1 << 16, u32 selectors, u32 error,
 // u32 single steps taken (max_iters per start = stopped early)
+constexpr uint32_t kSwapped = 1u << 31;
+
 __global__ void __launch_bounds__(256) refine_kernel(const uint8_t* __restrict__ rgba, uint32_t n,
                                                      const float* __restrict__ y, uint32_t max_iters, uint32_t starts,
                                                      uint32_t* __restrict__ out)
@@ -957,7 +898,6 @@ __global__ void __launch_bounds__(256) refine_kernel(const uint8_t* __restrict__
 #pragma unroll
     for (int i = 0; i < 16; i++)
         for (int k = 0; k < 3; k++) px[i][k] = rgba[(size_t)b * 64 + 4 * i + k];
-    const int lim[3] = {31, 63, 31};
     const bool refit = (starts & 8u) != 0;
     uint32_t best = 0xFFFFFFFFu, steps = 0;
     int keep[2][3] = {{0, 0, 0}, {0, 0, 0}};
@@ -971,74 +911,476 @@ __global__ void __launch_bounds__(256) refine_kernel(const uint8_t* __restrict__
                 for (int k = 0; k < 3; k++) keep[s][k] = e[s][k];
         }
     };
+    int e[2][3];
     if (starts & 1u) {
-        const float* yy = y + (size_t)b * 8;
-        int e[2][3];
-        for (int s = 0; s < 2; s++)
-            for (int k = 0; k < 3; k++)
-                e[s][k] = (int)fminf(fmaxf(rintf(yy[3 * s + k] * (float)lim[k]), 0.0f), (float)lim[k]);
+        net_start(y + (size_t)b * 8, e);
         consider(e);
     }
     if (starts & 2u) {
-        // brightest and darkest texels (first extreme), kept by value so that
-        // the texels are only ever indexed statically
-        int bl = -1, dl = 1 << 30, bc[3] = {0, 0, 0}, dc[3] = {0, 0, 0};
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int l = 2 * px[i][0] + 4 * px[i][1] + px[i][2];
-            if (l > bl) {
-                bl = l;
-                for (int k = 0; k < 3; k++) bc[k] = px[i][k];
-            }
-            if (l < dl) {
-                dl = l;
-                for (int k = 0; k < 3; k++) dc[k] = px[i][k];
-            }
-        }
-        int e[2][3];
-        for (int k = 0; k < 3; k++) {
-            e[0][k] = (int)rintf((float)bc[k] * (float)lim[k] / 255.0f);
-            e[1][k] = (int)rintf((float)dc[k] * (float)lim[k] / 255.0f);
-        }
+        box_start(px, e);
         consider(e);
     }
     if (starts & 4u) {
-        int e[2][3];
         pca_start(px, e);
         consider(e);
-    }
-    uint64_t perm = 0;   // 0: texels in their own order
-    if ((starts & 16u) && best) {
-        // The lattice scans 728 candidates whose sums stop at the current
-        // best: visit the texels in order of falling error under the kept
-        // endpoints so that losing candidates stop early.  Only the order of
-        // the integer sums changes (selectors are mapped back below), so
-        // every result is the same.
-        order_texels(px, keep, &perm);
-    }
-    if (starts & 16u) {
-        // polish the best result on the both-ends lattice, each improvement
-        // followed by the single-step descent (and refit)
-        for (int it = 0; it < 4 && best; it++) {
-            if (!box_step(px, keep, best)) break;
-            uint32_t st = 0;
-            best = refine_from(px, keep, max_iters, refit, st);
-            steps = max(steps, st);
-        }
     }
     uint32_t lo, hi, sel;
     pair_error(px, keep[0], keep[1], lo, hi);
     best = dxt1_error(px, lo, hi, &sel);
-    if (perm) {
-        uint32_t os = 0;
-#pragma unroll
-        for (int i = 0; i < 16; i++) os |= ((sel >> (2 * i)) & 3u) << (2 * ((perm >> (4 * i)) & 15u));
-        sel = os;
-    }
+    // the polish goes on from the endpoints in their own order
+    if ((starts & 16u) && pack565(keep[0]) < pack565(keep[1])) steps |= kSwapped;
     out[(size_t)b * 4 + 0] = lo | (hi << 16);
     out[(size_t)b * 4 + 1] = sel;
     out[(size_t)b * 4 + 2] = best;
     out[(size_t)b * 4 + 3] = steps;
+}
+
+// ------------------------------------------------------------------ polish
+// Best improving move among all 728 combinations of -1 / 0 / +1 on the six
+// endpoint components (refine_solution's both-ends lattice,
+// crnlib/crn_dxt1.cpp:601-643), up to four times, each followed by the
+// single-step descent (and refit); one wavefront per block.
+//
+// A candidate's palette is separable: every channel has nine (low, high)
+// moves, and a texel's distance to entry s is the sum of three per-channel
+// terms w (p^2 - 2 p c) (the texel's own w c^2 is the same for all).  The terms
+// are a product on the matrix cores, exact as in the cluster search: integers
+// of at most 8 significant bits times powers of two in bfloat16, sums below
+// 2^24 in float32.  K slots 0-7 hold red, 8-15 green, 16-23 blue, so that a
+// lane loads its 16 bytes of a candidate's row from a table of 3 x 9 moves, and
+// one v_mfma_f32_16x16x32_bf16 gives 4 candidates x 4 entries x 16 texels.
+// Red and green alone (81 moves) bound the whole error from below, with the
+// smallest blue error added; only moves whose bound is below the best are
+// scored in full.  Ties go to the lowest move number, the order of the
+// reference's loops.  Candidates with equal endpoints decode as three colours
+// and black and are scored on the side.
+// What bounds it: the vector operations around each product (minimum, sum over
+// 16 lanes).  One lane per block scanning 728 candidates took most of the
+// refinement's 7.04 ms for 262,144 blocks; both kernels together now 2.01 ms.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+struct PolishLds {
+    u32x4 row[3][9][4];      // channel, move, entry: 8 bfloat16
+    u32x4 zero;
+    uint32_t rg[84];         // error of red and green
+    uint32_t blue[12];       // error of blue
+    uint32_t list[732];      // candidates: moves of the channels (4 bits each) | number << 16
+};
+
+__device__ inline uint32_t bf2(float a, float b)
+{
+    return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xFFFF0000u);
+}
+
+__device__ inline uint32_t lane_value(uint32_t v, uint32_t l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l); }
+
+template <int Ctrl>
+__device__ inline uint32_t dpp_of(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, Ctrl, 0xF, 0xF, false);
+}
+
+// Sum over the 16 lanes of a row, on each of them.
+__device__ inline uint32_t row_sum(uint32_t v)
+{
+    v += dpp_of<0x128>(v);   // row_ror 8, 4, 2, 1
+    v += dpp_of<0x124>(v);
+    v += dpp_of<0x122>(v);
+    return v + dpp_of<0x121>(v);
+}
+
+__device__ inline uint32_t wave_min(uint32_t v)
+{
+    v = min(v, dpp_of<0x128>(v));
+    v = min(v, dpp_of<0x124>(v));
+    v = min(v, dpp_of<0x122>(v));
+    v = min(v, dpp_of<0x121>(v));
+    return min(min(lane_value(v, 0), lane_value(v, 16)), min(lane_value(v, 32), lane_value(v, 48)));
+}
+
+// The block on a wave: lane l holds texel l & 15 in `own` and texels
+// 4 (l & 3) .. + 3 in `quad` (r | g << 8 | b << 16).
+struct WaveBlock {
+    uint32_t own, quad[4];
+};
+
+struct Ends {
+    int e[2][3];
+};
+
+__device__ inline uint32_t colour_distance(uint32_t px, const int* p)
+{
+    const int dr = (int)(px & 255u) - p[0], dg = (int)((px >> 8) & 255u) - p[1], db = (int)((px >> 16) & 255u) - p[2];
+    return (uint32_t)(8 * dr * dr + 25 * dg * dg + db * db);
+}
+
+// dxt1_error's palette of the unordered pair (a, b).
+__device__ inline void pair_palette(const int* a, const int* b, int (*p)[3])
+{
+    const uint32_t ca = pack565(a), cb = pack565(b);
+    const bool four = ca != cb;
+    expand565(max(ca, cb), p[0]);
+    expand565(min(ca, cb), p[1]);
+    for (int k = 0; k < 3; k++) {
+        p[2][k] = four ? (2 * p[0][k] + p[1][k]) / 3 : (p[0][k] + p[1][k]) / 2;
+        p[3][k] = four ? (p[0][k] + 2 * p[1][k]) / 3 : 0;
+    }
+}
+
+// Error of each quad's pair (the same on its four lanes).
+__device__ inline uint32_t quad_error(const WaveBlock& B, const int* a, const int* b)
+{
+    int p[4][3];
+    pair_palette(a, b, p);
+    uint32_t err = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        err += min(min(colour_distance(B.quad[j], p[0]), colour_distance(B.quad[j], p[1])),
+                   min(colour_distance(B.quad[j], p[2]), colour_distance(B.quad[j], p[3])));
+    err += dpp_of<0xB1>(err);   // quad_perm 1 0 3 2
+    return err + dpp_of<0x4E>(err);   // quad_perm 2 3 0 1
+}
+
+// Selector of the lane's own texel under pair (a, b).
+__device__ inline uint32_t own_selector(const WaveBlock& B, const int* a, const int* b)
+{
+    int p[4][3];
+    pair_palette(a, b, p);
+    uint32_t best = 0xFFFFFFFFu, s = 0;
+    for (uint32_t t = 0; t < 4; t++) {
+        const uint32_t e = colour_distance(B.own, p[t]);
+        if (e < best) {
+            best = e;
+            s = t;
+        }
+    }
+    return s;
+}
+
+// descend() on a wave: the twelve steps of an iteration on a quad each.
+__device__ inline bool wave_descend(const WaveBlock& B, Ends& E, uint32_t& best, uint32_t max_iters, uint32_t& steps)
+{
+    const uint32_t c = (threadIdx.x & 63u) >> 2;
+    for (;;) {
+        if (steps >= max_iters) return false;
+        int f[2][3];
+        bool ok = c < 12;
+        for (uint32_t s = 0; s < 2; s++)
+            for (uint32_t k = 0; k < 3; k++) {
+                f[s][k] = E.e[s][k] + (c >> 1 == 3 * s + k ? ((c & 1u) ? 1 : -1) : 0);
+                ok &= f[s][k] >= 0 && f[s][k] <= (k == 1 ? 63 : 31);
+            }
+        const uint32_t er = quad_error(B, f[0], f[1]);   // out of range: not taken
+        const uint32_t m = wave_min(ok && er < best ? er << 4 | c : 0xFFFFFFFFu);
+        if (m == 0xFFFFFFFFu) return true;
+        const uint32_t t = m & 15u;
+        for (uint32_t s = 0; s < 2; s++)
+            for (uint32_t k = 0; k < 3; k++) E.e[s][k] += t >> 1 == 3 * s + k ? ((t & 1u) ? 1 : -1) : 0;
+        best = m >> 4;
+        steps++;
+    }
+}
+
+// lsq_endpoints() on a wave (four-colour pairs: a != b).
+__device__ inline bool wave_lsq(const WaveBlock& B, const Ends& E, Ends& F)
+{
+    const uint32_t sel = own_selector(B, E.e[0], E.e[1]);
+    const uint32_t u = sel == 0 ? 0u : sel == 1 ? 3u : sel == 2 ? 1u : 2u, v = 3u - u;
+    const float a11 = (float)(int)lane_value(row_sum(v * v), 0), a12 = (float)(int)lane_value(row_sum(u * v), 0),
+                a22 = (float)(int)lane_value(row_sum(u * u), 0);
+    const float det = a11 * a22 - a12 * a12;
+    if (!(det > 0.0f)) return false;
+    const float lim[3] = {31.0f, 63.0f, 31.0f};
+    for (int k = 0; k < 3; k++) {
+        const uint32_t x = (B.own >> (8 * k)) & 255u;
+        const float b1 = (float)(int)lane_value(row_sum(v * x), 0), b2 = (float)(int)lane_value(row_sum(u * x), 0);
+        const float A = 3.0f * (a22 * b1 - a12 * b2) / det;
+        const float C = 3.0f * (a11 * b2 - a12 * b1) / det;
+        F.e[0][k] = (int)fminf(fmaxf(rintf(A * lim[k] / 255.0f), 0.0f), lim[k]);
+        F.e[1][k] = (int)fminf(fmaxf(rintf(C * lim[k] / 255.0f), 0.0f), lim[k]);
+    }
+    return true;
+}
+
+// refine_from() on a wave.
+__device__ inline uint32_t wave_refine(const WaveBlock& B, Ends& E, uint32_t max_iters, bool refit, uint32_t& steps)
+{
+    uint32_t best = lane_value(quad_error(B, E.e[0], E.e[1]), 0), used = 0;
+    for (int round = 0;; round++) {
+        if (!wave_descend(B, E, best, max_iters, used) || !refit || round == 3) break;
+        if (pack565(E.e[0]) == pack565(E.e[1])) break;
+        Ends F;
+        if (!wave_lsq(B, E, F)) break;
+        const uint32_t ef = lane_value(quad_error(B, F.e[0], F.e[1]), 0);
+        if (ef >= best) break;
+        best = ef;
+        E = F;
+    }
+    steps = max(steps, used);
+    return best;
+}
+
+// Sums over the texels of the smallest entry distances (without the texels'
+// own w c^2) of the product of a row operand with the texels: lane group g's
+// candidate on its 16 lanes.
+__device__ inline int product_error(const u32x4& a, const u32x4& texels)
+{
+    typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    const f32x4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, texels),
+                                                            zero, 0, 0, 0);
+    return (int)row_sum((uint32_t)(int)fminf(fminf(d[0], d[1]), fminf(d[2], d[3])));
+}
+
+// One lattice step from E: true (E and best updated) if some move improves.
+__device__ inline bool wave_box_step(PolishLds& L, const WaveBlock& B, const u32x4& texels, int own_rg, int own_b,
+                                     Ends& E, uint32_t& best)
+{
+    const uint32_t lane = threadIdx.x & 63u, group = lane >> 4;
+    // the table: one move and entry of a channel per lane and turn
+    for (uint32_t i = lane; i < 3 * 9 * 4; i += 64) {
+        const uint32_t ch = i / 36, mv = i / 4 % 9, entry = i & 3u;
+        const int e0 = (ch == 0 ? E.e[0][0] : ch == 1 ? E.e[0][1] : E.e[0][2]) + (int)(mv % 3) - 1;
+        const int e1 = (ch == 0 ? E.e[1][0] : ch == 1 ? E.e[1][1] : E.e[1][2]) + (int)(mv / 3) - 1;
+        const int c0 = min(max(e0, 0), ch == 1 ? 63 : 31), c1 = min(max(e1, 0), ch == 1 ? 63 : 31);
+        const int p0 = ch == 1 ? (c0 << 2) | (c0 >> 4) : (c0 << 3) | (c0 >> 2);
+        const int p1 = ch == 1 ? (c1 << 2) | (c1 >> 4) : (c1 << 3) | (c1 >> 2);
+        const int p = entry == 0 ? p0 : entry == 1 ? p1 : entry == 2 ? (2 * p0 + p1) / 3 : (p0 + 2 * p1) / 3;
+        const uint32_t K = (ch == 0 ? 8u : ch == 1 ? 25u : 1u) * (uint32_t)(p * p);
+        const float f = (float)p, k2 = (float)(K & 0xFF0000u), k1 = (float)(K & 0xFF00u), k0 = (float)(K & 0xFFu);
+        u32x4 v;
+        if (ch == 1) v = u32x4{bf2(-32.0f * f, -16.0f * f), bf2(-2.0f * f, k2), bf2(k1, k0), 0u};
+        else v = u32x4{bf2(ch == 0 ? -16.0f * f : -2.0f * f, k2), bf2(k1, k0), 0u, 0u};
+        L.row[ch][mv][entry] = v;
+    }
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t cand = (lane & 15u) >> 2, entry = lane & 3u;   // of the lane's operand row
+    // blue alone, then red and green
+    for (uint32_t i = 0; i < 12; i += 4) {
+        const int e = product_error(group == 2 ? L.row[2][min(i + cand, 8u)][entry] : L.zero, texels) + own_b;
+        if ((lane & 15u) == 0) L.blue[i + group] = (uint32_t)e;
+    }
+    for (uint32_t i = 0; i < 84; i += 4) {
+        const uint32_t c = min(i + cand, 80u);
+        const int e = product_error(group == 0 ? L.row[0][c % 9][entry] : group == 1 ? L.row[1][c / 9][entry] : L.zero,
+                                    texels) + own_rg;
+        if ((lane & 15u) == 0) L.rg[i + group] = (uint32_t)e;
+    }
+    __builtin_amdgcn_wave_barrier();
+    // which moves keep a channel in range: bits 0-8 per channel
+    uint32_t in[3];
+    for (uint32_t k = 0; k < 3; k++) {
+        const int lim = k == 1 ? 63 : 31;
+        const uint32_t a = (E.e[0][k] > 0 ? 1u : 0u) | 2u | (E.e[0][k] < lim ? 4u : 0u);
+        in[k] = (E.e[1][k] > 0 ? a : 0u) | (a << 3) | (E.e[1][k] < lim ? a << 6 : 0u);
+    }
+    const uint32_t blue = lane < 9 && (in[2] >> lane & 1u) ? L.blue[min(lane, 8u)] : 0xFFFFFFFFu;
+    const uint32_t least_blue = wave_min(blue);
+    // moves that make a channel's two values equal
+    uint32_t eq[3];
+    for (uint32_t k = 0; k < 3; k++) {
+        eq[k] = 0;
+        for (uint32_t mv = 0; mv < 9; mv++)
+            eq[k] |= E.e[0][k] + (int)(mv % 3) == E.e[1][k] + (int)(mv / 3) ? 1u << mv : 0u;
+    }
+    // candidates: the red and green moves below the best, each with the nine blue ones
+    uint32_t count = 0;
+    for (uint32_t i0 = 0; i0 < 81; i0 += 64) {
+        const uint32_t i = min(i0 + lane, 80u), r = i % 9, g = i / 9;
+        uint64_t keep = __ballot(i0 + lane < 81 && (in[0] >> r & 1u) && (in[1] >> g & 1u) && L.rg[i] + least_blue < best);
+        while (keep) {
+            const uint32_t c = i0 + (uint32_t)__builtin_ctzll(keep);
+            keep &= keep - 1;
+            const uint32_t r9 = c % 9, g9 = c / 9, b9 = min(lane, 8u);
+            const uint32_t number = r9 % 3 + 3 * (g9 % 3) + 9 * (b9 % 3) + 27 * (r9 / 3) + 81 * (g9 / 3) + 243 * (b9 / 3);
+            const bool same = (eq[0] >> r9 & 1u) && (eq[1] >> g9 & 1u) && (eq[2] >> b9 & 1u);
+            const bool ok = lane < 9 && (in[2] >> b9 & 1u) && !same && number != 364 && L.rg[c] + blue < best;
+            const uint64_t mask = __ballot(ok);
+            if (ok) L.list[count + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = r9 | g9 << 4 | b9 << 8 | number << 16;
+            count += (uint32_t)__popcll(mask);
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    uint32_t least = best, which = 0xFFFFFFFFu;
+    for (uint32_t i = 0; i < count; i += 4) {
+        const uint32_t c = L.list[min(i + cand, count - 1)], mine = L.list[min(i + group, count - 1)];
+        const u32x4 a = group < 3 ? L.row[group][(c >> (4 * group)) & 15u][entry] : L.zero;
+        const uint32_t e = (uint32_t)(product_error(a, texels) + own_rg + own_b), number = mine >> 16;
+        if (e < least || (e == least && which != 0xFFFFFFFFu && number < which)) {
+            least = e;
+            which = number;
+        }
+    }
+    if (eq[0] && eq[1] && eq[2]) {
+        // equal endpoints: one colour and black; a lane per (low end's moves),
+        // the high end's follow
+        const uint32_t d[3] = {lane % 3, lane / 3 % 3, lane / 9 % 3};
+        bool ok = lane < 27;
+        int c[3];
+        uint32_t number = 0, scale = 1;
+        for (uint32_t k = 0; k < 3; k++) {
+            c[k] = E.e[0][k] + (int)d[k] - 1;
+            const int h = c[k] - E.e[1][k] + 1;
+            ok &= h >= 0 && h <= 2 && c[k] >= 0 && c[k] <= (k == 1 ? 63 : 31);
+            number += scale * (d[k] + 27u * (uint32_t)max(h, 0));
+            scale *= 3;
+        }
+        int p[3];
+        expand565(pack565(c) & 0xFFFFu, p);
+        const int black[3] = {0, 0, 0};
+        uint32_t e = 0;
+        for (uint32_t t = 0; t < 16; t++) {
+            const uint32_t px = lane_value(B.own, t);
+            e += min(colour_distance(px, p), colour_distance(px, black));
+        }
+        if (ok && number != 364 && (e < least || (e == least && which != 0xFFFFFFFFu && number < which))) {
+            least = e;
+            which = number;
+        }
+    }
+    // the wave's smallest error, the lowest number on ties
+    const uint32_t me = wave_min(which == 0xFFFFFFFFu ? 0xFFFFFFFFu : least);
+    if (me == 0xFFFFFFFFu) return false;
+    const uint32_t m = wave_min(which != 0xFFFFFFFFu && least == me ? which : 0xFFFFFFFFu);
+    uint32_t r = m;
+    for (int s = 0; s < 2; s++)
+        for (int k = 0; k < 3; k++) {
+            E.e[s][k] += (int)(r % 3) - 1;
+            r /= 3;
+        }
+    best = me;
+    return true;
+}
+
+__device__ inline WaveBlock wave_block(const uint8_t* px)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    WaveBlock B;
+    __builtin_memcpy(&B.own, px + 4 * (lane & 15u), 4);   // any alignment
+    for (uint32_t j = 0; j < 4; j++) B.quad[j] = (uint32_t)__shfl((int)B.own, (int)(4 * (lane & 3u) + j));
+    return B;
+}
+
+// Up to four lattice steps from E; true if any improved.
+__device__ inline bool wave_polish(PolishLds& L, const WaveBlock& B, Ends& E, uint32_t& best, uint32_t max_iters,
+                                   bool refit, uint32_t& steps)
+{
+    const uint32_t group = (threadIdx.x & 63u) >> 4;
+    const uint32_t r = B.own & 255u, g = (B.own >> 8) & 255u, b = (B.own >> 16) & 255u;
+    const int own_rg = (int)lane_value(row_sum(8 * r * r + 25 * g * g), 0);
+    const int own_b = (int)lane_value(row_sum(b * b), 0);
+    u32x4 texels = {0u, 0u, 0u, 0u};
+    if (group == 0) texels = u32x4{bf2((float)r, 1.0f), bf2(1.0f, 1.0f), 0u, 0u};
+    if (group == 1) texels = u32x4{bf2((float)g, (float)g), bf2((float)g, 1.0f), bf2(1.0f, 1.0f), 0u};
+    if (group == 2) texels = u32x4{bf2((float)b, 1.0f), bf2(1.0f, 1.0f), 0u, 0u};
+    bool moved = false;
+    for (int it = 0; it < 4 && best; it++) {
+        if (!wave_box_step(L, B, texels, own_rg, own_b, E, best)) break;
+        moved = true;
+        best = wave_refine(B, E, max_iters, refit, steps);
+    }
+    return moved;
+}
+
+// The output record of a block's endpoints.
+__device__ inline u32x4 wave_record(const WaveBlock& B, const Ends& E, uint32_t best, uint32_t steps)
+{
+    const uint32_t ca = pack565(E.e[0]), cb = pack565(E.e[1]);
+    uint32_t sel = own_selector(B, E.e[0], E.e[1]) << (2 * (threadIdx.x & 15u));
+    sel |= dpp_of<0x128>(sel);
+    sel |= dpp_of<0x124>(sel);
+    sel |= dpp_of<0x122>(sel);
+    sel |= dpp_of<0x121>(sel);
+    return u32x4{max(ca, cb) | min(ca, cb) << 16, sel, best, steps};
+}
+
+constexpr uint32_t kPolishWaves = 4;
+
+__global__ void __launch_bounds__(64 * kPolishWaves) polish_kernel(const uint8_t* __restrict__ rgba, uint32_t n,
+                                                                   uint32_t per, uint32_t max_iters, uint32_t refit,
+                                                                   uint32_t* __restrict__ out)
+{
+    __shared__ PolishLds lds[kPolishWaves];
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63u;
+    PolishLds& L = lds[wave];
+    const uint64_t first = ((uint64_t)blockIdx.x * kPolishWaves + wave) * per;
+    if (first >= n) return;
+    const uint32_t m = (uint32_t)min((uint64_t)per, n - first);
+    if (lane == 0) L.zero = u32x4{0u, 0u, 0u, 0u};
+    __builtin_amdgcn_wave_barrier();
+    // one block's state per lane; blocks of error zero have nothing to gain
+    uint32_t* rec = out + 4 * (first + min(lane, m - 1));
+    u32x4 mine;
+    __builtin_memcpy(&mine, rec, 16);   // (no more than the output's own alignment is known)
+    const uint64_t blocks = m == 64 ? ~0ull : (1ull << m) - 1ull;
+    uint64_t todo = __ballot(mine.z != 0) & blocks;
+    const uint32_t swapped = mine.w & kSwapped;
+    mine.w &= ~kSwapped;
+    while (todo) {
+        const uint32_t k = (uint32_t)__builtin_ctzll(todo);
+        todo &= todo - 1;
+        const WaveBlock B = wave_block(rgba + (first + k) * 64);
+        const uint32_t lohi = lane_value(mine.x, k), sw = lane_value(swapped, k);
+        uint32_t best = lane_value(mine.z, k), steps = lane_value(mine.w, k);
+        const uint32_t cc[2] = {sw ? lohi >> 16 : lohi & 0xFFFFu, sw ? lohi & 0xFFFFu : lohi >> 16};
+        Ends E;
+        for (int s = 0; s < 2; s++) {
+            E.e[s][0] = (int)(cc[s] >> 11);
+            E.e[s][1] = (int)((cc[s] >> 5) & 63u);
+            E.e[s][2] = (int)(cc[s] & 31u);
+        }
+        if (wave_polish(L, B, E, best, max_iters, refit != 0, steps)) {
+            const u32x4 q = wave_record(B, E, best, steps);
+            if (lane == k) mine = q;
+        }
+    }
+    if (lane < m) __builtin_memcpy(rec, &mine, 16);
+}
+
+// The whole refinement, one wavefront per block: for calls whose blocks would
+// leave refine_kernel's one lane per block a wave or less per SIMD, where its
+// time is that of the slowest block (4,096 blocks 3.68 ms with the polish in it,
+// here 74 us; 65,536 blocks 0.85 ms with the polish apart, here 0.74).
+// Beyond kWaveBlocks blocks refine_kernel's lanes do more work per operation
+// (both kernels 1.13 ms for 131,044 blocks; here 1.42).
+constexpr uint32_t kWaveBlocks = 65536;
+
+__global__ void __launch_bounds__(64 * kPolishWaves) refine_wave_kernel(const uint8_t* __restrict__ rgba, uint32_t n,
+                                                                        const float* __restrict__ y,
+                                                                        uint32_t max_iters, uint32_t starts,
+                                                                        uint32_t* __restrict__ out)
+{
+    __shared__ PolishLds lds[kPolishWaves];
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63u;
+    PolishLds& L = lds[wave];
+    const uint32_t b = blockIdx.x * kPolishWaves + wave;
+    if (b >= n) return;
+    if (lane == 0) L.zero = u32x4{0u, 0u, 0u, 0u};
+    __builtin_amdgcn_wave_barrier();
+    const WaveBlock B = wave_block(rgba + (size_t)b * 64);
+    int px[16][3];
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+        for (int k = 0; k < 3; k++) px[i][k] = (int)((lane_value(B.own, (uint32_t)i) >> (8 * k)) & 255u);
+    const bool refit = (starts & 8u) != 0;
+    uint32_t best = 0xFFFFFFFFu, steps = 0;
+    Ends keep = {{{0, 0, 0}, {0, 0, 0}}};
+    for (uint32_t t = 0; t < 3; t++) {
+        if (!(starts >> t & 1u)) continue;
+        Ends E;
+        if (t == 0) net_start(y + (size_t)b * 8, E.e);
+        else if (t == 1) box_start(px, E.e);
+        else pca_start(px, E.e);
+        const uint32_t eb = wave_refine(B, E, max_iters, refit, steps);
+        if (eb < best) {
+            best = eb;
+            keep = E;
+        }
+    }
+    if (starts & 16u) wave_polish(L, B, keep, best, max_iters, refit, steps);
+    const u32x4 q = wave_record(B, keep, best, steps);
+    if (lane == 0) __builtin_memcpy(out + 4 * (size_t)b, &q, 16);
 }
 
 // Error of given DXT1 blocks (c0 | c1 << 16 per block) under the same decode.
@@ -1184,9 +1526,24 @@ int crn2_dxt1_refine_device(const void* rgba, uint32_t n, const float* y, uint32
 {
     if (!n) return CRN2_OK;
     if (!rgba || !out || !(starts & 7u) || (starts & ~31u) || ((starts & 1u) && !y)) return CRN2_EINVAL;
+    if (n <= kWaveBlocks) {
+        hipLaunchKernelGGL(refine_wave_kernel, dim3(grid1(n, kPolishWaves)), dim3(64 * kPolishWaves), 0,
+                           static_cast<hipStream_t>(stream), static_cast<const uint8_t*>(rgba), n, y, max_iters, starts,
+                           out);
+        return hipGetLastError() == hipSuccess ? CRN2_OK : CRN2_EHIP;
+    }
     hipLaunchKernelGGL(refine_kernel, dim3(grid1(n, 256)), dim3(256), 0, static_cast<hipStream_t>(stream),
                        static_cast<const uint8_t*>(rgba), n, y, max_iters, starts, out);
-    return hipGetLastError() == hipSuccess ? CRN2_OK : CRN2_EHIP;
+    if (hipGetLastError() != hipSuccess) return CRN2_EHIP;
+    if (starts & 16u) {
+        // blocks per wave: one until the waves fill the GPU many times over
+        const uint32_t per = std::min<uint32_t>(64, std::max<uint32_t>(1, n >> 16));
+        hipLaunchKernelGGL(polish_kernel, dim3(grid1(n, per * kPolishWaves)), dim3(64 * kPolishWaves), 0,
+                           static_cast<hipStream_t>(stream), static_cast<const uint8_t*>(rgba), n, per, max_iters,
+                           (starts >> 3) & 1u, out);
+        if (hipGetLastError() != hipSuccess) return CRN2_EHIP;
+    }
+    return CRN2_OK;
 }
 
 int crn2_dxt1_block_error_device(const void* rgba, uint32_t n, const uint32_t* endpoints, uint32_t stride_u32,

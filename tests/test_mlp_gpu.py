@@ -163,6 +163,93 @@ def train_small(seed=0, steps=300, n=262144, batch=8192):
     return tr
 
 
+def _pair_errors(px, e):
+    """Errors of many endpoint pairs e (k x 2 x 3, 5:6:5 components) on one
+    block's texels (16 x 3), the pair in either order."""
+    w = np.array([1 << 11, 1 << 5, 1])
+    c = (e * w).sum(-1)
+    hi = np.where((c[:, 0] >= c[:, 1])[:, None], e[:, 0], e[:, 1])
+    lo = np.where((c[:, 0] >= c[:, 1])[:, None], e[:, 1], e[:, 0])
+
+    def ex(v):
+        return np.stack([v[:, 0] << 3 | v[:, 0] >> 2, v[:, 1] << 2 | v[:, 1] >> 4, v[:, 2] << 3 | v[:, 2] >> 2], 1)
+    p, q = ex(hi), ex(lo)
+    four = (c[:, 0] != c[:, 1])[:, None]
+    pal = np.stack([p, q, np.where(four, (2 * p + q) // 3, (p + q) // 2), np.where(four, (p + 2 * q) // 3, 0)], 1)
+    d = ((px[None, None] - pal[:, :, None]) ** 2 * W).sum(-1)
+    return d.min(1).sum(1)
+
+
+def _best_move(px, e, moves, err):
+    f = e[None] + moves
+    ok = ((f >= 0) & (f <= np.array([31, 63, 31]))).all((1, 2))
+    er = np.where(ok, _pair_errors(px, np.clip(f, 0, 63)), 1 << 40)
+    k = int(er.argmin())
+    return (k, int(er[k])) if er[k] < err else (None, err)
+
+
+@pytest.mark.parametrize("kind", ["texture", "near flat", "dark", "noise"])
+def test_polish_takes_the_first_best_lattice_move(gpu, kind):
+    """The polish against its own definition in numpy: from the unpolished
+    result (in both orders of the endpoints), up to four times the first of the
+    smallest errors among the 728 moves, then single steps while they help;
+    near-flat blocks have candidates with equal endpoints."""
+    print("polish", kind, flush=True)
+    rng = np.random.default_rng(len(kind))
+    n = 130
+    if kind == "texture":
+        blocks = dxt1.image_blocks(texture.synth(64, 64, 5, texture.RGB))[:n].copy()
+    else:
+        spread, top = {"near flat": (6, 250), "dark": (12, 13), "noise": (256, 1)}[kind]
+        blocks = (rng.integers(0, top, (n, 1, 4)) + rng.integers(0, spread, (n, 16, 4))).clip(0, 255).astype(np.uint8)
+    t = dev(blocks)
+    start = learned.refine(t, None, 16, learned.START_BOX).cpu().numpy().view(np.uint32)
+    got = learned.refine(t, None, 16, learned.START_BOX | learned.POLISH).cpu().numpy().view(np.uint32)
+    ms = np.arange(729)
+    box = np.stack([(ms // 3 ** k) % 3 - 1 for k in range(6)], 1).reshape(-1, 2, 3)[np.arange(729) != 364]
+    one = np.array([[s, k, d] for s in range(2) for k in range(3) for d in (-1, 1)])
+    steps = np.zeros((12, 2, 3), int)
+    steps[np.arange(12), one[:, 0], one[:, 1]] = one[:, 2]
+    moved = 0
+    for i in range(n):
+        px = blocks[i, :, :3].astype(np.int64)
+        best = int(start[i, 2])
+        results = []
+        for order in (0, 1):          # the start's endpoints in either order: only ties tell them apart
+            c = [int(start[i, 0] & 0xFFFF), int(start[i, 0] >> 16)]
+            e = np.array([[v >> 11, v >> 5 & 63, v & 31] for v in (c[::-1] if order else c)])
+            err = best
+            for _ in range(4):
+                if not err:
+                    break
+                k, err = _best_move(px, e, box, err)
+                if k is None:
+                    break
+                e = e + box[k]
+                for _ in range(16):
+                    k, err = _best_move(px, e, steps, err)
+                    if k is None:
+                        break
+                    e = e + steps[k]
+            words = (e * np.array([1 << 11, 1 << 5, 1])).sum(-1)
+            results.append((int(words.max()) | int(words.min()) << 16, err))
+        assert (int(got[i, 0]), int(got[i, 2])) in results, (i, results)
+        moved += int(got[i, 2]) < best
+    assert kind == "dark" or moved > 5
+
+
+@pytest.mark.parametrize("starts", [learned.START_NET, learned.ENCODE_STARTS])
+def test_refinement_paths_agree(gpu, starts):
+    """A call of 65,537 blocks (one lane per block, the polish on its own) gives
+    what calls of fewer (one wavefront per block) give for the same blocks."""
+    print("refinement paths", starts, flush=True)
+    t = dev(dxt1.image_blocks(texture.synth(1032, 1024, 12, texture.RGB))[:65537])
+    y = learned.infer(dev(np.load("crunch2_amd/data/dxt1_proposal.npy")), t)
+    whole = learned.refine(t, y, learned.ENCODE_ITERS, starts)
+    parts = [learned.refine(t[a:b], y[a:b], learned.ENCODE_ITERS, starts) for a, b in ((0, 65536), (65536, 65537))]
+    assert torch.equal(whole, torch.cat(parts))
+
+
 def test_training_gains_over_untrained_and_box_start(gpu):
     """Ablation on held-out blocks.  The method without the network refines
     from the block's brightest/darkest texels; with it, the refinement also
