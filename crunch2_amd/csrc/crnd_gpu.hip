@@ -9,14 +9,15 @@
 // it can be and runs everything else in parallel:
 //   1. crnd_tables_kernel (all bit positions in parallel): for every bit
 //      position, the bits eight even-row block pairs (with their odd-row
-//      flags), one pair, or two odd-row blocks (four variants by the two
-//      blocks' reference flags) would take if they started there; built in
-//      LDS per tile from per-position code lengths.
-//   2. crnd_walk_kernel (two waves per level): one wave follows the stream
-//      through the composed tables, one lookup per eight pairs or two odd-row
-//      blocks, in scalar registers; the other streams the tables into an LDS
-//      ring ahead of it.  Records the start bit of every group of 8 pairs /
-//      8 odd-row blocks.
+//      flags) and two or four odd-row blocks (a variant for each of the
+//      blocks' reference flags) would take if they started there, and where
+//      rows end in less than that, one pair (and one block); built in LDS per
+//      tile from per-position code lengths.
+//   2. crnd_walk_kernel (a workgroup per level): one wave follows the stream
+//      through the composed tables, one lookup per eight pairs or two or four
+//      odd-row blocks; the others stream the tables into an LDS ring ahead of
+//      it.  Records the start bit of every group of 8 pairs / 8 odd-row
+//      blocks.
 //   3. crnd_sym_kernel (one thread per group; even rows, then odd rows):
 //      endpoint deltas, selectors and reference codes from the start bits.
 //   4. crnd_index_{chunk,carry}_kernel: running endpoint indices by pointer
@@ -63,6 +64,15 @@ static bool kind_uses(int kind, uint32_t m)
     if (m == M_EP0 || m == M_SEL0) return kind == 0 || kind == 1;
     return kind != 0;
 }
+
+// The model's longest code length.
+static uint32_t longest_code(const HostModel& m)
+{
+    uint32_t longest = 0;
+    for (uint8_t size : m.sizes) longest = std::max<uint32_t>(longest, size);
+    return longest;
+}
+
 // ------------------------------------------------------------ shared types
 // Per-texture constants of a launch.
 struct TexInfo {
@@ -87,13 +97,14 @@ struct LevelJob {
     uint32_t src_size;
     uint32_t tex;                // index into the TexInfo array
     uint32_t gw, gh, faces;      // even-padded block grid
-    uint32_t tlen;               // table entries: multiple of kTabPerWG, >= 8 * src_size + 1024
+    uint32_t tlen;               // table entries: multiple of TabShape::kPerWG, >= 8 * src_size + 1024
     uint32_t wg_trans;           // first workgroup of the job in crnd_tables_kernel
     uint32_t wg_sym;             // first workgroup of the job in crnd_sym_kernel<false> (even rows)
     uint32_t wg_odd;             // first workgroup of the job in crnd_sym_kernel<true> (odd rows)
-    uint32_t* O2;                // two odd-row blocks, one entry per bit position
+    uint32_t* O2;                // two odd-row blocks, one entry per bit position (or O4)
+    uint4* O4;                   // four odd-row blocks, one entry per bit position
     uint32_t* E8;                // eight even-row pairs, one entry per bit position
-    uint16_t* X;                 // one even-row pair, one entry per bit position
+    void* X;                     // one even-row pair (u16), with O4 also one odd-row block (u32), one entry per bit position
     uint32_t* posE;              // start bit of each group of kGroup pairs of the even rows
     uint32_t* posO;              // start bit of each group of kGroup blocks of the odd rows
     uint8_t* gvals;              // faces * gh/2 * gw/2 reference group symbols
@@ -101,8 +112,9 @@ struct LevelJob {
     uint32_t crows;              // block rows per index chunk
     uint32_t nchunks;            // index chunks of the level
     uint32_t wg_idx;             // first workgroup of the job in crnd_index_chunk_kernel
-    uint32_t need_x;             // 1: the even rows end in a partial group of pairs, the only place the
-                                 // walk reads X; 0: X is neither written nor read
+    uint32_t need_x;             // 1: the rows end in a partial group of pairs (and perhaps of blocks), the
+                                 // only place the walk reads X; 0: X is neither written nor read
+    uint32_t wide;               // 1: four odd-row blocks can take 256 bits (every code 16 bits long)
     uint64_t blk_first;          // first block of the job in crnd_index_final_kernel
     uint64_t* ent;               // faces * gh * gw: (parent, index residues) after the chunk pass
     uint64_t* bnd;               // nchunks * gw: the chunks' last rows (resolved in place by crnd_index_carry_kernel)
@@ -183,14 +195,19 @@ __device__ inline uint32_t decode_top(const LdsTables& t, gcuint16* sorted, uint
 // run at least 1024 entries past it):
 //   O2[q], byte f (f = 0..3): bits taken by two odd-row blocks starting at q
 //          when bit 0 of f says the first carries endpoint deltas and bit 1
-//          the second
-//   E8[q], bits 0-10: bits taken by eight even-row pairs starting at q
-//          bits 11-26: the odd-row flags of those pairs, two per pair (the
+//          the second; or
+//   O4[q], byte 4 a + b: the same for four blocks, a for the first two and b
+//          for the others (modulo 256: four blocks with deltas may take 256)
+//   E8[q], bits 2-12: bits taken by eight even-row pairs starting at q
+//          bit 15: byte 15 of O4[q] stands for 256
+//          bits 16-31: the odd-row flags of those pairs, two per pair (the
 //          block below the pair's first / second block has reference code 0)
-//   X[q],  bits 0-7: bits taken by one even-row pair; bits 8-9: its two flags
-//          (only for a level whose even rows end in a partial group of
-//          pairs, LevelJob::need_x: the walk reads X nowhere else)
-// One workgroup computes kTabPerWG consecutive positions in three LDS passes:
+//   X[q],  bits 0-7: bits taken by one even-row pair; bits 8-9: its two flags;
+//          beside O4, bits 10-15: bits taken by an odd-row block without
+//          deltas; bits 16-23: by one with (only for a level whose even rows
+//          end in a partial group of pairs, LevelJob::need_x: the walk reads X
+//          nowhere else)
+// One workgroup computes TabShape::kPerWG consecutive positions in three LDS passes:
 //   1. per position: the reference group symbol and its code length, and the
 //      code lengths of one block's endpoint deltas and of its selectors
 //      (CW = GL | F << 8 | DL << 16 | SL << 24; two channels: both codes;
@@ -202,28 +219,37 @@ __device__ inline uint32_t decode_top(const LdsTables& t, gcuint16* sorted, uint
 //      takes at most 144 bits, a block 64 (32 without deltas), a code 16);
 //   3. the composed entries above from T (eight pairs reach 1008 entries on).
 // Each pass runs past the tile by what the next one reads.  Every thread
-// keeps several positions' lookup chains in flight at once (kTabU1..3, the
+// keeps several positions' lookup chains in flight at once (kU1..3, the
 // positions tid + 512 k), so that the dependent LDS reads of one position
 // overlap those of the others; the pass-1 code tables and the T array share
-// LDS (the tables are dead once pass 1 ends), 50,816 B per workgroup: three
-// workgroups per CU, two beside a stream walker's 40 KiB ring.  The tile of
-// 6,144 positions keeps the halo that passes 1 and 2 recompute to 19 % and
-// 17 % (measured on the 4096^2 pair: 4,096 positions 6.04 ms per plan of 32
-// copies, 5,120 6.02, 6,144 5.75, 8,192 6.03 at four waves per SIMD).
-constexpr uint32_t kTabPerWG = 6144;
-constexpr uint32_t kTabT = kTabPerWG + 1024;
-constexpr uint32_t kTabCW = kTabT + 160;
-constexpr uint32_t kTabWords = kTabCW / 32 + 3;
+// LDS (the tables are dead once pass 1 ends): three workgroups per CU, with
+// O4 (whose two-block entries take T's space once T is dead) at 46 KiB each,
+// with O2 at 50 KiB, two beside a stream walker's 40 KiB ring.
+// O2's tile of 6,144 positions keeps the halo that passes 1 and 2 recompute to
+// 19 % and 17 % (measured on the 4096^2 pair: 4,096 positions 6.04 ms per plan
+// of 32 copies, 5,120 6.02, 6,144 5.75, 8,192 6.03 at four waves per SIMD);
+// O4's of 5,120 to 23 % and 20 % (6,144 would leave two workgroups per CU).
+//
+// O4 costs 20 B per bit to write where O2 costs 8 (the same plan: 8.25 against
+// 5.46 ms), and takes a third off the longest level's walk: build_plan.
 constexpr uint32_t kTabThreads = 512;
-constexpr uint32_t kTabU1 = 8;   // pass 1: two rounds of 8 slots cover kTabCW (7,328 = 14.3 x 512)
-constexpr uint32_t kTabU2 = 7;   // pass 2: two rounds of 7 cover kTabT
-constexpr uint32_t kTabU3 = 6;   // pass 3b: two rounds of 6 cover kTabPerWG
-constexpr uint32_t kTabE2 = kTabPerWG + 6 * 144;   // two-pair entries an eight-pair chain reads
-constexpr uint32_t kTabU3a = 7;  // pass 3a: two rounds of 7 cover kTabE2
-static_assert(2 * kTabU1 * kTabThreads >= kTabCW && 2 * kTabU2 * kTabThreads == kTabT &&
-                  2 * kTabU3 * kTabThreads == kTabPerWG && 2 * kTabU3a * kTabThreads >= kTabE2 &&
-                  kTabE2 + 144 <= kTabT && kTabE2 * 2 <= kTabCW * 4,
-              "table pass rounds");
+template <bool FOUR>
+struct TabShape {
+    static constexpr uint32_t kPerWG = FOUR ? 5120 : 6144;
+    static constexpr uint32_t kT = kPerWG + 1024;
+    static constexpr uint32_t kCW = kT + 160;
+    static constexpr uint32_t kWords = kCW / 32 + 3;
+    static constexpr uint32_t kU1 = FOUR ? 7 : 8;        // pass 1: two rounds of kU1 slots cover kCW
+    static constexpr uint32_t kU2 = kT / (2 * kTabThreads);
+    static constexpr uint32_t kU3 = kPerWG / (2 * kTabThreads);
+    static constexpr uint32_t kE2 = kPerWG + 6 * 144;    // two-pair entries an eight-pair chain reads
+    static constexpr uint32_t kU3a = kU2;                // pass 3a: two rounds cover kE2
+    static constexpr uint32_t kO2 = kPerWG + 128;        // two-block entries a four-block entry reads
+    static_assert(2 * kU1 * kTabThreads >= kCW && 2 * kU2 * kTabThreads == kT && 2 * kU3 * kTabThreads == kPerWG &&
+                      2 * kU3a * kTabThreads >= kE2 && kE2 + 144 <= kT && kE2 * 2 <= kCW * 4 && kO2 <= kE2 &&
+                      kO2 + 64 <= kT,
+                  "table pass rounds");
+};
 
 __device__ inline uint32_t be_bytes_word(const uint8_t* src, uint32_t size, uint32_t b)
 {
@@ -275,28 +301,34 @@ typedef __attribute__((address_space(1))) uint16_t guint16;
 
 constexpr uint32_t kTabRefSyms = 1024;   // reference-model symbols (low bytes) staged in LDS; the rest read from memory
 
+template <bool FOUR>
 struct TabCodes {
     uint32_t cw1[kLutSize];   // TexInfo::cw1
     uint16_t cw2[kLutSize];   // TexInfo::cw2
     CodeLimits lim[M_COUNT];
     uint8_t ref_sym[kTabRefSyms];
-    uint32_t words[kTabWords];
+    uint32_t words[TabShape<FOUR>::kWords];
 };
 
+template <bool FOUR>
 union TabShared {
-    TabCodes c;          // pass 1
+    TabCodes<FOUR> c;         // pass 1
     struct {
-        uint16_t lo[kTabT];   // passes 2 and 3: pair bits | odd flags << 8 | bits of an odd block without deltas << 10
-        uint8_t hi[kTabT];    //                 bits of an odd block with deltas
+        uint16_t lo[TabShape<FOUR>::kT];   // passes 2 and 3: pair bits | odd flags << 8 | bits of an odd block without deltas << 10
+        uint8_t hi[TabShape<FOUR>::kT];    //                 bits of an odd block with deltas
     } t;
+    uint32_t o2[FOUR ? TabShape<FOUR>::kO2 : 1];   // pass 3b: two odd blocks, byte f = bits by their two flags
 };
 
 // tab_job[wg] = the level job of tables workgroup wg.
+template <bool FOUR>
 __global__ void __launch_bounds__(kTabThreads) crnd_tables_kernel(const LevelJob* __restrict__ jobs,
                                                                   const uint32_t* __restrict__ tab_job,
                                                                   const TexInfo* __restrict__ texs)
 {
-    __shared__ TabShared s_u;
+    using Shape = TabShape<FOUR>;
+    constexpr uint32_t kTabPerWG = Shape::kPerWG, kTabCW = Shape::kCW, kTabWords = Shape::kWords, kTabE2 = Shape::kE2;
+    __shared__ TabShared<FOUR> s_u;
     __shared__ uint32_t s_cw[kTabCW];
     const uint32_t tid = threadIdx.x;
     const LevelJob& j = jobs[tab_job[blockIdx.x]];
@@ -339,7 +371,7 @@ __global__ void __launch_bounds__(kTabThreads) crnd_tables_kernel(const LevelJob
         const CodeLimits& S1 = s_u.c.lim[M_SEL1];
         const bool two = two_channels(kind);
         const uint16_t* ref_sorted = tx.sorted + M_REF * kMaxSyms;
-        constexpr uint32_t U = kTabU1;
+        constexpr uint32_t U = Shape::kU1;
 #pragma unroll 1
         for (uint32_t i0 = 0; i0 < 2 * U; i0 += U) {
             uint32_t r[U], w32[U], c[U];   // w32: the 32 bits from r on; top = w32 >> 16
@@ -404,7 +436,7 @@ __global__ void __launch_bounds__(kTabThreads) crnd_tables_kernel(const LevelJob
     {
         uint16_t* T = s_u.t.lo;
         uint8_t* T8 = s_u.t.hi;
-        constexpr uint32_t U = kTabU2;
+        constexpr uint32_t U = Shape::kU2;
 #pragma unroll 1
         for (uint32_t i0 = 0; i0 < 2 * U; i0 += U) {
             uint32_t r[U], c[U], e[U], x[U], od[U];
@@ -446,89 +478,150 @@ __global__ void __launch_bounds__(kTabThreads) crnd_tables_kernel(const LevelJob
     __syncthreads();
 
     // 3. composed entries (stores at 32-bit offsets from the tile's base).
-    // 3a: O2 and X, and two-pair entries E2 = len (9 bits) | four odd flags
-    // << 9 for every position an E8 chain reaches (kTabPerWG + 6 x 144), into
-    // the CW array's space (dead after pass 2); 3b: E8 from four E2 lookups
-    // (three dependent LDS reads instead of seven).
+    // 3a: X, the two-block entries O2 (for O4 kept in registers until T is dead)
+    // and two-pair entries E2 = len (9 bits) | four odd flags << 9 for every
+    // position an E8 chain reaches (kTabPerWG + 6 x 144), into the CW array's
+    // space (dead after pass 2); 3b: E8 from four E2 lookups (three dependent
+    // LDS reads instead of seven), and O4 from five O2 lookups.
     {
         const uint16_t* T = s_u.t.lo;
         const uint8_t* T8 = s_u.t.hi;
         uint16_t* E2 = reinterpret_cast<uint16_t*>(s_cw);
         typedef __attribute__((address_space(1))) uint8_t guint8;
+        typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(1))) u4 gu4;
         guint8* O2 = (guint8*)(j.O2 + P0);
+        guint8* O4 = (guint8*)(j.O4 + P0);
         guint8* E8 = (guint8*)(j.E8 + P0);
-        guint8* X = (guint8*)(j.X + P0);
+        guint8* X = (guint8*)j.X + (FOUR ? 4 : 2) * (size_t)P0;
         const bool need_x = j.need_x != 0;
-        {
-            constexpr uint32_t U = kTabU3a;
-#pragma unroll 1
-            for (uint32_t i0 = 0; i0 < 2 * U; i0 += U) {
-                uint32_t r[U], t0[U], o1[U], ta[U], tb[U], ta8[U], tb8[U], tp[U];
+        uint32_t o2[2][Shape::kU3a];
+        auto pass_3a = [&](uint32_t h) {
+            constexpr uint32_t U = Shape::kU3a;
+            uint32_t r[U], t0[U], o1[U], ta[U], tb[U], ta8[U], tb8[U], tp[U];
 #pragma unroll
-                for (uint32_t u = 0; u < U; u++) {
-                    r[u] = min(tid + (i0 + u) * kTabThreads, kTabE2 - 1);
-                    t0[u] = T[r[u]];
-                    o1[u] = T8[r[u]];
-                }
+            for (uint32_t u = 0; u < U; u++) {
+                r[u] = min(tid + (h * U + u) * kTabThreads, kTabE2 - 1);
+                t0[u] = T[r[u]];
+                o1[u] = T8[r[u]];
+            }
 #pragma unroll
-                for (uint32_t u = 0; u < U; u++) {
-                    ta[u] = T[r[u] + (t0[u] >> 10)];
-                    ta8[u] = T8[r[u] + (t0[u] >> 10)];
-                    tb[u] = T[r[u] + o1[u]];
-                    tb8[u] = T8[r[u] + o1[u]];
-                    tp[u] = T[r[u] + (t0[u] & 0xFFu)];
-                }
+            for (uint32_t u = 0; u < U; u++) {
+                ta[u] = T[r[u] + (t0[u] >> 10)];
+                ta8[u] = T8[r[u] + (t0[u] >> 10)];
+                tb[u] = T[r[u] + o1[u]];
+                tb8[u] = T8[r[u] + o1[u]];
+                tp[u] = T[r[u] + (t0[u] & 0xFFu)];
+            }
 #pragma unroll
-                for (uint32_t u = 0; u < U; u++) {
-                    const uint32_t q = tid + (i0 + u) * kTabThreads;
-                    if (q < kTabE2)
-                        E2[r[u]] = (uint16_t)(((t0[u] & 0xFFu) + (tp[u] & 0xFFu)) | ((t0[u] & 0x300u) << 1) |
-                                              ((tp[u] & 0x300u) << 3));
-                    if (q < kTabPerWG) {
-                        const uint32_t o0 = t0[u] >> 10;
-                        *(guint32*)(O2 + 4 * r[u]) = (o0 + (ta[u] >> 10)) | ((o1[u] + (tb[u] >> 10)) << 8) |
-                                                     ((o0 + ta8[u]) << 16) | ((o1[u] + tb8[u]) << 24);
-                        if (need_x) *(guint16*)(X + 2 * r[u]) = (uint16_t)(t0[u] & 0x3FFu);
-                    }
+            for (uint32_t u = 0; u < U; u++) {
+                const uint32_t q = tid + (h * U + u) * kTabThreads;
+                if (q < kTabE2)
+                    E2[r[u]] = (uint16_t)(((t0[u] & 0xFFu) + (tp[u] & 0xFFu)) | ((t0[u] & 0x300u) << 1) |
+                                          ((tp[u] & 0x300u) << 3));
+                const uint32_t o0 = t0[u] >> 10;
+                const uint32_t two = (o0 + (ta[u] >> 10)) | ((o1[u] + (tb[u] >> 10)) << 8) | ((o0 + ta8[u]) << 16) |
+                                     ((o1[u] + tb8[u]) << 24);
+                if (FOUR) o2[h][u] = two;
+                if (q < kTabPerWG) {
+                    if (!FOUR) *(guint32*)(O2 + 4 * r[u]) = two;
+                    if (need_x && FOUR) *(guint32*)(X + 4 * r[u]) = t0[u] | (o1[u] << 16);
+                    if (need_x && !FOUR) *(guint16*)(X + 2 * r[u]) = (uint16_t)(t0[u] & 0x3FFu);
                 }
             }
+        };
+        if constexpr (FOUR) {
+            pass_3a(0);
+            pass_3a(1);
+        } else {
+#pragma unroll 1
+            for (uint32_t h = 0; h < 2; h++) pass_3a(h);
         }
         __syncthreads();
+        if constexpr (FOUR) {
+#pragma unroll
+            for (uint32_t h = 0; h < 2; h++)
+#pragma unroll
+                for (uint32_t u = 0; u < Shape::kU3a; u++) {
+                    const uint32_t q = tid + (h * Shape::kU3a + u) * kTabThreads;
+                    if (q < Shape::kO2) s_u.o2[q] = o2[h][u];
+                }
+            __syncthreads();
+        }
         {
-            constexpr uint32_t U = kTabU3;
+            constexpr uint32_t U = Shape::kU3;
 #pragma unroll 1
             for (uint32_t i0 = 0; i0 < 2 * U; i0 += U) {
-                uint32_t r[U], p[U], fl[U];
+                uint32_t r[U], p[U], fl[U], big[U];
 #pragma unroll
                 for (uint32_t u = 0; u < U; u++) {
                     r[u] = tid + (i0 + u) * kTabThreads;
                     p[u] = r[u];
                     fl[u] = 0;
+                    big[u] = 0;
                 }
-                // odd flags gathered at bit 9 + 4 i, shifted down once
+                if constexpr (FOUR) {
+                    uint32_t e[U];
+                    u4 o[U];
+#pragma unroll
+                    for (uint32_t u = 0; u < U; u++) e[u] = s_u.o2[r[u]];
+                    // a first half's length, then the second half's four from there
+                    // (added to all four bytes: only the top one can reach 256)
+#pragma unroll
+                    for (uint32_t a = 0; a < 4; a++) {
+#pragma unroll
+                        for (uint32_t u = 0; u < U; u++) {
+                            const uint32_t len = (e[u] >> (8 * a)) & 0xFFu, n = s_u.o2[r[u] + len];
+                            o[u][a] = n + len * 0x01010101u;
+                            if (a == 3) big[u] = (n >> 24) + len >= 256u ? 1u << 15 : 0u;
+                        }
+                    }
+#pragma unroll
+                    for (uint32_t u = 0; u < U; u++) *(gu4*)(O4 + 16 * r[u]) = o[u];
+                }
+                // odd flags gathered at bit 9 + 4 i, shifted up once
 #pragma unroll
                 for (uint32_t i = 0; i < 4; i++) {
 #pragma unroll
                     for (uint32_t u = 0; u < U; u++) {
-                        const uint32_t e = E2[p[u]];
-                        fl[u] |= (e & 0x1E00u) << (4 * i);
-                        p[u] += e & 0x1FFu;
+                        const uint32_t e2 = E2[p[u]];
+                        fl[u] |= (e2 & 0x1E00u) << (4 * i);
+                        p[u] += e2 & 0x1FFu;
                     }
                 }
 #pragma unroll
                 for (uint32_t u = 0; u < U; u++)
-                    *(guint32*)(E8 + 4 * r[u]) = (p[u] - r[u]) | ((fl[u] >> 9) << 11);
+                    *(guint32*)(E8 + 4 * r[u]) = ((p[u] - r[u]) << 2) | (fl[u] << 7) | big[u];
             }
         }
     }
 }
 
-// --------------------------------------------------------- stage 2: walker
-// One workgroup of two waves per level stream.  Wave 0 follows the stream
-// from bit 0 and records the start bit of every group of kGroup pairs (even
-// rows) or kGroup blocks (odd rows); wave 1 streams the composed tables from
-// memory into an LDS ring ahead of it, so the walking wave never waits on
-// memory and holds no staging registers.
+// --------------------------------------------------------- stage 2: walkers
+// One workgroup per level stream.  Its wave 0 follows the stream from bit 0 and
+// records the start bit of every group of kGroup pairs (even rows) or kGroup
+// blocks (odd rows); the others stream the composed tables from memory into an
+// LDS ring ahead of it, so the walking wave never waits on memory and holds no
+// staging registers.  Two of them: over O2 tables (namespace two) and over O4
+// tables (namespace four); build_plan chooses.
+constexpr uint32_t kPlanJobsSmallRing = 512;          // plans of more levels take the small rings
+constexpr uint32_t kGroup = 8;                        // pairs / blocks per recorded start bit
+constexpr uint32_t kMaxEGroups = 64;                  // even-row groups per row (one per lane): grids up to 1024 blocks wide
+// Either side waits for the other at most this many sleeps (about a quarter
+// of a second; a real wait lasts microseconds).  Past it a producer stops
+// and the walker finishes its loops on whatever the ring holds and reports
+// CRN2_EHIP, so a fault in the hand-off cannot hang the device.
+constexpr uint32_t kSpinCap = 1u << 21;
+
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) const u32x4 gconst_u32x4;
+
+__device__ inline uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ inline uint32_t lds_get(const uint32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+__device__ inline void lds_put(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+
+namespace two {
+// Two waves, one of them a producer.
 //
 // A lone wave issues about one instruction every four cycles, so the walking
 // loop is kept short and wave-uniform (scalar registers):
@@ -546,15 +639,7 @@ constexpr uint32_t kSeg = 1024;                       // table entries per ring 
 // at a time: 8 (80 KiB of LDS, one walker per CU, the deepest prefetch: the
 // shortest walk of a lone level) or 4 (40 KiB, three walkers per CU: more
 // levels at once when a plan holds hundreds of them).
-constexpr uint32_t kPlanJobsSmallRing = 512;
-constexpr uint32_t kGroup = 8;                        // pairs / blocks per recorded start bit
-constexpr uint32_t kMaxEGroups = 64;                  // even-row groups per row (one per lane): grids up to 1024 blocks wide
 constexpr uint32_t kNeed = 1152 + 128 + 64;           // a group's longest move + the two windows
-// Either wave waits for the other at most this many sleeps (about a quarter
-// of a second; a real wait lasts microseconds).  Past it the producer stops
-// and the walker finishes its loops on whatever the ring holds and reports
-// CRN2_EHIP, so a fault in the hand-off cannot hang the device.
-constexpr uint32_t kSpinCap = 1u << 21;
 
 template <uint32_t RS>
 struct WalkLds {
@@ -567,18 +652,11 @@ struct WalkLds {
     uint32_t done;        // the walker has finished
 };
 
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(1))) const u32x4 gconst_u32x4;
-
 // Two-bit flag pairs x = f0 | f1 << 2 | f2 << 4 | f3 << 6 -> bytes f_k * 8.
 __device__ inline uint32_t spread_flags(uint32_t x)
 {
     return ((x & 3u) | ((x & 0xCu) << 6) | ((x & 0x30u) << 12) | ((x & 0xC0u) << 18)) << 3;
 }
-
-__device__ inline uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
-__device__ inline uint32_t lds_get(const uint32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
-__device__ inline void lds_put(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 
 // Per lane and segment: 4 + 4 vectors of O2 / E8 entries, 2 of X entries.
 template <uint32_t RS>
@@ -597,7 +675,7 @@ __device__ inline void producer_load(const LevelJob& j, uint32_t tsegs, uint32_t
         const size_t at = (size_t)min(s0 + b, tsegs - 1) * kSeg;
         const gconst_u32x4* po = (const gconst_u32x4*)(j.O2 + at);
         const gconst_u32x4* pe = (const gconst_u32x4*)(j.E8 + at);
-        const gconst_u32x4* px = (const gconst_u32x4*)(j.X + at);
+        const gconst_u32x4* px = (const gconst_u32x4*)((const uint16_t*)j.X + at);
 #pragma unroll
         for (uint32_t i = 0; i < 4; i++) {
             r.v[b][i] = po[64 * i + lane];
@@ -731,8 +809,8 @@ __device__ void walk_stream(const LevelJob& j, WalkLds<RS>& sh, uint32_t lane, i
                 const bool mine = lane == g;
                 vE = mine ? p : vE;
                 const uint32_t e = uniform(sh.e8[p & kMask]);
-                p += e & 0x7FFu;
-                vflags = mine ? (e >> 11) : vflags;
+                p += (e >> 2) & 0x7FFu;
+                vflags = mine ? (e >> 16) : vflags;
             }
             if (u0 < npairs) {
                 if (__builtin_expect(p >= chk, 0)) ring_check(p);
@@ -837,6 +915,313 @@ __global__ void __launch_bounds__(128) crnd_walk_kernel(const LevelJob* __restri
     if (threadIdx.x >= 64) walk_producer(j, sh, threadIdx.x - 64);
     else walk_stream(j, sh, threadIdx.x, texs[j.tex].status);
 }
+}  // namespace two
+
+namespace four {
+// Nine waves, eight of them producers, a segment each in turn.
+//
+// What bounds it: one dependent LDS read after another.
+//   even row: one E8 entry per group of eight pairs, one X entry per pair in a
+//             row's last, partial group;
+//   odd row:  one O4 byte per four blocks, chosen by the blocks' flags, one X
+//             entry per block of a last pair.
+// The position stays in a vector register (the same on all lanes): an entry
+// that goes through v_readlane or v_readfirstlane into scalar registers costs
+// 96 to 126 cycles a step, a vector chain of read, add, mask and address 100
+// to 110.  So the addresses take one vector instruction behind the read (two
+// where a row group starts): the part without the step's bits is added while
+// the read is in flight, and the large ring repeats its first segments behind
+// its last one, so that kSteps steps need no wrap.
+// One test of the ring's fill covers kSteps odd-row steps.  It compares with
+// the fill that the test before it read, reports the walk's segment and reads
+// the fill again, all behind a step's read, with no branch taken unless the
+// ring has run dry; that step's read then goes out again.  Tests that asked
+// eight producers and waited for the answer took 700 cycles each.
+// Level 0 of a 2048^2 DXT5 texture (v_readlane from entries of two blocks, one
+// E8 entry per readfirstlane): 4.26 ms, now 2.87 ms, about
+// 140 cycles a step.
+//
+// The walker reports the segment it has reached; the producers never overwrite
+// that segment or a later unread one.
+constexpr uint32_t kSeg = 512;                        // table entries per ring segment
+// The ring holds RS segments (template parameter), and each producer one more
+// in registers: 8 (96 KiB of LDS, one walker per CU: the shortest walk of a lone
+// level) or 4 (48 KiB, three walkers per CU: more levels at once when a plan
+// holds hundreds of them).
+constexpr uint32_t kProducers = 8;
+constexpr uint32_t kWalkThreads = 64 * (1 + kProducers);
+
+template <uint32_t RS>
+struct WalkLds {
+    static constexpr uint32_t kRingPos = kSeg * RS;
+    static constexpr uint32_t kMirror = RS >= 8 ? 2 : 0;   // segments of O4 repeated behind the ring's end
+    static_assert(4 * kRingPos <= 1u << 15, "an even-row address takes an E8 entry's low 15 bits");
+    u32x4 o4[kRingPos + kMirror * kSeg];
+    uint32_t e8[kRingPos];
+    uint32_t x[kRingPos];
+    uint32_t filled;              // segments below this one are (or have been) in the ring
+    uint32_t consumed;            // the walker reads no segment below this one any more; kWalkDone: it has finished
+};
+constexpr uint32_t kWalkDone = 0xFFFFFFFFu;
+
+// A segment in a producer's registers: vectors of O4, E8 and X.
+constexpr uint32_t kSegO4 = kSeg / 64, kSegE8 = kSeg / 256, kSegX = kSeg / 256;
+struct SegVecs {
+    u32x4 o4[kSegO4], e8[kSegE8], x[kSegX];
+};
+
+// Segments past the table reload its last one: every entry from the end of
+// the stream on is the same, and the table's last segment lies past the end.
+__device__ inline void producer_load(const LevelJob& j, uint32_t tsegs, uint32_t s, uint32_t lane, SegVecs& r)
+{
+    const size_t at = (size_t)min(s, tsegs - 1) * kSeg;
+    const gconst_u32x4* po = (const gconst_u32x4*)(j.O4 + at);
+    const gconst_u32x4* pe = (const gconst_u32x4*)(j.E8 + at);
+    const gconst_u32x4* px = (const gconst_u32x4*)((const uint32_t*)j.X + at);
+#pragma unroll
+    for (uint32_t i = 0; i < kSegO4; i++) r.o4[i] = po[64 * i + lane];
+#pragma unroll
+    for (uint32_t i = 0; i < kSegE8; i++) r.e8[i] = pe[64 * i + lane];
+    if (j.need_x) {
+#pragma unroll
+        for (uint32_t i = 0; i < kSegX; i++) r.x[i] = px[64 * i + lane];
+    }
+}
+
+template <uint32_t RS>
+__device__ inline void producer_store(WalkLds<RS>& sh, uint32_t s, uint32_t lane, const SegVecs& r, bool need_x)
+{
+    const uint32_t at = (s % RS) * kSeg;
+    u32x4* pe = reinterpret_cast<u32x4*>(sh.e8 + at);
+    u32x4* px = reinterpret_cast<u32x4*>(sh.x + at);
+#pragma unroll
+    for (uint32_t i = 0; i < kSegO4; i++) sh.o4[at + 64 * i + lane] = r.o4[i];
+    if (s % RS < WalkLds<RS>::kMirror) {
+#pragma unroll
+        for (uint32_t i = 0; i < kSegO4; i++) sh.o4[WalkLds<RS>::kRingPos + at + 64 * i + lane] = r.o4[i];
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kSegE8; i++) pe[64 * i + lane] = r.e8[i];
+    if (need_x) {
+#pragma unroll
+        for (uint32_t i = 0; i < kSegX; i++) px[64 * i + lane] = r.x[i];
+    }
+}
+
+// Producer w: segments w, w + kProducers, ...; loads the next one while it
+// waits for ring space; stops when the walker says it is done.
+template <uint32_t RS>
+__device__ void walk_producer(const LevelJob& j, WalkLds<RS>& sh, uint32_t w, uint32_t lane)
+{
+    const uint32_t tsegs = j.tlen / kSeg;
+    const bool need_x = j.need_x != 0;
+    SegVecs r;
+    uint32_t s = w;
+    for (;;) {
+        producer_load(j, tsegs, s, lane, r);
+#pragma unroll 1
+        for (uint32_t spin = 0;; spin++) {
+            const uint32_t used = uniform(lds_get(&sh.consumed));
+            if (used == kWalkDone) return;
+            if (s < used + RS) break;   // the walk has passed, so the ring has held, the space's last segment
+            if (spin >= kSpinCap) return;
+            // the producers whose turn is further off leave the LDS to the walker
+            if (s > used + RS) __builtin_amdgcn_s_sleep(8);
+            else __builtin_amdgcn_s_sleep(2);
+        }
+        producer_store(sh, s, lane, r, need_x);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        // in order: the segments before this one are in the ring too
+#pragma unroll 1
+        for (uint32_t spin = 0; uniform(lds_get(&sh.filled)) != s; spin++) {
+            if (spin >= kSpinCap || uniform(lds_get(&sh.consumed)) == kWalkDone) return;
+            __builtin_amdgcn_s_sleep(1);
+        }
+        lds_put(&sh.filled, s + 1);
+        s += kProducers;
+    }
+}
+
+// Wave 0.  p: the current bit, the same on all lanes.
+// WIDE: four blocks can take 256 bits (LevelJob::wide).
+template <uint32_t RS, bool WIDE>
+__device__ void walk_stream(const LevelJob& j, WalkLds<RS>& sh, uint32_t lane, int32_t* status)
+{
+    constexpr uint32_t kMask = kSeg * RS - 1;
+    // Odd-row steps per test, at most 256 bits each, and the segments past
+    // the first read's that they reach.
+    constexpr uint32_t kSteps = RS >= 8 ? 4 : 2, kReach = kSteps * 256 / kSeg;
+    constexpr bool kMirrored = WalkLds<RS>::kMirror != 0;
+    static_assert((kSteps - 1) * 256 < kReach * kSeg && kReach + 2 <= RS, "ring");
+    static_assert(!kMirrored || WalkLds<RS>::kMirror >= kReach, "ring");
+    // volatile: a read stays where it is written, ahead of the test on it
+    typedef __attribute__((address_space(3))) const volatile uint8_t lds_u8;
+    typedef __attribute__((address_space(3))) const volatile uint32_t lds_u32;
+    typedef __attribute__((address_space(3))) volatile uint32_t lds_w32;
+    lds_u8* o4 = (lds_u8*)sh.o4;
+    lds_u8* e8 = (lds_u8*)sh.e8;
+    lds_u32* xt = (lds_u32*)sh.x;
+    lds_u32* filled = (lds_u32*)&sh.filled;
+    lds_w32* consumed = (lds_w32*)&sh.consumed;
+    bool stuck = false;
+    uint32_t lim = 0;                 // sh.filled as the last test read it
+    // Whether the next kSteps odd-row reads (or one even-row read) from bit
+    // `pos` on may find entries that are not in the ring: then it waits until
+    // they are.
+    auto dry = [&](uint32_t pos) -> bool {
+        const uint32_t seg = pos / kSeg;
+        if (__builtin_expect(!__any(seg + kReach >= lim), 1) || stuck) return false;
+        *consumed = seg;
+#pragma unroll 1
+        for (uint32_t spin = 0; !stuck; spin++) {
+            lim = *filled;
+            if (!__any(seg + kReach >= lim)) break;
+            stuck = spin >= kSpinCap;
+            __builtin_amdgcn_s_sleep(1);
+        }
+        return true;
+    };
+    // Reports the walk's segment, and the fill for the next test.
+    auto refresh = [&](uint32_t pos) {
+        *consumed = pos / kSeg;
+        lim = *filled;
+    };
+
+    const uint32_t gw = j.gw, gh = j.gh, faces = j.faces;
+    const uint32_t npairs = gw >> 1;
+    const uint32_t gE = (npairs + kGroup - 1) / kGroup;   // even-row groups per row (at most 64)
+    const uint32_t gO = (gw + kGroup - 1) / kGroup;       // odd-row groups per row (at most 128)
+    guint32* posE = (guint32*)j.posE;
+    guint32* posO = (guint32*)j.posO;
+    __builtin_amdgcn_s_setprio(3);    // the chain's few instructions go ahead of the producers' on a shared SIMD
+    uint32_t p, omask, emask;         // (the compiler must not see that they are uniform)
+    __asm__ volatile("v_mov_b32 %0, 0" : "=v"(p));
+    __asm__ volatile("v_mov_b32 %0, %1" : "=v"(omask) : "s"(16 * kMask));
+    __asm__ volatile("v_mov_b32 %0, %1" : "=v"(emask) : "s"(4 * kMask));
+    const uint32_t rowpairs = faces * (gh >> 1);
+    for (uint32_t rowpair = 0; rowpair < rowpairs; rowpair++) {
+        // even row: one E8 entry per full group of eight pairs; lane g keeps
+        // group g's start bit (vE) and odd-row flags (vflags)
+        uint32_t vE = 0, vflags = 0;
+        uint32_t u0 = 0, g = 0;
+        uint32_t q4 = (p << 2) & emask;   // the entry's byte address
+        for (; u0 + kGroup <= npairs; u0 += kGroup, g++) {
+            uint32_t e;
+            do e = *(lds_u32*)(e8 + q4);
+            while (dry(p));
+            refresh(p);
+            const bool mine = lane == g;
+            vE = mine ? p : vE;
+            q4 = (q4 + e) & emask;        // (the bits above the length lie outside the ring)
+            vflags = mine ? e >> 16 : vflags;
+            p += (e >> 2) & 0x7FFu;
+        }
+        if (u0 < npairs) {
+            vE = lane == g ? p : vE;
+            uint32_t fw = 0;
+            for (uint32_t k = 0; u0 + k < npairs; k++) {
+                uint32_t x;
+                do x = xt[p & kMask];
+                while (dry(p));
+                fw |= ((x >> 8) & 3u) << (2 * k);
+                p += x & 0xFFu;
+            }
+            vflags = lane == g ? fw : vflags;
+        }
+        if (lane < gE) posE[rowpair * gE + lane] = vE;
+        // odd row: one O4 byte per four blocks.  Lane h holds the flags of the
+        // 16 blocks under its group; nibble k, halves swapped, is the byte of
+        // step k's entry.
+        const uint32_t vbyte = ((vflags & 0x3333u) << 2) | ((vflags >> 2) & 0x3333u);
+        uint32_t vOa = 0, vOb = 0;        // lane h: start bits of odd groups 2h, 2h + 1
+        uint32_t q = (p << 4) & omask;    // the position's byte address in o4
+        auto advance = [&](uint32_t b, uint32_t f) {
+            // 0 in byte 15 stands for 256 if the position's E8 entry says so
+            if (WIDE && f == 15u && __any(b == 0) && (uniform(*(lds_u32*)(e8 + ((p << 2) & emask))) >> 15 & 1u)) b = 256;
+            p += b;
+            return b;
+        };
+        // A step whose entry is byte f of the position's: `at` is its address,
+        // afterwards that of the next step's entry, byte fn of its position's.
+        auto step = [&](uint32_t& at, uint32_t f, uint32_t fn, bool test, bool wrap, bool report) {
+            uint32_t b;
+            do b = o4[at];
+            while (test && dry(p));
+            if (report) refresh(p);
+            uint32_t t = q + fn;
+            __asm__ volatile("" : "+v"(t), "+v"(q));   // (computed while the read is in flight)
+            b = advance(b, f);
+            if (wrap) {
+                __asm__("v_lshl_add_u32 %0, %1, 4, %2" : "=v"(q) : "v"(b), "v"(q));
+                q &= omask;
+                at = q | fn;
+            } else {
+                // (one instruction behind the read: the compiler would share b << 4 with q)
+                __asm__("v_lshl_add_u32 %0, %1, 4, %2" : "=v"(at) : "v"(b), "v"(t));
+                q += b << 4;
+            }
+        };
+        const uint32_t n4 = gw / 4;       // steps of the row
+        uint32_t h = 0;
+        uint32_t f = (uint32_t)__builtin_amdgcn_readlane((int)vbyte, 0);
+        uint32_t at = q | (f & 15u);
+        for (; 4 * h + 4 <= n4; h++) {
+            const uint32_t fn = (uint32_t)__builtin_amdgcn_readlane((int)vbyte, (int)((h + 1) & 63u));
+            const bool mine = lane == h;
+            vOa = mine ? p : vOa;
+            step(at, f & 15u, (f >> 4) & 15u, true, !kMirrored, false);
+            step(at, (f >> 4) & 15u, (f >> 8) & 15u, false, !kMirrored, true);
+            vOb = mine ? p : vOb;
+            step(at, (f >> 8) & 15u, f >> 12, kSteps == 2, !kMirrored, false);
+            step(at, f >> 12, fn & 15u, false, true, kSteps == 2);
+            f = fn;
+        }
+        uint32_t blk = 16 * h;            // blocks left: 0..14, even
+        if (blk < gw) {
+            const bool mine = lane == h;
+            for (uint32_t k = 0; blk + 4 <= gw; k++, blk += 4) {
+                if (k == 0) vOa = mine ? p : vOa;
+                if (k == 2) vOb = mine ? p : vOb;
+                step(at, (f >> (4 * k)) & 15u, (f >> (4 * k + 4)) & 15u, true, true, false);
+            }
+            if (blk < gw) {
+                // two blocks, one X entry each; their flags are the low half of the
+                // next nibble (the high half of its swapped form)
+                const uint32_t k = (blk >> 2) & 3u, two = (f >> (4 * k + 2)) & 3u;
+                if (k == 0) vOa = mine ? p : vOa;
+                if (k == 2) vOb = mine ? p : vOb;
+                for (uint32_t i = 0; i < 2; i++) {
+                    uint32_t x;
+                    do x = xt[p & kMask];
+                    while (dry(p));
+                    p += two >> i & 1u ? (x >> 16) & 0xFFu : (x >> 10) & 0x3Fu;
+                }
+            }
+        }
+        if (2 * lane < gO) posO[rowpair * gO + 2 * lane] = vOa;
+        if (2 * lane + 1 < gO) posO[rowpair * gO + 2 * lane + 1] = vOb;
+    }
+    lds_put(&sh.consumed, kWalkDone);
+    if (stuck && lane == 0) atomicExch(status, CRN2_EHIP);
+}
+
+template <uint32_t RS>
+__global__ void __launch_bounds__(kWalkThreads) crnd_walk_kernel(const LevelJob* __restrict__ jobs,
+                                                                 const TexInfo* __restrict__ texs)
+{
+    __shared__ __align__(16) WalkLds<RS> sh;
+    const LevelJob& j = jobs[blockIdx.x];
+    if (threadIdx.x == 0) {
+        sh.filled = 0;
+        sh.consumed = 0;
+    }
+    __syncthreads();
+    const uint32_t wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    if (wave) walk_producer(j, sh, wave - 1, lane);
+    else if (uniform(j.wide)) walk_stream<RS, true>(j, sh, lane, texs[j.tex].status);
+    else walk_stream<RS, false>(j, sh, lane, texs[j.tex].status);
+}
+}  // namespace four
 
 // ------------------------------------------------------ stage 3: symbols
 // One thread per recorded group decodes, from the group's start bit, the
@@ -1420,6 +1805,7 @@ struct crn2_batch {
     WritePalettes* d_pals = nullptr;
     uint32_t* d_tab_job = nullptr;  // level job of every crnd_tables_kernel workgroup
     uint8_t* d_scratch = nullptr;   // transition tables, start bits, symbol records
+    bool four = false;              // O4 tables (build_plan)
     uint32_t njobs = 0;
     uint32_t wg_trans = 0, wg_sym = 0, wg_odd = 0, wg_idx = 0;
     uint32_t max_gw = 0;
@@ -1685,17 +2071,43 @@ struct PlanPart {
     std::vector<uint32_t> pitch;                // per level
 };
 
-static int build_plan(std::vector<PlanPart>& parts, crn2_batch** out)
+// Whether a plan takes O4 tables: they cost 1.9 us more per Mbit of stream to
+// write than O2 tables, at the whole chip's rate, and shorten the walk, which
+// lasts as long as its longest level, by 270 us per Mbit of that level (2048^2
+// DXT5 with its levels, 7.1 Mbit in all and 5.2 in level 0: walk 4.26 -> 2.87
+// ms, tables 45 -> 65 us; 64 textures of 64^2 to 1024^2: walk 1.24 -> 0.81 ms,
+// tables 122 -> 188 us; 32 pairs of 4096^2 DXT1 and DXT5, 74 times the longest
+// level: walk 17.9 -> 14.7 ms, tables 5.5 -> 8.2 ms, and four such plans on
+// four streams, where one's walk runs beside another's tables, 45.9 -> 65.2
+// ms).  Up to 32 times the longest level the tables cost a quarter of the gain.
+// The second bound keeps the tables within 5 GiB (O2: 2).
+static bool takes_o4(const std::vector<PlanPart>& parts)
+{
+    uint64_t total = 0, longest = 0;
+    for (const PlanPart& P : parts)
+        for (uint32_t l = P.first; l < P.first + P.count; l++) {
+            const Header& h = P.c->h;
+            const uint32_t next = (l + 1 < h.levels) ? h.level_ofs[l + 1] : P.c->size;
+            const uint64_t bits = 8 * (uint64_t)(P.src_override ? P.src_size : next - h.level_ofs[l]);
+            total += bits;
+            longest = std::max(longest, bits);
+        }
+    return total <= 32 * longest && total <= 1ull << 28;
+}
+
+static int build_plan_as(std::vector<PlanPart>& parts, bool four, crn2_batch** out)
 {
     *out = nullptr;
     crn2_batch* B = new (std::nothrow) crn2_batch();
     if (!B) return CRN2_ENOMEM;
+    B->four = four;
+    const uint32_t per_wg = four ? TabShape<true>::kPerWG : TabShape<false>::kPerWG;
     std::vector<LevelJob> jobs;
     std::vector<TexInfo> texs;
     std::vector<WriteJob> wj;
     std::vector<WritePalettes> pals;
     size_t scratch = 0;
-    struct Ofs { size_t O2, E8, X, E, O, G, pre, ent, bnd; };
+    struct Ofs { size_t odd, E8, X, E, O, G, pre, ent, bnd; };
     std::vector<Ofs> ofs;
     uint32_t wg_trans = 0, wg_sym = 0, wg_odd = 0, wg_idx = 0, max_gw = 0;
     uint64_t blk_total = 0;
@@ -1715,6 +2127,10 @@ static int build_plan(std::vector<PlanPart>& parts, crn2_batch** out)
         t.n_cs = c->n_cs;
         t.n_ae = c->n_ae;
         t.n_as = c->n_as;
+        uint32_t longest = 0;   // the longest block: deltas and selectors of the longest codes
+        for (uint32_t m = M_EP0; m < M_COUNT; m++)
+            if (kind_uses(c->kind, m)) longest += longest_code(c->models[m]);
+        const uint32_t wide = 4 * longest >= 256 ? 1u : 0u;
         for (uint32_t i = 0; i < P.count; i++) {
             const uint32_t l = P.first + i;
             const uint32_t bx = (level_dim(h.width, l) + 3) >> 2, by = (level_dim(h.height, l) + 3) >> 2;
@@ -1737,11 +2153,12 @@ static int build_plan(std::vector<PlanPart>& parts, crn2_batch** out)
             j.tex = (uint32_t)texs.size();
             j.gw = gw;
             j.need_x = ((gw >> 1) % kGroup) != 0 ? 1u : 0u;
+            j.wide = wide;
             j.gh = gh;
             j.faces = h.faces;
-            j.tlen = (uint32_t)align_up((size_t)j.src_size * 8 + 1024, kTabPerWG);
+            j.tlen = (uint32_t)align_up((size_t)j.src_size * 8 + 1024, per_wg);
             j.wg_trans = wg_trans;
-            wg_trans += j.tlen / kTabPerWG;
+            wg_trans += j.tlen / per_wg;
             const uint64_t rowpairs = (uint64_t)h.faces * (gh / 2);
             const uint64_t gE = rowpairs * ((gw / 2 + kGroup - 1) / kGroup), gO = rowpairs * ((gw + kGroup - 1) / kGroup);
             j.wg_sym = wg_sym;
@@ -1757,12 +2174,12 @@ static int build_plan(std::vector<PlanPart>& parts, crn2_batch** out)
             j.blk_first = blk_total;
             blk_total += (uint64_t)rows * gw;
             Ofs o;
-            o.O2 = scratch;
-            scratch = align_up(scratch + (size_t)j.tlen * 4, 256);
+            o.odd = scratch;
+            scratch = align_up(scratch + (size_t)j.tlen * (four ? 16 : 4), 256);
             o.E8 = scratch;
             scratch = align_up(scratch + (size_t)j.tlen * 4, 256);
             o.X = scratch;
-            scratch = align_up(scratch + (size_t)j.tlen * 2, 256);
+            scratch = align_up(scratch + (j.need_x ? (size_t)j.tlen * (four ? 4 : 2) : 0), 256);
             o.E = scratch;
             scratch = align_up(scratch + gE * 4, 256);
             o.O = scratch;
@@ -1808,7 +2225,7 @@ static int build_plan(std::vector<PlanPart>& parts, crn2_batch** out)
     B->ncarry = (uint32_t)carry.size();
     std::vector<uint32_t> tab_job(wg_trans);
     for (uint32_t i = 0; i < (uint32_t)jobs.size(); i++)
-        std::fill(tab_job.begin() + jobs[i].wg_trans, tab_job.begin() + jobs[i].wg_trans + jobs[i].tlen / kTabPerWG, i);
+        std::fill(tab_job.begin() + jobs[i].wg_trans, tab_job.begin() + jobs[i].wg_trans + jobs[i].tlen / per_wg, i);
     // one allocation and one upload for the tables (the scratch memory follows them)
     size_t tables = 0;
     auto part = [&](size_t bytes) {
@@ -1831,9 +2248,10 @@ static int build_plan(std::vector<PlanPart>& parts, crn2_batch** out)
     B->d_carry = reinterpret_cast<uint32_t*>(B->d_mem + o_carry);
     B->d_scratch = B->d_mem + tables;
     for (size_t i = 0; i < jobs.size(); i++) {
-        jobs[i].O2 = reinterpret_cast<uint32_t*>(B->d_scratch + ofs[i].O2);
+        if (four) jobs[i].O4 = reinterpret_cast<uint4*>(B->d_scratch + ofs[i].odd);
+        else jobs[i].O2 = reinterpret_cast<uint32_t*>(B->d_scratch + ofs[i].odd);
         jobs[i].E8 = reinterpret_cast<uint32_t*>(B->d_scratch + ofs[i].E8);
-        jobs[i].X = reinterpret_cast<uint16_t*>(B->d_scratch + ofs[i].X);
+        jobs[i].X = B->d_scratch + ofs[i].X;
         jobs[i].ent = reinterpret_cast<uint64_t*>(B->d_scratch + ofs[i].ent);
         jobs[i].bnd = reinterpret_cast<uint64_t*>(B->d_scratch + ofs[i].bnd);
         jobs[i].gvals = B->d_scratch + ofs[i].G;
@@ -1860,6 +2278,15 @@ static int build_plan(std::vector<PlanPart>& parts, crn2_batch** out)
     return CRN2_OK;
 }
 
+static int build_plan(std::vector<PlanPart>& parts, crn2_batch** out)
+{
+    if (takes_o4(parts)) {
+        const int rc = build_plan_as(parts, true, out);
+        if (rc != CRN2_ENOMEM) return rc;
+    }
+    return build_plan_as(parts, false, out);
+}
+
 // Queues the plan's launches on `stream`; with `ev`, records an event before
 // each stage and after the last.
 static int launch_plan(crn2_batch* B, hipStream_t stream, Profile::Ev* ev)
@@ -1867,14 +2294,15 @@ static int launch_plan(crn2_batch* B, hipStream_t stream, Profile::Ev* ev)
     const bool prof = ev != nullptr;
     if (prof) HIPCHK(hipEventRecord(ev->e[0], stream));
     if (B->njobs) {
-        hipLaunchKernelGGL(crnd_tables_kernel, dim3(B->wg_trans), dim3(kTabThreads), 0, stream, B->d_jobs,
-                           B->d_tab_job, B->d_texs);
+        const bool small = B->njobs >= kPlanJobsSmallRing;
+        const auto tables = B->four ? crnd_tables_kernel<true> : crnd_tables_kernel<false>;
+        hipLaunchKernelGGL(tables, dim3(B->wg_trans), dim3(kTabThreads), 0, stream, B->d_jobs, B->d_tab_job, B->d_texs);
         HIPCHK(hipGetLastError());
         if (prof) HIPCHK(hipEventRecord(ev->e[1], stream));
-        if (B->njobs >= kPlanJobsSmallRing)
-            hipLaunchKernelGGL(crnd_walk_kernel<4>, dim3(B->njobs), dim3(128), 0, stream, B->d_jobs, B->d_texs);
-        else
-            hipLaunchKernelGGL(crnd_walk_kernel<8>, dim3(B->njobs), dim3(128), 0, stream, B->d_jobs, B->d_texs);
+        const auto walk = B->four ? (small ? four::crnd_walk_kernel<4> : four::crnd_walk_kernel<8>)
+                                  : (small ? two::crnd_walk_kernel<4> : two::crnd_walk_kernel<8>);
+        hipLaunchKernelGGL(walk, dim3(B->njobs), dim3(B->four ? four::kWalkThreads : 128), 0, stream, B->d_jobs,
+                           B->d_texs);
         HIPCHK(hipGetLastError());
         if (prof) HIPCHK(hipEventRecord(ev->e[2], stream));
         hipLaunchKernelGGL(crnd_sym_kernel<false>, dim3(B->wg_sym), dim3(256), 0, stream, B->d_jobs, B->njobs,

@@ -181,6 +181,73 @@ def test_batch_plan_mixed_textures_and_graph_replay(gpu):
         assert crnd.unpack_end(c)
 
 
+def run_plan(files, copies=1):
+    """Every file `copies` times in one plan; returns each output's bytes."""
+    import torch
+    ctxs = [crnd.unpack_begin(d) for d in files for _ in range(copies)]
+    outs = [torch.zeros(crnd.levels_size(c, 0, crnd.get_texture_info(d)["levels"]), dtype=torch.uint8, device="cuda")
+            for c, d in zip(ctxs, [d for d in files for _ in range(copies)])]
+    n = len(ctxs)
+    plan = C.c_void_p()
+    assert lib().crn2_batch_create((C.c_void_p * n)(*[c.handle for c in ctxs]), n,
+                                   (C.c_void_p * n)(*[o.data_ptr() for o in outs]),
+                                   (C.c_uint64 * n)(*[o.numel() for o in outs]), C.byref(plan)) == 0
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert lib().crn2_batch_run(plan, stream) == 0
+    assert lib().crn2_batch_status(plan, stream) == 0
+    assert lib().crn2_batch_destroy(plan) == 0
+    for c in ctxs:
+        assert crnd.unpack_end(c)
+    return [o.cpu().numpy() for o in outs]
+
+
+def oracle_bytes(data):
+    ref = oracle.unpack_all(data)
+    return np.concatenate([np.concatenate([f.reshape(-1) for f in ref[l]]) for l in sorted(ref)])
+
+
+# One file alone takes the tables of four odd-row blocks, 40 copies those of two
+# (more than 32 times the longest level): rows of 2 to 34 blocks end in every
+# remainder of a 16-block group.
+@pytest.mark.parametrize("copies", [1, 40])
+@pytest.mark.parametrize("fmt", [FMT_DXT1, FMT_DXT5, FMT_DXN_XY])
+def test_row_remainders_both_tables(gpu, fmt, copies):
+    for bw in ([2, 6, 8, 14, 16, 18, 20, 30, 34] if copies == 1 else [6, 16, 34]):
+        say("rows of", bw, "blocks, format", fmt, "copies", copies)
+        data = texture.synth_crn((4 * bw, 40), 50 + bw, fmt)
+        exp = oracle_bytes(data)
+        for got in run_plan([data], copies):
+            assert np.array_equal(got, exp), (bw, fmt)
+
+
+def test_four_blocks_of_256_bits(gpu):
+    """Symbols of geometric frequencies, and groups of four odd-row blocks whose
+    every symbol occurs once among 98,304: 16-bit codes in all four models, so
+    that a group takes 256 bits, which its table entry's byte holds as 0."""
+    rng = np.random.default_rng(3)
+    gw, gh, n = 256, 384, 1024
+    def skewed(first):
+        return np.minimum(rng.geometric(0.5, gw * gh) - 1 + first, 16)
+    idx = [skewed(1), skewed(0), skewed(1), skewed(0)]   # endpoint steps and selectors, colour and alpha
+    rare = 20
+    for g in range(64):
+        at = (6 * g + 1) * gw + 4 * ((7 * g) % 64)
+        for m in idx:
+            m[at:at + 4] = rare + np.arange(4)
+        rare += 4
+    ends = [np.cumsum(m) % n for m in (idx[0], idx[2])]
+    ce = rng.integers(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32)
+    ae = rng.integers(0, 1 << 16, n, dtype=np.uint64).astype(np.uint32)
+    cs = rng.integers(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32)
+    al = rng.integers(0, 1 << 48, n, dtype=np.uint64)
+    data = texture.pack(4 * gw, 4 * gh, 1, 1, FMT_DXT5, ce, cs, ae, al, ends[0], idx[1], ends[1], idx[3])
+    exp = oracle_bytes(data)
+    say("256-bit groups, file of", len(data))
+    for copies in (1, 40):
+        for got in run_plan([data], copies):
+            assert np.array_equal(got, exp), copies
+
+
 @pytest.mark.parametrize("fmt,pal,factor", crn_cases.SHRUNK)
 def test_out_of_range_palette_indices_fail_like_oracle(gpu, fmt, pal, factor):
     """A palette cut short makes some levels reach past it: each level must
