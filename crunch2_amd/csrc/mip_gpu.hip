@@ -11,22 +11,35 @@
 // (-ffp-contract=off), so every sum rounds exactly as the reference's.  A
 // list is stored as runs of contributors: a run of one texel repeated (the
 // clamped edge of a wide filter: most of the contributors of the deepest
-// levels) loads it once; a run of consecutive texels walks them.
+// levels) or a run of consecutive texels.  An output's longest consecutive run
+// is its main one (all there is, away from the edges).
+// Neighbouring outputs share most of their texels (5.4 outputs each with the
+// default Kaiser filter), so a wave sums kGroup = 4 outputs at once: the runs
+// before their main ones, output by output; then the texels of all four main
+// runs in order, each loaded and converted once for four products, with
+// weight 0 where it is outside an output's run (s + v * 0 == s up to the sign
+// of a zero sum, which nothing later tells apart); then the runs behind.
+// What bounds it: the loads and table look-ups of samples where lists are
+// short, one output's serial chain where they are long (dot_long).  3840x2160
+// with the default filter, one output at a time and a texel per load: pass 1
+// 595 us, pass 2 272 us; now 253 and 122 us.  Eight outputs at once would load a
+// quarter less, and multiply by more zeros.
 // The order of the passes is the reference's choice per level: X then Y
 // (always, for the multithreaded resampler) or, where the single-thread
 // Resampler delays X, Y then X.  Y then X is run as X then Y on the
 // transposed image -- the same sums in the same order.
 //
 // Layout in HBM (one plane per component c):
-//   level-0 planes ... bytes, lx[c][x][y] (column-major: the lanes of a wave
-//                      are 64 consecutive rows, so every contributor column is
-//                      one coalesced 64-byte load) and/or ly[c][y][x]; every
-//                      level re-reads them, so bytes rather than floats (the
-//                      sRGB table sits in LDS) cut the dominant traffic 4x;
+//   level-0 planes ... bytes, four texels of a line in a word: lx[c][x / 4][y]
+//                      (the lanes of a wave are 64 consecutive rows, so a
+//                      load is 256 coalesced bytes) and/or ly[c][y / 4][x];
+//                      every level re-reads them, so bytes rather than floats
+//                      (the sRGB table sits in LDS) cut the dominant traffic
+//                      4x;
 //   pass-1 output .... inter[c][line][o], o along the first pass's axis;
 //   pass 2 ........... lanes = 64 consecutive o, one wave per component, the
-//                      contributor list of the block's output line in scalar
-//                      registers; clamp to [0, 1], (int)(255 x + .5) or the
+//                      contributor lists of the block's four output lines in
+//                      scalar registers; clamp to [0, 1], (int)(255 x + .5) or the
 //                      linear-to-sRGB table, optional renorm_normal_map, one
 //                      RGBA8 texel per lane.
 // Both passes cover every level in one launch, the deepest levels first:
@@ -38,6 +51,7 @@
 #include <algorithm>
 #include <cstring>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "crn2_internal.h"
@@ -45,22 +59,32 @@
 
 namespace {
 
-// pass-1 outputs per lane: a lane's outputs are contiguous in its line of
-// the intermediate, so 16 of them leave as four 16-byte stores (lanes are
-// lines, a line apart); a level whose outputs have long lists takes one per
-// lane (shorter serial chains, more waves)
-constexpr uint32_t kOutPerLane = 16;
-constexpr uint32_t kLongList = 256;
+// outputs that a wave sums at once
+constexpr uint32_t kGroup = 4;
+// groups per pass-1 wave, one after the other: 16 outputs (64 bytes of each
+// lane's line) where lists are shorter than kMidList, one group where they are
+// longer (shorter serial chains, more waves)
+constexpr uint32_t kGroupsPerWave = 4;
+constexpr uint32_t kMidList = 64;
+// Lists of at least this many contributors per output take a wave for each
+// output (dot_long): the deepest levels' sums are the longest chains of the
+// launch.  Pass 1 has a wave for every 64 lines all the same, and a level of 690
+// contributors takes 17 us in groups; pass 2 has few waves, and the same level
+// takes 44 us in groups and 2 us a wave for each output.
+constexpr uint32_t kLongList = 1024, kLongList2 = 256;
+constexpr uint32_t kChunk = 256;   // weights that dot_long fetches at once
+constexpr uint32_t kRunPad = 16;   // a run's weights are padded with zeros to a multiple of this (so that runs start at 16-byte steps)
 
 struct Pass1Level {
     uint32_t unit0;   // first wave of this level
     uint32_t nlb;     // blocks of 64 lines
-    uint32_t per;     // outputs per lane (1 or kOutPerLane)
-    uint32_t runs;    // groups of `per` outputs
+    uint32_t single;  // 1: a wave sums one output, 0: `per` groups
+    uint32_t per;
+    uint32_t runs;    // waves per line block
     uint32_t lines;   // lines (rows for X first, columns for Y first)
     uint32_t d;       // outputs per line
     uint32_t s;       // source samples per line
-    uint32_t list;    // index of the list's offs[0]
+    uint32_t list;    // index of the list's first group
     uint32_t layout;  // 0 = lx, 1 = ly
     uint64_t inter;   // float offset of this level's pass-1 output
 };
@@ -69,6 +93,7 @@ struct Pass2Level {
     uint32_t block0;  // first block of this level
     uint32_t nxb;     // blocks of 64 pass-1 outputs
     uint32_t d2;      // output lines of pass 2
+    uint32_t single;  // 1: a block makes one of them, 0: kGroup
     uint32_t lines;   // contributors' range (pass-1 lines)
     uint32_t d;       // pass-1 outputs per line = lanes
     uint32_t list;
@@ -82,10 +107,24 @@ struct Run {
     uint32_t pix, n, step, w;
 };
 
+// kGroup neighbouring outputs, output i the sum of the runs [run[i], end[i]);
+// unless the list is long: texel pre_pix with pre_n weights per output at
+// wt[pre_w + kGroup * k + i] and then the runs [run[i], before[i]) (one of the
+// two is empty); texels pix .. pix + n - 1 (pix a multiple of 4)
+// with weights wt[w + kGroup * k + i] of output i stand for its runs
+// [before[i], after[i]); then texel post_pix and the runs [after[i], end[i]) in
+// the same way.  Outputs past the list's
+// last have no runs and weights 0.
+struct alignas(16) Group {
+    uint32_t pix, n, w;
+    uint32_t pre_pix, pre_n, pre_w, post_pix, post_n, post_w, pad[3];
+    uint32_t run[kGroup], before[kGroup], after[kGroup], end[kGroup];
+};
+
 struct Tables {
     const Pass1Level* p1;
     const Pass2Level* p2;
-    const uint32_t* sofs;  // runs of output o of a list: sofs[list + o] .. sofs[list + o + 1]
+    const Group* groups;
     const Run* runs;
     const float* wt;
     const float* s2l;
@@ -102,24 +141,24 @@ __device__ __forceinline__ float unif(float v) { return __int_as_float(__builtin
 enum Src { kFloat, kLinear8, kTable8 };
 
 template <Src S>
-__device__ __forceinline__ float sample(const void* base, uint32_t i, const float* tab)
+__device__ __forceinline__ float convert8(uint32_t v, const float* tab)
 {
-    if constexpr (S == kFloat) {
-        return static_cast<const float*>(base)[i];
-    } else {
-        const uint32_t v = static_cast<const uint8_t*>(base)[i];
-        if constexpr (S == kTable8) return tab[v];
-        else return __fmul_rn((float)v, 1.0f / 255.0f);
-    }
+    if constexpr (S == kTable8) return tab[v];
+    else return __fmul_rn((float)v, 1.0f / 255.0f);
 }
 
-// s + src(p * stride + lane) * w over the runs [rb, re) of one output, in
-// order.  Lists, runs and weights are wave-uniform (scalar loads); each
-// contributor of a consecutive run is one coalesced load of 64 samples, 16 in
-// flight.  A batch past the end of a run repeats its last texel with weight
-// 0: s + v * 0 == s (up to the sign of a zero sum), so the sums are the
-// reference's.  The weights of a batch are read as 16 consecutive floats
-// (the table buffer continues past the last list).
+// Texel p of the lane's line.
+template <Src S>
+__device__ __forceinline__ float sample(const void* base, uint32_t p, uint32_t lane, uint32_t stride, const float* tab)
+{
+    if constexpr (S == kFloat) return static_cast<const float*>(base)[p * stride + lane];
+    else return convert8<S>(static_cast<const uint8_t*>(base)[4 * ((p >> 2) * stride + lane) + (p & 3u)], tab);
+}
+
+// s + src(p) * w over the runs [rb, re) of one output, in order.  Runs and
+// weights are wave-uniform (scalar loads).  A batch past the end of a run
+// repeats its last texel with weight 0; the weights of a batch are read as 16
+// consecutive floats (the table buffer continues past the last list).
 template <Src S>
 __device__ __forceinline__ float dot_runs(const Tables& t, uint32_t rb, uint32_t re, const void* base,
                                           uint32_t lane, uint32_t stride, float s, const float* tab)
@@ -129,7 +168,7 @@ __device__ __forceinline__ float dot_runs(const Tables& t, uint32_t rb, uint32_t
         const uint32_t n = uni(r.n), p = uni(r.pix);
         const float* wp = t.wt + uni(r.w);
         if (uni(r.step) == 0) {
-            const float v = sample<S>(base, p * stride + lane, tab);
+            const float v = sample<S>(base, p, lane, stride, tab);
             uint32_t k = 0;
             for (; k + 16 <= n; k += 16) {
 #pragma unroll
@@ -140,7 +179,7 @@ __device__ __forceinline__ float dot_runs(const Tables& t, uint32_t rb, uint32_t
             for (uint32_t k = 0; k < n; k += 16) {
                 float v[16];
 #pragma unroll
-                for (int i = 0; i < 16; i++) v[i] = sample<S>(base, (p + min(k + i, n - 1)) * stride + lane, tab);
+                for (int i = 0; i < 16; i++) v[i] = sample<S>(base, p + min(k + i, n - 1), lane, stride, tab);
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const float w = unif(wp[k + i]);
@@ -152,13 +191,164 @@ __device__ __forceinline__ float dot_runs(const Tables& t, uint32_t rb, uint32_t
     return s;
 }
 
+// kGroup sums over one texel repeated: n weights per output, a multiple of 4.
+template <Src S>
+__device__ __forceinline__ void dot_repeat(const float* wp, uint32_t n, const void* base, uint32_t p, uint32_t lane,
+                                           uint32_t stride, float (&s)[kGroup], const float* tab)
+{
+    if (!n) return;
+    const float v = sample<S>(base, p, lane, stride, tab);
+    for (uint32_t k = 0; k < n; k += 4) {
+#pragma unroll
+        for (uint32_t b = 0; b < 4; b++) {
+#pragma unroll
+            for (uint32_t i = 0; i < kGroup; i++)
+                s[i] = __fadd_rn(s[i], __fmul_rn(v, unif(wp[kGroup * (k + b) + i])));
+        }
+    }
+}
+
+// The kGroup sums of group G.  Its texels come in batches of 8, the next
+// batch's loads in flight while one is summed; a batch past the end repeats
+// the last texels with weights 0 (the table holds them).
+template <Src S>
+__device__ __forceinline__ void dot_group(const Tables& t, const Group& G, const void* base, uint32_t lane,
+                                          uint32_t stride, float (&s)[kGroup], const float* tab)
+{
+#pragma unroll
+    for (uint32_t i = 0; i < kGroup; i++)
+        s[i] = dot_runs<S>(t, uni(G.run[i]), uni(G.before[i]), base, lane, stride, 0.0f, tab);
+    dot_repeat<S>(t.wt + uni(G.pre_w), uni(G.pre_n), base, uni(G.pre_pix), lane, stride, s, tab);
+    const uint32_t p = uni(G.pix), n = uni(G.n);
+    const float* wp = t.wt + uni(G.w);
+    constexpr uint32_t kBatch = 8, kWords = S == kFloat ? kBatch : kBatch / 4;
+    typedef typename std::conditional<S == kFloat, float, uint32_t>::type Word;
+    const Word* src = static_cast<const Word*>(base) + (size_t)(S == kFloat ? p : p >> 2) * stride + lane;
+    const uint32_t words = S == kFloat ? n : (n + 3) >> 2;
+    Word v[kWords];
+#pragma unroll
+    for (uint32_t i = 0; i < kWords; i++) v[i] = words ? src[min(i, words - 1) * stride] : Word(0);
+    for (uint32_t k = 0, w = 0; k < n; k += kBatch) {
+        w += kWords;
+        Word x[kWords];
+#pragma unroll
+        for (uint32_t i = 0; i < kWords; i++) x[i] = src[min(w + i, words - 1) * stride];
+#pragma unroll
+        for (uint32_t b = 0; b < kBatch; b++) {
+            float f;
+            if constexpr (S == kFloat) f = v[b];
+            else f = convert8<S>((v[b / 4] >> (8 * (b % 4))) & 0xFFu, tab);
+#pragma unroll
+            for (uint32_t i = 0; i < kGroup; i++)
+                s[i] = __fadd_rn(s[i], __fmul_rn(f, unif(wp[kGroup * (k + b) + i])));
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < kWords; i++) v[i] = x[i];
+    }
+    dot_repeat<S>(t.wt + uni(G.post_w), uni(G.post_n), base, uni(G.post_pix), lane, stride, s, tab);
+#pragma unroll
+    for (uint32_t i = 0; i < kGroup; i++)
+        s[i] = dot_runs<S>(t, uni(G.after[i]), uni(G.end[i]), base, lane, stride, s[i], tab);
+}
+
+// One output's sum where its list is long: a serial chain of thousands of
+// products and adds, which nothing overlaps at the end of the launch, so all
+// that it reads is under way long before.  The weights come 256 at a time,
+// four to a lane, one to two chunks ahead of the sum, and are handed round
+// through `wl` (two chunks of LDS, this wave's own); a consecutive run's texels come 32 (of
+// the byte planes 64, four to a load) at a time, a batch ahead.  With scalar loads of the weights, and waits for each
+// batch of 16 texels, a contributor took some 60 cycles, and the one sum of the
+// deepest level of a 2160-row image all of pass 2's 272 us.
+template <Src S>
+__device__ float dot_long(const Tables& t, uint32_t rb, uint32_t re, const void* base, uint32_t lane,
+                          uint32_t stride, const float* tab, float* wl)
+{
+    const uint32_t me = threadIdx.x & 63u;
+    float s = 0.0f;
+    for (uint32_t g = rb; g < re; g++) {
+        const Run r = t.runs[g];
+        const uint32_t n = uni(r.n), p = uni(r.pix), step = uni(r.step);
+        const float4* wp = reinterpret_cast<const float4*>(t.wt + uni(r.w)) + me;
+        float4* mine = reinterpret_cast<float4*>(wl) + me;
+        // chunk 0 in place, chunk 1 under way
+        mine[0] = wp[0];
+        float4 ahead = wp[kChunk / 4];
+        auto chunk = [&](uint32_t c) {   // halfway through chunk c: puts chunk c + 1 in place
+            mine[kChunk / 4 * ((c + 1) & 1u)] = ahead;
+            ahead = wp[kChunk / 4 * (c + 2)];
+        };
+        auto read16 = [&](uint32_t k, float (&w)[16]) {
+            const float4* q = reinterpret_cast<const float4*>(wl + (k & (2 * kChunk - 1)));
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++) {
+                const float4 v = q[i];
+                w[4 * i] = v.x;
+                w[4 * i + 1] = v.y;
+                w[4 * i + 2] = v.z;
+                w[4 * i + 3] = v.w;
+            }
+        };
+        float w[16];
+        read16(0, w);
+        if (step == 0) {
+            const float v = sample<S>(base, p, lane, stride, tab);
+            for (uint32_t k = 0; k < n; k += 16) {
+                if ((k & (kChunk - 1)) == kChunk / 2) chunk(k / kChunk);
+                float wn[16];
+                read16(k + 16, wn);
+#pragma unroll
+                for (uint32_t i = 0; i < 16; i++) s = __fadd_rn(s, __fmul_rn(v, w[i]));
+#pragma unroll
+                for (uint32_t i = 0; i < 16; i++) w[i] = wn[i];
+            }
+        } else {
+            // (a run in the byte planes starts at a word: add_list)
+            typedef typename std::conditional<S == kFloat, float, uint32_t>::type Word;
+            constexpr uint32_t kPer = S == kFloat ? 1 : 4, kWords = S == kFloat ? 32 : 16, kBatch = kPer * kWords;
+            const Word* src = static_cast<const Word*>(base) + (size_t)(p / kPer) * stride + lane;
+            const uint32_t words = (n + kPer - 1) / kPer;
+            Word v[kWords];
+#pragma unroll
+            for (uint32_t i = 0; i < kWords; i++) v[i] = src[min(i, words - 1) * stride];
+            for (uint32_t k = 0, q = 0; k < n; k += kBatch) {
+                q += kWords;
+                Word vn[kWords];
+#pragma unroll
+                for (uint32_t i = 0; i < kWords; i++) vn[i] = src[min(q + i, words - 1) * stride];
+#pragma unroll
+                for (uint32_t h = 0; h < kBatch / 16; h++) {
+                    const uint32_t at = k + 16 * h;
+                    if (at < n) {
+                        if ((at & (kChunk - 1)) == kChunk / 2) chunk(at / kChunk);
+                        float wn[16];
+                        read16(at + 16, wn);
+#pragma unroll
+                        for (uint32_t i = 0; i < 16; i++) {
+                            float f;
+                            if constexpr (S == kFloat) f = v[16 * h + i];
+                            else f = convert8<S>((v[4 * h + i / 4] >> (8 * (i % 4))) & 0xFFu, tab);
+                            s = __fadd_rn(s, __fmul_rn(f, w[i]));
+                        }
+#pragma unroll
+                        for (uint32_t i = 0; i < 16; i++) w[i] = wn[i];
+                    }
+                }
+#pragma unroll
+                for (uint32_t i = 0; i < kWords; i++) v[i] = vn[i];
+            }
+        }
+    }
+    return s;
+}
+
 // ------------------------------------------------------------ level-0 planes
 
-// RGBA8 -> one byte plane per component, column-major (lx) and/or row-major
-// (ly); 32x32 tiles, the column-major planes written from the transposed tile.
+// RGBA8 -> byte planes per component, a word for four texels along x (lx) and/or
+// along y (ly), zero past the edge; also copies the image to `copy` (level 0 of
+// the chain) where that is another buffer.  32x32 tiles.
 __global__ void __launch_bounds__(256) mip_planes_kernel(const uint32_t* __restrict__ rgba, uint32_t w, uint32_t h,
-                                                         uint8_t* __restrict__ lx, uint8_t* __restrict__ ly,
-                                                         uint32_t ncomp)
+                                                         uint32_t* __restrict__ lx, uint32_t* __restrict__ ly,
+                                                         uint32_t ncomp, uint32_t* __restrict__ copy)
 {
     __shared__ uint32_t tile[32][33];
     const uint32_t tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
@@ -169,31 +359,41 @@ __global__ void __launch_bounds__(256) mip_planes_kernel(const uint32_t* __restr
         const bool in = x < w && y < h;
         const uint32_t p = in ? rgba[(size_t)y * w + x] : 0;
         tile[ty + 8 * i][tx] = p;
-        if (ly && in)
-            for (uint32_t c = 0; c < ncomp; c++) ly[((size_t)c * h + y) * w + x] = (uint8_t)(p >> (8 * c));
+        if (copy && in) copy[(size_t)y * w + x] = p;
     }
-    if (!lx) return;
     __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint32_t x = x0 + ty + 8 * i, y = y0 + tx;
-        if (x < w && y < h) {
-            const uint32_t p = tile[tx][ty + 8 * i];
-            for (uint32_t c = 0; c < ncomp; c++) lx[((size_t)c * w + x) * h + y] = (uint8_t)(p >> (8 * c));
+    const uint32_t w4 = (w + 3) / 4, h4 = (h + 3) / 4;
+    auto gather = [](uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t comp) {
+        const uint32_t k = 8 * comp;
+        return ((a >> k) & 0xFFu) | ((b >> k) & 0xFFu) << 8 | ((c >> k) & 0xFFu) << 16 | (d >> k) << 24;
+    };
+    if (lx) {
+        const uint32_t q = x0 / 4 + ty, y = y0 + tx;
+        if (q < w4 && y < h) {
+            const uint32_t* r = &tile[tx][4 * ty];
+            for (uint32_t c = 0; c < ncomp; c++) lx[((size_t)c * w4 + q) * h + y] = gather(r[0], r[1], r[2], r[3], c);
+        }
+    }
+    if (ly) {
+        const uint32_t q = y0 / 4 + ty, x = x0 + tx;
+        if (q < h4 && x < w) {
+            const uint32_t a = tile[4 * ty][tx], b = tile[4 * ty + 1][tx], c2 = tile[4 * ty + 2][tx],
+                           d = tile[4 * ty + 3][tx];
+            for (uint32_t c = 0; c < ncomp; c++) ly[((size_t)c * h4 + q) * w + x] = gather(a, b, c2, d, c);
         }
     }
 }
 
 // ------------------------------------------------------------------- pass 1
 
-// One wave per (level, component, 64 lines, 1 or kOutPerLane outputs); lanes
-// are lines.  Results wait in LDS (each lane's own) and leave as rows.
-__global__ void __launch_bounds__(256) mip_pass1_kernel(Tables t, const uint8_t* __restrict__ lx,
-                                                        const uint8_t* __restrict__ ly, float* __restrict__ inter,
+// One wave per (level, component, 64 lines, `per` groups or one
+// output); lanes are lines.
+__global__ void __launch_bounds__(256) mip_pass1_kernel(Tables t, const uint32_t* __restrict__ lx,
+                                                        const uint32_t* __restrict__ ly, float* __restrict__ inter,
                                                         uint32_t nlevels, uint32_t units, uint32_t ncomp, int srgb)
 {
-    __shared__ float stage[4][kOutPerLane][64];
     __shared__ float tab[256];
+    __shared__ __align__(16) float wl[4][2 * kChunk];
     tab[threadIdx.x] = t.s2l[threadIdx.x];
     __syncthreads();
     const uint32_t u = uni(blockIdx.x * 4 + (threadIdx.x >> 6));
@@ -208,26 +408,32 @@ __global__ void __launch_bounds__(256) mip_pass1_kernel(Tables t, const uint8_t*
     const uint32_t line = lb * 64 + (threadIdx.x & 63);
     const bool valid = line < L.lines;
     const uint32_t rl = valid ? line : L.lines - 1;
-    const uint8_t* base = (L.layout ? ly : lx) + (size_t)c * L.s * L.lines;
-    float* out = inter + L.inter + ((size_t)c * L.lines + rl) * L.d + run * L.per;
-    const uint32_t nout = min(L.per, L.d - run * L.per);
-    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t* base = (L.layout ? ly : lx) + (size_t)c * ((L.s + 3) / 4) * L.lines;
     const bool table = srgb && c < 3;
-    for (uint32_t r = 0; r < nout; r++) {
-        const uint32_t o = run * L.per + r;
-        const uint32_t rb = uni(t.sofs[L.list + o]), re = uni(t.sofs[L.list + o + 1]);
-        stage[w][r][lane] = table ? dot_runs<kTable8>(t, rb, re, base, rl, L.lines, 0.0f, tab)
-                                  : dot_runs<kLinear8>(t, rb, re, base, rl, L.lines, 0.0f, tab);
+    if (L.single) {
+        const Group& G = t.groups[L.list + run / kGroup];
+        const uint32_t rb = uni(G.run[run % kGroup]), re = uni(G.end[run % kGroup]);
+        float* mine = wl[threadIdx.x >> 6];
+        const float s = table ? dot_long<kTable8>(t, rb, re, base, rl, L.lines, tab, mine)
+                              : dot_long<kLinear8>(t, rb, re, base, rl, L.lines, tab, mine);
+        if (valid) inter[L.inter + ((size_t)c * L.lines + rl) * L.d + run] = s;
+        return;
     }
-    if (!valid) return;
-    // each lane reads back only what it wrote
-    if (nout == kOutPerLane && !(reinterpret_cast<uintptr_t>(out) & 15)) {
+    const uint32_t ngroups = (L.d + kGroup - 1) / kGroup;
+    for (uint32_t g = run * L.per; g < min(ngroups, (run + 1) * L.per); g++) {
+        float s[kGroup];
+        const Group& G = t.groups[L.list + g];
+        if (table) dot_group<kTable8>(t, G, base, rl, L.lines, s, tab);
+        else dot_group<kLinear8>(t, G, base, rl, L.lines, s, tab);
+        float* out = inter + L.inter + ((size_t)c * L.lines + rl) * L.d + kGroup * g;
+        if (!valid) continue;
+        if (!(L.d & 3u)) {
+            *reinterpret_cast<float4*>(out) = make_float4(s[0], s[1], s[2], s[3]);
+        } else {
 #pragma unroll
-        for (uint32_t q = 0; q < kOutPerLane; q += 4)
-            *reinterpret_cast<float4*>(out + q) =
-                make_float4(stage[w][q][lane], stage[w][q + 1][lane], stage[w][q + 2][lane], stage[w][q + 3][lane]);
-    } else {
-        for (uint32_t r = 0; r < nout; r++) out[r] = stage[w][r][lane];
+            for (uint32_t i = 0; i < kGroup; i++)
+                if (kGroup * g + i < L.d) out[i] = s[i];
+        }
     }
 }
 
@@ -273,41 +479,51 @@ __device__ void renorm(uint32_t* c)
     }
 }
 
-// One block per (level, output line of pass 2, 64 lanes), one wave per
-// component; texels packed by wave 0.
-__global__ void __launch_bounds__(256) mip_pass2_kernel(Tables t, const float* __restrict__ inter,
+// One block per (level, kGroup output lines of pass 2 or one, 64 lanes), one
+// wave per component; wave i packs the texels of line i.
+__global__ void __launch_bounds__(256, 4) mip_pass2_kernel(Tables t, const float* __restrict__ inter,
                                                         uint32_t* __restrict__ out, uint32_t nlevels,
                                                         uint32_t ncomp, int srgb, int renormalize)
 {
-    __shared__ uint32_t px[4][64];
+    __shared__ uint32_t px[kGroup][4][64];
+    __shared__ __align__(16) float wl[4][2 * kChunk];
     const uint32_t b = blockIdx.x;
     uint32_t l = 0;
     while (l + 1 < nlevels && t.p2[l + 1].block0 <= b) l++;
     const Pass2Level L = t.p2[l];
     const uint32_t rem = b - L.block0;
-    const uint32_t xb = rem % L.nxb, o2 = rem / L.nxb;
+    const uint32_t xb = rem % L.nxb, g = rem / L.nxb;
     const uint32_t c = uni(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const uint32_t x = xb * 64 + lane;
     const bool valid = x < L.d;
     const uint32_t rx = valid ? x : L.d - 1;
-    uint32_t val = 255;
+    float s[kGroup] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const uint32_t nout = L.single ? 1 : kGroup;
     if (c < ncomp) {
         const float* base = inter + L.inter + (size_t)c * L.lines * L.d;
-        float s = dot_runs<kFloat>(t, uni(t.sofs[L.list + o2]), uni(t.sofs[L.list + o2 + 1]), base, rx, L.d, 0.0f,
-                                   nullptr);
-        s = clamp01(s);
-        if (!srgb || c == 3) {
-            const int v = (int)__fadd_rn(__fmul_rn(255.0f, s), .5f);
-            val = (uint32_t)min(255, max(0, v));
+        if (L.single) {
+            const Group& G = t.groups[L.list + g / kGroup];
+            s[0] = dot_long<kFloat>(t, uni(G.run[g % kGroup]), uni(G.end[g % kGroup]), base, rx, L.d, nullptr, wl[c]);
         } else {
-            const int j = (int)__fadd_rn(__fmul_rn(8192.0f, s), .5f);
-            val = t.l2s[min(8191, max(0, j))];
+            dot_group<kFloat>(t, t.groups[L.list + g], base, rx, L.d, s, nullptr);
         }
     }
-    px[c][lane] = val;
+#pragma unroll
+    for (uint32_t i = 0; i < kGroup; i++) {
+        uint32_t val = 255;
+        const float v = clamp01(s[i]);
+        if (c >= ncomp) {
+        } else if (!srgb || c == 3) {
+            val = (uint32_t)min(255, max(0, (int)__fadd_rn(__fmul_rn(255.0f, v), .5f)));
+        } else {
+            val = t.l2s[min(8191, max(0, (int)__fadd_rn(__fmul_rn(8192.0f, v), .5f)))];
+        }
+        px[i][c][lane] = val;
+    }
     __syncthreads();
-    if (c == 0 && valid) {
-        uint32_t q[4] = {px[0][lane], px[1][lane], px[2][lane], px[3][lane]};
+    const uint32_t o2 = nout * g + c;
+    if (c < nout && o2 < L.d2 && valid) {
+        uint32_t q[4] = {px[c][0][lane], px[c][1][lane], px[c][2][lane], px[c][3][lane]};
         if (renormalize) renorm(q);
         out[L.out + (size_t)o2 * L.os_o + (size_t)x * L.os_lane] = q[0] | q[1] << 8 | q[2] << 16 | q[3] << 24;
     }
@@ -328,7 +544,7 @@ struct crn2_mip_plan {
     void* tables = nullptr;
     void* scratch = nullptr;
     Tables t{};
-    uint8_t *lx = nullptr, *ly = nullptr;  // level-0 byte planes
+    uint32_t *lx = nullptr, *ly = nullptr;  // level-0 planes, four texels a word
     float* inter = nullptr;
     uint32_t units1 = 0, blocks2 = 0;
     // stage timing (HIP events on the run stream): planes, pass 1, pass 2
@@ -421,32 +637,94 @@ int crn2_mip_plan_create(uint32_t width, uint32_t height, const crn2_mip_params*
     // host image of the device tables
     std::vector<Pass1Level> p1(nl);
     std::vector<Pass2Level> p2(nl);
-    std::vector<uint32_t> sofs;
+    std::vector<Group> groups;
     std::vector<Run> runs;
     std::vector<float> wt;
     bool need_lx = false, need_ly = false;
     uint64_t inter_floats = 0;
     uint32_t units = 0, blocks = 0;
-    // a list as runs: one texel repeated (step 0) or consecutive texels (step 1)
-    auto add_list = [&](const crn2mip::List& L) {
-        const uint32_t at = (uint32_t)sofs.size(), base = (uint32_t)wt.size();
-        wt.insert(wt.end(), L.wt.begin(), L.wt.end());
-        for (size_t o = 0; o + 1 < L.offs.size(); o++) {
-            sofs.push_back((uint32_t)runs.size());
-            for (uint32_t k = L.offs[o], end = L.offs[o + 1]; k < end;) {
-                const uint32_t p = L.pix[k];
-                uint32_t n = 1, step = 1;
-                if (k + 1 < end && L.pix[k + 1] == p) {
-                    step = 0;
-                    while (k + n < end && L.pix[k + n] == p) n++;
-                } else {
-                    while (k + n < end && L.pix[k + n] == p + n) n++;
+    // a list as runs (one texel repeated, step 0, or consecutive texels, step 1)
+    // and groups of outputs
+    auto add_list = [&](const crn2mip::List& L, bool single) {
+        const uint32_t at = (uint32_t)groups.size();
+        const size_t n = L.offs.size() - 1;
+        for (size_t o0 = 0; o0 < n; o0 += kGroup) {
+            Group G;
+            std::memset(&G, 0, sizeof(G));
+            uint32_t lo = 0xFFFFFFFFu, hi = 0;
+            Run main[kGroup] = {};
+            for (uint32_t i = 0; i < kGroup && o0 + i < n; i++) {
+                G.run[i] = (uint32_t)runs.size();
+                uint32_t best = 0xFFFFFFFFu;
+                for (uint32_t k = L.offs[o0 + i], end = L.offs[o0 + i + 1]; k < end;) {
+                    const uint32_t p = L.pix[k];
+                    uint32_t m = 1, step = 1;
+                    if (k + 1 < end && L.pix[k + 1] == p) {
+                        step = 0;
+                        while (k + m < end && L.pix[k + m] == p) m++;
+                    } else {
+                        while (k + m < end && L.pix[k + m] == p + m) m++;
+                    }
+                    if (step && (best == 0xFFFFFFFFu || m > runs[best].n)) best = (uint32_t)runs.size();
+                    // a consecutive run starts at a multiple of 4, from there on with weights 0
+                    const uint32_t lead = step ? p & 3u : 0;
+                    runs.push_back(Run{p - lead, m + lead, step, (uint32_t)wt.size()});
+                    wt.resize(wt.size() + lead, 0.0f);
+                    wt.insert(wt.end(), L.wt.begin() + k, L.wt.begin() + k + m);
+                    wt.resize((wt.size() - runs.back().w + kRunPad - 1) / kRunPad * kRunPad + runs.back().w, 0.0f);
+                    k += m;
                 }
-                runs.push_back(Run{p, n, step, base + k});
-                k += n;
+                G.end[i] = (uint32_t)runs.size();
+                G.before[i] = G.after[i] = G.end[i];
+                if (best == 0xFFFFFFFFu) continue;
+                G.before[i] = best;
+                G.after[i] = best + 1;
+                main[i] = runs[best];
+                lo = std::min(lo, main[i].pix);
+                hi = std::max(hi, main[i].pix + main[i].n);
             }
+            if (hi && !single) {
+                G.pix = lo & ~3u;
+                G.n = hi - G.pix;
+                G.w = (uint32_t)wt.size();
+                wt.resize(wt.size() + (size_t)kGroup * ((G.n + 7) & ~7u), 0.0f);
+                for (uint32_t i = 0; i < kGroup; i++)
+                    for (uint32_t k = 0; k < main[i].n; k++)
+                        wt[G.w + kGroup * (size_t)(main[i].pix - G.pix + k) + i] = wt[main[i].w + k];
+            }
+            // the runs on one side of the main ones, where each is at most one
+            // texel repeated, the same for all outputs: the shorter ones with
+            // weights 0 on the side away from the main runs
+            auto repeats = [&](uint32_t* from, uint32_t* to, bool before, uint32_t& pix, uint32_t& cnt, uint32_t& at_w) {
+                uint32_t n_max = 0, texel = 0;
+                for (uint32_t i = 0; i < kGroup; i++) {
+                    if (from[i] == to[i]) continue;
+                    const Run& r = runs[from[i]];
+                    if (to[i] - from[i] > 1 || r.step || (n_max && r.pix != texel)) return;
+                    texel = r.pix;
+                    n_max = std::max(n_max, r.n);
+                }
+                if (!n_max) return;
+                n_max = (n_max + 3) & ~3u;
+                pix = texel;
+                cnt = n_max;
+                at_w = (uint32_t)wt.size();
+                wt.resize(wt.size() + (size_t)kGroup * n_max, 0.0f);
+                for (uint32_t i = 0; i < kGroup; i++) {
+                    if (from[i] == to[i]) continue;
+                    const Run r = runs[from[i]];
+                    for (uint32_t k = 0; k < r.n; k++)
+                        wt[at_w + kGroup * (size_t)(before ? n_max - r.n + k : k) + i] = wt[r.w + k];
+                    if (before) from[i] = to[i];
+                    else to[i] = from[i];
+                }
+            };
+            if (hi && !single) {
+                repeats(G.run, G.before, true, G.pre_pix, G.pre_n, G.pre_w);
+                repeats(G.after, G.end, false, G.post_pix, G.post_n, G.post_w);
+            }
+            groups.push_back(G);
         }
-        sofs.push_back((uint32_t)runs.size());
         return at;
     };
     // deepest level first in both launches
@@ -463,20 +741,22 @@ int crn2_mip_plan_create(uint32_t width, uint32_t height, const crn2_mip_params*
         a.layout = v.xfirst ? 0 : 1;
         (v.xfirst ? need_lx : need_ly) = true;
         a.nlb = (a.lines + 63) / 64;
-        a.per = first.ops() / a.d >= kLongList ? 1 : kOutPerLane;
-        a.runs = (a.d + a.per - 1) / a.per;
+        a.single = first.ops() / a.d >= kLongList ? 1 : 0;
+        a.per = first.ops() / a.d >= kMidList ? 1 : kGroupsPerWave;
+        a.runs = a.single ? a.d : ((a.d + kGroup - 1) / kGroup + a.per - 1) / a.per;
         a.unit0 = units;
         units += nc * a.nlb * a.runs;
-        a.list = add_list(first);
+        a.list = add_list(first, a.single);
         a.inter = inter_floats;
-        inter_floats += (uint64_t)nc * a.lines * a.d;
+        inter_floats += ((uint64_t)nc * a.lines * a.d + 3) & ~3ull;   // (16-byte stores)
         b.lines = a.lines;
         b.d = a.d;
         b.d2 = v.xfirst ? v.height : v.width;
         b.nxb = (b.d + 63) / 64;
         b.block0 = blocks;
-        blocks += b.d2 * b.nxb;
-        b.list = add_list(second);
+        b.single = second.ops() / b.d2 >= kLongList2 ? 1 : 0;
+        blocks += (b.single ? b.d2 : (b.d2 + kGroup - 1) / kGroup) * b.nxb;
+        b.list = add_list(second, b.single);
         b.inter = a.inter;
         b.out = p->level_ofs[level] / 4;
         b.os_lane = v.xfirst ? 1 : v.width;
@@ -493,12 +773,12 @@ int crn2_mip_plan_create(uint32_t width, uint32_t height, const crn2_mip_params*
     at = align_up(at + nl * sizeof(Pass1Level), 256);
     const size_t o_p2 = at;
     at = align_up(at + nl * sizeof(Pass2Level), 256);
-    const size_t o_sofs = at;
-    at = align_up(at + sofs.size() * 4, 256);
+    const size_t o_groups = at;
+    at = align_up(at + groups.size() * sizeof(Group), 256);
     const size_t o_runs = at;
     at = align_up(at + runs.size() * sizeof(Run), 256);
     const size_t o_wt = at;
-    at = align_up(at + wt.size() * 4 + 64, 256);  // batches read up to 15 weights past a list
+    at = align_up(at + wt.size() * 4 + 4 * 3 * kChunk, 256);  // chunks read fewer than 3 * kChunk weights past a run
     const size_t o_s2l = at;
     at = align_up(at + sizeof(s2l), 256);
     const size_t o_l2s = at;
@@ -506,13 +786,14 @@ int crn2_mip_plan_create(uint32_t width, uint32_t height, const crn2_mip_params*
     std::vector<uint8_t> host(at, 0);
     std::memcpy(host.data() + o_p1, p1.data(), nl * sizeof(Pass1Level));
     std::memcpy(host.data() + o_p2, p2.data(), nl * sizeof(Pass2Level));
-    std::memcpy(host.data() + o_sofs, sofs.data(), sofs.size() * 4);
+    std::memcpy(host.data() + o_groups, groups.data(), groups.size() * sizeof(Group));
     std::memcpy(host.data() + o_runs, runs.data(), runs.size() * sizeof(Run));
     std::memcpy(host.data() + o_wt, wt.data(), wt.size() * 4);
     std::memcpy(host.data() + o_s2l, s2l, sizeof(s2l));
     std::memcpy(host.data() + o_l2s, l2s.data(), l2s.size());
-    const uint64_t plane = align_up((uint64_t)nc * width * height, 256);  // bytes
-    const uint64_t scratch_bytes = (need_lx ? plane : 0) + (need_ly ? plane : 0) + inter_floats * sizeof(float);
+    const uint64_t plane_x = align_up((uint64_t)nc * ((width + 3) / 4) * height * 4, 256);  // bytes
+    const uint64_t plane_y = align_up((uint64_t)nc * ((height + 3) / 4) * width * 4, 256);
+    const uint64_t scratch_bytes = (need_lx ? plane_x : 0) + (need_ly ? plane_y : 0) + inter_floats * sizeof(float);
     int rc = CRN2_OK;
     if (!hip_ok(hipMalloc(&p->tables, at)) || !hip_ok(hipMalloc(&p->scratch, scratch_bytes)))
         rc = CRN2_ENOMEM;
@@ -525,14 +806,14 @@ int crn2_mip_plan_create(uint32_t width, uint32_t height, const crn2_mip_params*
     const uint8_t* d = static_cast<const uint8_t*>(p->tables);
     p->t.p1 = reinterpret_cast<const Pass1Level*>(d + o_p1);
     p->t.p2 = reinterpret_cast<const Pass2Level*>(d + o_p2);
-    p->t.sofs = reinterpret_cast<const uint32_t*>(d + o_sofs);
+    p->t.groups = reinterpret_cast<const Group*>(d + o_groups);
     p->t.runs = reinterpret_cast<const Run*>(d + o_runs);
     p->t.wt = reinterpret_cast<const float*>(d + o_wt);
     p->t.s2l = reinterpret_cast<const float*>(d + o_s2l);
     p->t.l2s = d + o_l2s;
     uint8_t* f = static_cast<uint8_t*>(p->scratch);
-    if (need_lx) { p->lx = f; f += plane; }
-    if (need_ly) { p->ly = f; f += plane; }
+    if (need_lx) { p->lx = reinterpret_cast<uint32_t*>(f); f += plane_x; }
+    if (need_ly) { p->ly = reinterpret_cast<uint32_t*>(f); f += plane_y; }
     p->inter = reinterpret_cast<float*>(f);
     *out = p;
     return CRN2_OK;
@@ -555,12 +836,15 @@ int crn2_mip_plan_run(crn2_mip_plan* p, const void* rgba, void* out, uint64_t ou
     if ((reinterpret_cast<uintptr_t>(rgba) | reinterpret_cast<uintptr_t>(out)) & 3) return CRN2_EINVAL;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const uint64_t l0 = (uint64_t)p->width * p->height * 4;
-    if (out != rgba && !hip_ok(hipMemcpyAsync(out, rgba, l0, hipMemcpyDeviceToDevice, st))) return CRN2_EHIP;
-    if (p->levels == 1) return CRN2_OK;
+    if (p->levels == 1) {
+        if (out != rgba && !hip_ok(hipMemcpyAsync(out, rgba, l0, hipMemcpyDeviceToDevice, st))) return CRN2_EHIP;
+        return CRN2_OK;
+    }
     const int srgb = (p->params.flags & CRN2_MIP_SRGB) != 0;
     if (p->prof) (void)hipEventRecord(p->ev[0], st);
     hipLaunchKernelGGL(mip_planes_kernel, dim3((p->width + 31) / 32, (p->height + 31) / 32), dim3(256), 0, st,
-                       static_cast<const uint32_t*>(rgba), p->width, p->height, p->lx, p->ly, p->ncomp);
+                       static_cast<const uint32_t*>(rgba), p->width, p->height, p->lx, p->ly, p->ncomp,
+                       out != rgba ? static_cast<uint32_t*>(out) : nullptr);
     if (p->prof) (void)hipEventRecord(p->ev[1], st);
     hipLaunchKernelGGL(mip_pass1_kernel, dim3((p->units1 + 3) / 4), dim3(256), 0, st, p->t, p->lx, p->ly, p->inter,
                        p->levels - 1, p->units1, p->ncomp, srgb);

@@ -81,6 +81,16 @@ def test_every_filter_and_mode(gpu, filt, flags):
     assert_same(gpu_levels(img, filt, flags), oracle_levels(img, filt, flags)[0], (filt, flags))
 
 
+# One side long enough for every way of summing a list (groups of four outputs
+# with short, middle and long lists, an output a wave), the other odd; a filter
+# with one contributor per texel, and wrapped lists.
+@pytest.mark.parametrize("filt,flags", [(KAISER, SRGB | ALPHA), (LANCZOS4, ALPHA | WRAP), (BOX, SRGB)])
+@pytest.mark.parametrize("h,w", [(5, 1031), (1029, 67)])
+def test_list_lengths(gpu, h, w, filt, flags):
+    img = rand_img(h, w, 17)
+    assert_same(gpu_levels(img, filt, flags), oracle_levels(img, filt, flags)[0], (h, w, filt, flags))
+
+
 def test_yfirst_levels_are_exercised(gpu):
     for h, w in [(2048, 2), (1024, 3), (3, 1024)]:
         img = rand_img(h, w, 5)
