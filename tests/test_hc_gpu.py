@@ -67,6 +67,26 @@ def run_alpha_gpu(vals, ei, pal, sel, scatter):
             det.cpu().numpy().view(np.uint32), used.cpu().numpy())
 
 
+# Totals gathered per run of blocks: two and three times 16 blocks a workgroup
+# with a ragged last one, half of the blocks flat (one selector for all of
+# them), fewer and more selectors than a workgroup has slots for.
+@pytest.mark.parametrize("n,m", [(16391, 20), (24577, 300)])
+def test_totals_of_frequent_selectors(gpu, n, m):
+    from tests.hc_cases import make_alpha_case
+    blocks, ei, cols, sel = make_case(n, 30, m, seed=m, subblocks=False)
+    blocks[::2] = blocks[0, 0]
+    ei[::2] = ei[0]
+    _, _, d, u = run_gpu(blocks, ei, cols, sel, False, True)
+    _, _, rd, ru = oracle.hc_color_selectors(blocks, ei, cols, sel, False, True)
+    assert np.array_equal(d, rd) and np.array_equal(u, ru)
+    vals, ei, pal, _, sel = make_alpha_case(n, 30, m, seed=m)
+    vals[::2] = vals[0, 0]
+    ei[::2] = ei[0]
+    _, _, d, u = run_alpha_gpu(vals, ei, pal, sel, None)
+    _, _, rd, ru = oracle.hc_alpha_selectors(vals, ei, pal, sel, None)
+    assert np.array_equal(d, rd) and np.array_equal(u, ru)
+
+
 @pytest.mark.parametrize("n,k,m", [(1, 1, 1), (45, 4, 31), (700, 50, 1500), (3000, 200, 9000)])
 @pytest.mark.parametrize("scatter", [False, True])
 def test_alpha_matches_oracle(gpu, n, k, m, scatter):
