@@ -1924,10 +1924,15 @@ static void ctx_free_device(crn2_unpack_ctx* c)
     if (c->d_mem) (void)hipFree(c->d_mem);
 }
 
+// A refused allocation is answered by the caller (an error code, or smaller
+// tables), so its error leaves the thread here: the runtime keeps it through
+// later successes, and the next launch's check would take it for its own.
 template <typename T>
 static hipError_t dmalloc(T** p, size_t bytes)
 {
-    return hipMalloc(reinterpret_cast<void**>(p), std::max<size_t>(bytes, 16));
+    const hipError_t e = hipMalloc(reinterpret_cast<void**>(p), std::max<size_t>(bytes, 16));
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
 }
 
 static size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
