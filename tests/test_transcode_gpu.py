@@ -220,7 +220,7 @@ def test_row_remainders_both_tables(gpu, fmt, copies):
             assert np.array_equal(got, exp), (bw, fmt)
 
 
-def test_four_blocks_of_256_bits(gpu):
+def wide_file():
     """Symbols of geometric frequencies, and groups of four odd-row blocks whose
     every symbol occurs once among 98,304: 16-bit codes in all four models, so
     that a group takes 256 bits, which its table entry's byte holds as 0."""
@@ -240,12 +240,38 @@ def test_four_blocks_of_256_bits(gpu):
     ae = rng.integers(0, 1 << 16, n, dtype=np.uint64).astype(np.uint32)
     cs = rng.integers(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32)
     al = rng.integers(0, 1 << 48, n, dtype=np.uint64)
-    data = texture.pack(4 * gw, 4 * gh, 1, 1, FMT_DXT5, ce, cs, ae, al, ends[0], idx[1], ends[1], idx[3])
+    return texture.pack(4 * gw, 4 * gh, 1, 1, FMT_DXT5, ce, cs, ae, al, ends[0], idx[1], ends[1], idx[3])
+
+
+def test_four_blocks_of_256_bits(gpu):
+    data = wide_file()
     exp = oracle_bytes(data)
     say("256-bit groups, file of", len(data))
     for copies in (1, 40):
         for got in run_plan([data], copies):
             assert np.array_equal(got, exp), copies
+
+
+# The walk over four-block tables with the small rings, which plans of at least
+# 512 levels take, and with the large ones: one large texture (of ordinary
+# codes, or of 16-bit ones, so that four blocks can take 256 bits) makes the
+# longest level, small ones of every format and row remainder the others.
+@pytest.mark.parametrize("sets,wide", [(1, False), (4, False), (1, True), (4, True)])
+def test_many_levels_beside_a_long_one(gpu, sets, wide):
+    big = wide_file() if wide else texture.synth_crn(1024, 61, FMT_DXT5)
+    small = []
+    for s in range(sets):
+        for i, bw in enumerate([2, 4, 6, 8, 10, 12, 14, 16, 18, 20, 22, 24, 26, 28, 30, 32, 34, 36, 46, 64]):
+            fmt = (FMT_DXT1, FMT_DXT5, FMT_DXN_XY, FMT_DXT5A)[(i + s) % 4]
+            small.append(texture.synth_crn((4 * bw - (i & 3), 40 + 8 * s), 300 + 20 * s + i, fmt))
+    files = [big] + small
+    levels = sum(crnd.get_texture_info(d)["levels"] for d in files)
+    assert (levels >= 512) == (sets == 4), levels
+    # within the line up to which plans take the four-block tables
+    assert 8 * sum(map(len, files)) + 12000 * levels < 30 * 8 * 0.6 * len(big)
+    say("one of", len(big), "bytes and", len(small), "small files,", levels, "levels, wide", wide)
+    for d, got in zip(files, run_plan(files)):
+        assert np.array_equal(got, oracle_bytes(d)), (len(d), crnd.get_texture_info(d))
 
 
 @pytest.mark.parametrize("fmt,pal,factor", crn_cases.SHRUNK)
