@@ -2080,15 +2080,30 @@ struct PlanPart {
 // write than O2 tables, at the whole chip's rate, and shorten the walk, which
 // lasts as long as its longest level, by 270 us per Mbit of that level (2048^2
 // DXT5 with its levels, 7.1 Mbit in all and 5.2 in level 0: walk 4.26 -> 2.87
-// ms, tables 45 -> 65 us; 64 textures of 64^2 to 1024^2: walk 1.24 -> 0.81 ms,
-// tables 122 -> 188 us; 32 pairs of 4096^2 DXT1 and DXT5, 74 times the longest
-// level: walk 17.9 -> 14.7 ms, tables 5.5 -> 8.2 ms, and four such plans on
-// four streams, where one's walk runs beside another's tables, 45.9 -> 65.2
-// ms).  Up to 32 times the longest level the tables cost a quarter of the gain.
-// The second bound keeps the tables within 5 GiB (O2: 2).
+// ms, tables 45 -> 65 us).
+// A plan alone gains far beyond the line below.  But where plans run on several
+// streams, one's tables run beside another's walk, and the chip's time decides,
+// of which a level takes about as much as 12 kbit of stream (a workgroup, its
+// first segments).  The line is where four plans at once, as many as a process
+// has hardware queues, begin to lose more than a plan alone gains.  Time with
+// O4 over time with O2, for one plan and for four at once, by the streams (with
+// 12 kbit for each level past one texture's) over the longest level:
+//   12 textures of 2048^2 DXT1   18   0.66  0.78
+//   12 of 1024^2 DXT5            19   0.70  0.90
+//   64 of 64^2 to 1024^2         21   0.84  1.07
+//   16 of 1024^2 DXT5            25   0.71  1.00
+//   28 of up to 325^2            27   0.79  1.11
+//   40 of up to 446^2            29   0.76  1.15
+//   49 of up to 531^2            32   0.85  1.21
+//   24 of 1024^2 DXT5            37   0.74  1.30
+//   40 of up to 193^2            75   0.89  1.18
+// The second bound keeps the tables within 6 GiB (24 B per bit where X is
+// written; O2: 10).
+constexpr uint64_t kLevelBits = 12000, kO4Limit = 30;
+
 static bool takes_o4(const std::vector<PlanPart>& parts)
 {
-    uint64_t total = 0, longest = 0;
+    uint64_t total = 0, longest = 0, levels = 0;
     for (const PlanPart& P : parts)
         for (uint32_t l = P.first; l < P.first + P.count; l++) {
             const Header& h = P.c->h;
@@ -2096,8 +2111,10 @@ static bool takes_o4(const std::vector<PlanPart>& parts)
             const uint64_t bits = 8 * (uint64_t)(P.src_override ? P.src_size : next - h.level_ofs[l]);
             total += bits;
             longest = std::max(longest, bits);
+            levels++;
         }
-    return total <= 32 * longest && total <= 1ull << 28;
+    const uint64_t more = levels > kMaxLevels ? levels - kMaxLevels : 0;   // than one texture's
+    return total + kLevelBits * more <= kO4Limit * longest && total <= 1ull << 28;
 }
 
 static int build_plan_as(std::vector<PlanPart>& parts, bool four, crn2_batch** out)

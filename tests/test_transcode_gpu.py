@@ -207,7 +207,7 @@ def oracle_bytes(data):
 
 
 # One file alone takes the tables of four odd-row blocks, 40 copies those of two
-# (more than 32 times the longest level): rows of 2 to 34 blocks end in every
+# (more than 30 times the longest level): rows of 2 to 34 blocks end in every
 # remainder of a 16-block group.
 @pytest.mark.parametrize("copies", [1, 40])
 @pytest.mark.parametrize("fmt", [FMT_DXT1, FMT_DXT5, FMT_DXN_XY])
