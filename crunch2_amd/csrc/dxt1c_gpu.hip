@@ -547,6 +547,7 @@ __device__ bool try_list(St& s, Lds& L, uint32_t kind, uint32_t n, int alt, bool
     bool took = false;
     while (first < n && s.best.err) {
         uint32_t cnt = 0, next = first;
+        __builtin_amdgcn_wave_barrier();   // the last batch has been read
         while (next < n && cnt < kBatch) {
             const uint32_t i = next + lane;
             uint32_t lo = 0, hi = 0;

@@ -1139,6 +1139,7 @@ __device__ inline bool wave_box_step(PolishLds& L, const WaveBlock& B, const u32
 {
     const uint32_t lane = threadIdx.x & 63u, group = lane >> 4;
     // the table: one move and entry of a channel per lane and turn
+    __builtin_amdgcn_wave_barrier();   // the last step's has been read
     for (uint32_t i = lane; i < 3 * 9 * 4; i += 64) {
         const uint32_t ch = i / 36, mv = i / 4 % 9, entry = i & 3u;
         const int e0 = (ch == 0 ? E.e[0][0] : ch == 1 ? E.e[0][1] : E.e[0][2]) + (int)(mv % 3) - 1;
