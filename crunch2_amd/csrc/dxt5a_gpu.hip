@@ -94,10 +94,14 @@ __device__ inline void pair_errors(uint32_t uval, uint32_t uw, uint32_t nu, uint
 __device__ inline E2Result dxt5a_search(const uint32_t (&w)[4], int quality, bool both)
 {
     const uint32_t lane = lane_id(), t = lane & 15u;
-    const uint32_t word = t < 8 ? (t < 4 ? w[0] : w[1]) : (t < 12 ? w[2] : w[3]);
+    // (values, not places: an array read at a lane's index would live in LDS, and each
+    // wave would read the launch packet in host memory for its place there, 10 us)
+    const uint32_t w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3];
+    const uint32_t word = t < 8 ? (t < 4 ? w0 : w1) : (t < 12 ? w2 : w3);
     const uint32_t mine = (word >> (8 * (t & 3u))) & 0xFFu;
     // distinct values in first-appearance order: lane u < nu holds value u
     uint32_t before = 0, count = 0;
+#pragma unroll
     for (uint32_t k = 0; k < 16; k++) {
         const bool eq = ((w[k >> 2] >> (8 * (k & 3u))) & 0xFFu) == mine;
         before |= eq && k < t ? 1u : 0u;
@@ -246,11 +250,12 @@ __device__ inline E2Result dxt5a_wave(const uint32_t (&w)[4], uint32_t n, int qu
     return r;
 }
 
-// Blocks per wave: one while the waves fill the 1,024 SIMDs at most 32 deep
-// (a wave searches its blocks in turn), up to one per lane beyond,
-// so that images of flat blocks cost a lane each.  Measured at 1024^2 (65,536
-// blocks), runs of 1 / 4: a normal map 1,267 / 1,359 us, a flat channel 21 / 13.
-inline uint32_t blocks_per_wave(uint64_t n) { return (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, n >> 15)); }
+// Blocks per wave: one up to 43,690 blocks, then as many as keep the waves to
+// about 21,845 (a wave searches its blocks in turn, but one with nothing to
+// search costs little more than its start), up to one per lane.  Measured at
+// 1024^2 (65,536 blocks), runs of 2 / 3 / 4: a normal map 1,289 / 1,320 / 1,354
+// us, a flat channel 10.2 / 7.8 / 7.8 (one lane per block: 8.5).
+inline uint32_t blocks_per_wave(uint64_t n) { return (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, n * 3 >> 16)); }
 
 // The wave's first block and its number of blocks.
 __device__ inline uint32_t wave_blocks(uint32_t per, uint32_t total, uint32_t& first)

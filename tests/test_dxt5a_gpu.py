@@ -40,7 +40,7 @@ def test_image_encode_matches_oracle(gpu, w, h, comp):
     assert np.array_equal(err.cpu().numpy().view(np.uint64), e)
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 32768 * 2 + 1, 32768 * 3 + 3])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 43690, 43691, 32768 * 2 + 1, 32768 * 3 + 3])
 @pytest.mark.parametrize("quality", [1, 4])
 def test_runs_of_blocks_match_oracle(gpu, n, quality):
     """Block counts around the lengths of the runs that a wave takes, with
