@@ -377,7 +377,8 @@ int set_launch(const crn2_encode_set* s, int t, int shape, uint64_t begin, uint6
     const SetShape sh = kSetShapes[shape];
     // colour elements take one wavefront each, alpha elements a run per wavefront
     const uint64_t n = end - begin;
-    const uint32_t run = t == 0 ? 1 : crn2_dxt5a_set_per_wave(n);
+    // (of the whole set's length also where only the tuner's sample is encoded: what is timed is what runs)
+    const uint32_t run = t == 0 ? 1 : crn2_dxt5a_set_per_wave(s->total[1]);
     const uint64_t per = (uint64_t)(sh.tb / 64) * run, full = (n + per - 1) / per;
     const uint64_t cap = sh.wg_per_cu ? (uint64_t)cus * sh.wg_per_cu : full;
     const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(full, std::min<uint64_t>(cap, 1u << 30)));
@@ -394,8 +395,10 @@ int set_choose_shapes(crn2_encode_set* s, hipStream_t st)
     for (int t = 0; t < 2; t++) {
         if (s->shape[t] >= 0 || !s->total[t]) continue;
         const uint64_t end = std::min<uint64_t>(s->total[t], kTuneSample);
-        // the tuner keys its choice by kernel and the sample's size class
-        s->shape[t] = crn2::tuner().pick(t == 0 ? crn2::TUNE_DXT1_SET : crn2::TUNE_DXT5A_SET, end, kNumSetShapes, 0,
+        // the tuner keys its choice by kernel and the set's size class (alpha: what decides the runs' length)
+        // or the sample's (colour: the same launch from there on)
+        s->shape[t] = crn2::tuner().pick(t == 0 ? crn2::TUNE_DXT1_SET : crn2::TUNE_DXT5A_SET,
+                                         t == 0 ? end : s->total[t], kNumSetShapes, 0,
                                          st, [&](int sh) {
                                              return set_launch(s, t, sh, 0, end, st) == CRN2_OK ? hipSuccess
                                                                                                   : hipErrorUnknown;

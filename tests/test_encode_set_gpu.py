@@ -88,3 +88,38 @@ def test_set_matches_per_image_encoder(gpu, tune):
                                               oracle.DXT1_PERCEPTUAL | oracle.DXT1_ALPHA_BLOCKS)[:4]
         w = exp[k].view(np.uint16).reshape(-1, 4)
         assert np.array_equal(w[:, 0], lo) and np.array_equal(w[:, 1], hi), k
+
+
+def test_tuned_set_beyond_the_sample(gpu):
+    """An alpha set of more elements than the tuner's sample (131,072), whose
+    runs are longer than the sample alone would take; flat, two-valued and
+    searched blocks, the same bytes as the per-image encoder."""
+    rng = np.random.default_rng(5)
+    imgs = []
+    for k, (w, h) in enumerate([(2048, 2100), (1021, 515), (7, 5)]):
+        im = np.full((h, w, 4), 200, np.uint8)
+        im[: h // 2, ::2, 3] = 90
+        im[-40:, -40:, 3] = rng.integers(0, 256, im[-40:, -40:, 3].shape)
+        imgs.append(im)
+    srcs = [torch.from_numpy(im.reshape(-1)).cuda() for im in imgs]
+    outs = [torch.zeros(((im.shape[1] + 3) // 4) * ((im.shape[0] + 3) // 4) * 8, dtype=torch.uint8, device="cuda")
+            for im in imgs]
+    items = (EncodeItem * 3)(*[EncodeItem(s.data_ptr(), im.shape[1], im.shape[0], FMT_DXT5A, o.data_ptr())
+                               for s, im, o in zip(srcs, imgs, outs)])
+    lib().crn2_autotune_mode(1)
+    try:
+        s = C.c_void_p()
+        assert lib().crn2_encode_set_create(items, 3, 4, 1 | 2, C.byref(s)) == 0
+        st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        assert lib().crn2_encode_set_run(s, st) == 0
+        torch.cuda.synchronize()
+        ae = C.c_uint64()
+        assert lib().crn2_encode_set_info(s, None, C.byref(ae), None, None) == 0 and ae.value > 1 << 18
+        sh, ms = C.c_int(), C.c_float()
+        assert lib().crn2_autotune_choice(5, ae.value, C.byref(sh), C.byref(ms)) == 0 and 0 <= sh.value < 6
+        print("alpha elements", ae.value, "shape", sh.value, flush=True)
+        for o, im in zip(outs, imgs):
+            assert np.array_equal(o.cpu().numpy(), per_image(FMT_DXT5A, im, 4, 1 | 2)), im.shape
+        assert lib().crn2_encode_set_destroy(s) == 0
+    finally:
+        lib().crn2_autotune_mode(0)
