@@ -71,7 +71,16 @@ constexpr uint32_t kMidList = 64;
 // launch.  Pass 1 has a wave for every 64 lines all the same, and a level of 690
 // contributors takes 17 us in groups; pass 2 has few waves, and the same level
 // takes 44 us in groups and 2 us a wave for each output.
+// So where the waves of single outputs are few, they are taken from much shorter
+// lists on: then nothing hides a chain of four outputs' texels (pass 1 up to
+// 1,024 waves a level, pass 2 up to 256 blocks; with the limits for any number of
+// waves alone, 100x37 with the default filter 36 us before groups, 40 with them,
+// 26 so; 256^2 92 / 57 / 36; 1000x700 box 89 / 106 / 84; with twice as many
+// waves 2048^2 takes 2 % longer again).  Not with wrapped edges, whose lists are
+// many runs: a single sum starts afresh with each (16x16: 18 us in groups, 20
+// singly).
 constexpr uint32_t kLongList = 1024, kLongList2 = 256;
+constexpr uint32_t kFewList = 64, kFewWaves = 1024, kFewList2 = 32, kFewBlocks2 = 256;
 constexpr uint32_t kChunk = 256;   // weights that dot_long fetches at once
 constexpr uint32_t kRunPad = 16;   // a run's weights are padded with zeros to a multiple of this (so that runs start at 16-byte steps)
 
@@ -675,6 +684,13 @@ int crn2_mip_plan_create(uint32_t width, uint32_t height, const crn2_mip_params*
     uint32_t units = 0, blocks = 0;
     // a list as runs (one texel repeated, step 0, or consecutive texels, step 1)
     // and groups of outputs
+    // Every output's texels in one piece, edge texels perhaps repeated (no wrapped edges)
+    auto one_piece = [](const crn2mip::List& L) {
+        for (size_t o = 0; o + 1 < L.offs.size(); o++)
+            for (uint32_t k = L.offs[o] + 1; k < L.offs[o + 1]; k++)
+                if (L.pix[k] != L.pix[k - 1] && L.pix[k] != L.pix[k - 1] + 1) return false;
+        return true;
+    };
     auto add_list = [&](const crn2mip::List& L, bool single) {
         const uint32_t at = (uint32_t)groups.size();
         const size_t n = L.offs.size() - 1;
@@ -712,6 +728,18 @@ int crn2_mip_plan_create(uint32_t width, uint32_t height, const crn2_mip_params*
                 main[i] = runs[best];
                 lo = std::min(lo, main[i].pix);
                 hi = std::max(hi, main[i].pix + main[i].n);
+            }
+            // Outputs whose texels lie far apart (box filters, narrow ones) are summed
+            // each by its own runs: a texel loaded once for four products, most of
+            // weight 0, costs about as much as a contributor of a run, which loads
+            // 16 at a time (2048^2, filter scale 0.1: 99 us, all in groups 103).
+            if (hi && !single) {
+                uint32_t own = 0;
+                for (uint32_t i = 0; i < kGroup; i++) own += (main[i].n + 15) & ~15u;
+                if (hi - (lo & ~3u) > own) {
+                    for (uint32_t i = 0; i < kGroup; i++) G.before[i] = G.after[i] = G.end[i];
+                    hi = 0;
+                }
             }
             if (hi && !single) {
                 G.pix = lo & ~3u;
@@ -771,8 +799,10 @@ int crn2_mip_plan_create(uint32_t width, uint32_t height, const crn2_mip_params*
         a.layout = v.xfirst ? 0 : 1;
         (v.xfirst ? need_lx : need_ly) = true;
         a.nlb = (a.lines + 63) / 64;
-        a.single = first.ops() / a.d >= kLongList ? 1 : 0;
-        a.per = first.ops() / a.d >= kMidList ? 1 : kGroupsPerWave;
+        const uint32_t list = first.ops() / a.d;
+        a.single = list >= kLongList ||
+                   (list >= kFewList && nc * a.nlb * a.d <= kFewWaves && one_piece(first)) ? 1 : 0;
+        a.per = list >= kMidList ? 1 : kGroupsPerWave;
         a.runs = a.single ? a.d : ((a.d + kGroup - 1) / kGroup + a.per - 1) / a.per;
         a.unit0 = units;
         units += nc * a.nlb * a.runs;
@@ -784,7 +814,9 @@ int crn2_mip_plan_create(uint32_t width, uint32_t height, const crn2_mip_params*
         b.d2 = v.xfirst ? v.height : v.width;
         b.nxb = (b.d + 63) / 64;
         b.block0 = blocks;
-        b.single = second.ops() / b.d2 >= kLongList2 ? 1 : 0;
+        const uint32_t list2 = second.ops() / b.d2;
+        b.single = list2 >= kLongList2 ||
+                   (list2 >= kFewList2 && b.d2 * b.nxb <= kFewBlocks2 && one_piece(second)) ? 1 : 0;
         blocks += (b.single ? b.d2 : (b.d2 + kGroup - 1) / kGroup) * b.nxb;
         b.list = add_list(second, b.single);
         b.inter = a.inter;

@@ -81,6 +81,17 @@ def test_every_filter_and_mode(gpu, filt, flags):
     assert_same(gpu_levels(img, filt, flags), oracle_levels(img, filt, flags)[0], (filt, flags))
 
 
+# Levels small enough for a wave per output from short lists on, with edges in
+# one piece and wrapped; filters so narrow that neighbouring outputs share no
+# texels and are summed each by its own run, and on the line between.
+@pytest.mark.parametrize("filt,flags,fs", [(KAISER, SRGB | ALPHA, 0.1), (KAISER, ALPHA | WRAP, 0.4), (BOX, SRGB, 0.5),
+                                           (BOX, ALPHA | WRAP, 0.9), (TENT, SRGB | WRAP, 2.0), (MITCHELL, 0, 0.9)])
+@pytest.mark.parametrize("h,w", [(16, 16), (64, 64), (37, 100), (33, 520)])
+def test_sparse_groups_and_few_waves(gpu, h, w, filt, flags, fs):
+    img = rand_img(h, w, 19)
+    assert_same(gpu_levels(img, filt, flags, fs), oracle_levels(img, filt, flags, fs)[0], (h, w, filt, flags, fs))
+
+
 # One side long enough for every way of summing a list (groups of four outputs
 # with short, middle and long lists, an output a wave), the other odd; a filter
 # with one contributor per texel, and wrapped lists.
