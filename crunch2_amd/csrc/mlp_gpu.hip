@@ -1342,10 +1342,11 @@ __global__ void __launch_bounds__(64 * kPolishWaves) polish_kernel(const uint8_t
 // The whole refinement, one wavefront per block: for calls whose blocks would
 // leave refine_kernel's one lane per block a wave or less per SIMD, where its
 // time is that of the slowest block (4,096 blocks 3.68 ms with the polish in it,
-// here 74 us; 65,536 blocks 0.85 ms with the polish apart, here 0.74).
-// Beyond kWaveBlocks blocks refine_kernel's lanes do more work per operation
-// (both kernels 1.13 ms for 131,044 blocks; here 1.42).
-constexpr uint32_t kWaveBlocks = 65536;
+// here 74 us).  Beyond kWaveBlocks blocks refine_kernel's lanes do more work per
+// operation: 65,536 blocks, one lane per block / here, without the polish 455 /
+// 510 us, of near-flat blocks with it 553 to 753 / 837, of a texture 702 / 677;
+// 49,152 blocks 451 / 386, 515 / 631 (767 with the polish in it), 639 / 512.
+constexpr uint32_t kWaveBlocks = 57344;
 
 __global__ void __launch_bounds__(64 * kPolishWaves) refine_wave_kernel(const uint8_t* __restrict__ rgba, uint32_t n,
                                                                         const float* __restrict__ y,

@@ -239,6 +239,18 @@ def test_polish_takes_the_first_best_lattice_move(gpu, kind):
 
 
 @pytest.mark.parametrize("starts", [learned.START_NET, learned.ENCODE_STARTS])
+def test_refinement_paths_agree_at_the_switch(gpu, starts):
+    """The largest call of one wavefront per block (57,344 blocks) and the
+    smallest of one lane per block give the same for the same blocks."""
+    print("refinement switch", starts, flush=True)
+    t = dev(dxt1.image_blocks(texture.synth(1032, 1024, 13, texture.RGB))[:57345])
+    y = learned.infer(dev(np.load("crunch2_amd/data/dxt1_proposal.npy")), t)
+    lanes = learned.refine(t, y, learned.ENCODE_ITERS, starts)
+    waves = learned.refine(t[:57344], y[:57344], learned.ENCODE_ITERS, starts)
+    assert torch.equal(lanes[:57344], waves)
+
+
+@pytest.mark.parametrize("starts", [learned.START_NET, learned.ENCODE_STARTS])
 def test_refinement_paths_agree(gpu, starts):
     """A call of 65,537 blocks (one lane per block, the polish on its own) gives
     what calls of fewer (one wavefront per block) give for the same blocks."""
