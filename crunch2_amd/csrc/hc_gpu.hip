@@ -171,23 +171,31 @@ __global__ void __launch_bounds__(64 * WAVES) crn2_hc_sel_gemm_kernel(SelArgs a)
 // the banks after its first 16, and so on; the next slot is 16 banks on.
 constexpr uint32_t kScatterIters = 32;
 
-// 16 blocks at a time, as many times as leave 512 workgroups.
+// 16 blocks at a time, as many times as leave 512 workgroups; 0: 16 blocks, the
+// totals straight to memory, where the blocks are too few to wait for one another
+// long (100 blocks, 300 selectors: 22.8 us, through LDS 25.0; 1,000 blocks, 4
+// selectors: 43.9, through LDS 18.7).
+constexpr uint32_t kScatterDirect = 128;
+
 static uint32_t scatter_iters(uint32_t n_blocks)
 {
+    if (n_blocks <= kScatterDirect) return 0;
     const uint32_t n = n_blocks / (16 * 512);
     return n < 1 ? 1 : n > kScatterIters ? kScatterIters : n;
 }
 
 template <uint32_t N, uint32_t SLOTS>
 struct SelTotals {
-    static constexpr uint32_t kFree = 0xFFFFFFFFu, kPitch = N + 16;
+    static constexpr uint32_t kFree = 0xFFFFFFFFu, kPitch = N + 16, kNone = SLOTS;
+    static_assert(SLOTS % 4 == 0 && SLOTS <= 256, "four waves, a slot of each per lane");
     uint32_t tag[SLOTS];
-    uint32_t sum[SLOTS * kPitch];
+    alignas(16) uint32_t sum[SLOTS * kPitch];
 
     __device__ void clear()
     {
         for (uint32_t i = threadIdx.x; i < SLOTS; i += blockDim.x) tag[i] = kFree;
-        for (uint32_t i = threadIdx.x; i < SLOTS * kPitch; i += blockDim.x) sum[i] = 0;
+        for (uint32_t i = threadIdx.x; i < SLOTS * kPitch / 4; i += blockDim.x)
+            reinterpret_cast<uint4*>(sum)[i] = make_uint4(0, 0, 0, 0);
         __syncthreads();
     }
     // The slot of selector s, or SLOTS; the 16 lanes of a block (texel p each) ask together.
@@ -210,9 +218,16 @@ struct SelTotals {
     __device__ void flush(uint32_t* details)
     {
         __syncthreads();
-        for (uint32_t i = threadIdx.x; i < SLOTS * N; i += blockDim.x) {
-            const uint32_t slot = i / N, k = i % N, v = sum[slot * kPitch + 16 * (k % (N / 16)) + k / (N / 16)];
-            if (tag[slot] != kFree && v) atomicAdd(&details[(size_t)tag[slot] * N + k], v);
+        // four waves, every fourth slot each; most are free where few blocks came
+        const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+        const uint32_t mine = tag[(4 * lane + wave) % SLOTS];
+        for (uint64_t m = __ballot(lane < SLOTS / 4 && mine != kFree); m; m &= m - 1) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(m), slot = 4 * l + wave;
+            const uint32_t s = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)l);
+            for (uint32_t k = lane; k < N; k += 64) {
+                const uint32_t v = sum[slot * kPitch + 16 * (k % (N / 16)) + k / (N / 16)];
+                if (v) atomicAdd(&details[(size_t)s * N + k], v);
+            }
         }
     }
 };
@@ -220,7 +235,9 @@ struct SelTotals {
 __global__ void __launch_bounds__(256) crn2_hc_sel_scatter_kernel(SelArgs a, uint32_t iters)
 {
     __shared__ SelTotals<64, 64> totals;
-    if (a.details) totals.clear();
+    const bool gather = a.details && iters;
+    if (gather) totals.clear();
+    if (!iters) iters = 1;
     const uint32_t p = threadIdx.x & 15u;
     for (uint32_t it = 0; it < iters; it++) {
         const uint64_t b = ((uint64_t)blockIdx.x * iters + it) * 16 + (threadIdx.x >> 4);
@@ -230,10 +247,10 @@ __global__ void __launch_bounds__(256) crn2_hc_sel_scatter_kernel(SelArgs a, uin
         if (!a.details) continue;
         uint32_t e[4];
         e2_pixel(a, (uint32_t)b, p, e);
-        const uint32_t slot = totals.claim(s, p);
+        const uint32_t slot = gather ? totals.claim(s, p) : totals.kNone;
         for (uint32_t c = 0; c < 4; c++) totals.add(slot, a.details, s, p, c, e[c]);
     }
-    if (a.details) totals.flush(a.details);
+    if (gather) totals.flush(a.details);
 }
 
 // ----------------------------------------------------------------------------
@@ -364,7 +381,9 @@ __global__ void __launch_bounds__(64 * WAVES) crn2_hc_alpha_sel_gemm_kernel(Alph
 __global__ void __launch_bounds__(256) crn2_hc_alpha_sel_scatter_kernel(AlphaSelArgs a, uint32_t iters)
 {
     __shared__ SelTotals<128, 32> totals;
-    if (a.details) totals.clear();
+    const bool gather = a.details && iters;
+    if (gather) totals.clear();
+    if (!iters) iters = 1;
     const uint32_t p = threadIdx.x & 15u;
     for (uint32_t it = 0; it < iters; it++) {
         const uint64_t b = ((uint64_t)blockIdx.x * iters + it) * 16 + (threadIdx.x >> 4);
@@ -374,13 +393,13 @@ __global__ void __launch_bounds__(256) crn2_hc_alpha_sel_scatter_kernel(AlphaSel
         if (!a.details) continue;
         const int x = a.block_vals[b * 16 + p];
         const uint8_t* cv = a.scatter_values + (size_t)a.endpoint_index[b] * 8;
-        const uint32_t slot = totals.claim(s, p);
+        const uint32_t slot = gather ? totals.claim(s, p) : totals.kNone;
         for (uint32_t v = 0; v < 8; v++) {
             const int d = x - (int)cv[v];
             totals.add(slot, a.details, s, p, v, (uint32_t)(d * d));
         }
     }
-    if (a.details) totals.flush(a.details);
+    if (gather) totals.flush(a.details);
 }
 
 // Per codebook entry and texel, the value with the smallest accumulated error,
@@ -460,7 +479,7 @@ extern "C" int crn2_hc_color_selectors_device(const void* blocks, const uint32_t
     const int shape = crn2::tuner().pick(crn2::TUNE_HC_SEL, (uint64_t)n_blocks * n_selectors, 3, 0, s, launch);
     if (launch(shape) != hipSuccess) return CRN2_EHIP;
     if (details || used) {
-        const uint32_t iters = scatter_iters(n_blocks), run = 16 * iters;
+        const uint32_t iters = scatter_iters(n_blocks), run = 16 * (iters ? iters : 1);
         hipLaunchKernelGGL(crn2_hc_sel_scatter_kernel, dim3((uint32_t)(((uint64_t)n_blocks + run - 1) / run)), dim3(256),
                            0, s, a, iters);
         if (hipGetLastError() != hipSuccess) return CRN2_EHIP;
@@ -492,7 +511,7 @@ extern "C" int crn2_hc_alpha_selectors_device(const void* block_vals, const uint
     hipLaunchKernelGGL(crn2_hc_alpha_sel_gemm_kernel<4>, dim3(wgs), dim3(256), 0, s, a);
     if (hipGetLastError() != hipSuccess) return CRN2_EHIP;
     if (details || used) {
-        const uint32_t iters = scatter_iters(n_blocks), run = 16 * iters;
+        const uint32_t iters = scatter_iters(n_blocks), run = 16 * (iters ? iters : 1);
         hipLaunchKernelGGL(crn2_hc_alpha_sel_scatter_kernel, dim3((uint32_t)(((uint64_t)n_blocks + run - 1) / run)),
                            dim3(256), 0, s, a, iters);
         if (hipGetLastError() != hipSuccess) return CRN2_EHIP;

@@ -69,8 +69,9 @@ def run_alpha_gpu(vals, ei, pal, sel, scatter):
 
 # Totals gathered per run of blocks: two and three times 16 blocks a workgroup
 # with a ragged last one, half of the blocks flat (one selector for all of
-# them), fewer and more selectors than a workgroup has slots for.
-@pytest.mark.parametrize("n,m", [(16391, 20), (24577, 300)])
+# them), fewer and more selectors than a workgroup has slots for; and block
+# counts on either side of the switch to totals straight to memory.
+@pytest.mark.parametrize("n,m", [(128, 20), (129, 300), (16391, 20), (24577, 300)])
 def test_totals_of_frequent_selectors(gpu, n, m):
     from tests.hc_cases import make_alpha_case
     blocks, ei, cols, sel = make_case(n, 30, m, seed=m, subblocks=False)
