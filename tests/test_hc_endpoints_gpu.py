@@ -93,3 +93,44 @@ def test_refiner_sums_any_size(gpu, sizes, what):
     ref = oracle.hc_alpha_endpoints(vals, ofs, bc, av, enc)
     assert np.array_equal(got[0].cpu().numpy().view(np.uint32), ref[0])
     assert np.array_equal(got[1].cpu().numpy(), ref[1]) and np.array_equal(got[2].cpu().numpy(), ref[2])
+
+
+# Two neighbouring values, how often each, and the step j: the mean of their
+# float32 values over 255 is exactly j / 256 (of the last, 43 / 64 too).
+ON_THE_LINE = [(164, 466, 257, 165), (138, 916, 771, 139), (216, 1430, 257, 217), (171, 2105, 1028, 172)]
+
+
+@pytest.mark.parametrize("k", [1, 3])
+@pytest.mark.parametrize("far", [0, 255])
+def test_refiner_start_on_a_line_of_the_cut(gpu, k, far):
+    """The best block gives both values one end and the far one the other, so
+    that end's least-squares start lies on a line of its cut: the bound of the
+    parallel sums reaches over it, and the sums are taken in texel order.  The
+    endpoints are the oracle's."""
+    print("refiner start on the line", k, far, flush=True)
+    rng = np.random.default_rng(k + far)
+    parts = []
+    for v, a, b, j in ON_THE_LINE:
+        x = [float(np.float32(u) / np.float32(255.0)) for u in (v, v + 1)]
+        assert (a * x[0] + b * x[1]) * 256 == (a + b) * j      # (exact in doubles)
+        for _ in range(3):
+            parts.append(rng.permutation(np.array([v] * (a * k) + [v + 1] * (b * k) + [far] * 70, np.uint8)))
+    ofs, bc, blocks = _one_cluster_each([len(v) for v in parts])
+    vals = np.concatenate(parts)
+    av, enc = blocks[:, :, 3].copy(), np.zeros(2, np.uint8)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    got = hc.alpha_endpoints(d(vals), d(ofs.astype(np.int32)), d(bc.view(np.int32)), d(av), d(enc))
+    torch.cuda.synchronize()
+    ref = oracle.hc_alpha_endpoints(vals, ofs, bc, av, enc)
+    for c, v in enumerate(parts):     # one end for the two values, the other for the far one
+        near = ref[1][c].astype(int)
+        assert sorted(near[[0, 7]])[0 if far else 1] in (v[v != far].min(), v[v != far].max()) and far in near[[0, 7]]
+    assert np.array_equal(got[0].cpu().numpy().view(np.uint32), ref[0])
+    assert np.array_equal(got[1].cpu().numpy(), ref[1]) and np.array_equal(got[2].cpu().numpy(), ref[2])
+    # the same as grey colours (cut to 32 and 64 steps)
+    px = np.full((len(vals), 4), 255, np.uint8)
+    px[:, :3] = vals[:, None]
+    w = np.ones(2, np.float32)
+    ends, cv, _, ne = run_gpu(px, ofs, bc, blocks, w, enc, True)
+    rends, rcv, _ = oracle.hc_color_endpoints(px, ofs, bc, blocks, w, enc, True)
+    assert ne == 0 and np.array_equal(cv, rcv) and np.array_equal(ends, rends)
