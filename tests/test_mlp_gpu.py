@@ -2,12 +2,15 @@
 (oracle/mlp.py): features, the strided GEMM, forward/backward gradients of the
 training kernels, the bfloat16 matrix-core inference, the exact refinement
 error, and an ablation showing what the trained network gains."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 from oracle import mlp as omlp
 from crunch2_amd import dxt1, learned, texture
+from crunch2_amd._lib import check, lib
 from tests.hc_cases import blocks_from_texture
 
 pytestmark = pytest.mark.gpu
@@ -161,6 +164,55 @@ def train_small(seed=0, steps=300, n=262144, batch=8192):
         idx = torch.randint(0, x.shape[0], (batch,), device="cuda", generator=g)
         tr.step(x[idx].contiguous(), t[idx].contiguous())
     return tr
+
+
+def layered_gradients(theta, X, T, labels):
+    """The loss and gradient layer by layer through the layers' own entry points."""
+    n, o, N, H, K = X.shape[0], learned.OFFSETS, learned.N_IN, learned.N_H, learned.N_OUT
+    new = lambda *s: torch.zeros(s, dtype=torch.float32, device="cuda")
+    p = lambda t, ofs=0: C.c_void_p(t.data_ptr() + 4 * ofs if t is not None else 0)
+    s, L, mm = C.c_void_p(torch.cuda.current_stream().cuda_stream), lib(), learned.gemm
+    Z1, A1, Z2, A2, dA, dZ, Y, dY = new(n, H), new(n, H), new(n, H), new(n, H), new(n, H), new(n, H), new(n, K), new(n, K)
+    g, loss, ones = torch.zeros_like(theta), new(1), torch.ones(1, device="cuda")
+    mm(n, H, N, X, N, 1, theta, H, 1, Z1, H, round_a=True, round_b=True, b_ofs=o["W1"])
+    check(L.crn2_mlp_bias_act_device(p(Z1), p(A1), p(theta, o["b1"]), n, H, 1, s))
+    mm(n, H, H, A1, H, 1, theta, H, 1, Z2, H, round_b=True, b_ofs=o["W2"])
+    check(L.crn2_mlp_bias_act_device(p(Z2), p(A2), p(theta, o["b2"]), n, H, 1, s))
+    mm(n, K, H, A2, H, 1, theta, K, 1, Y, K, round_b=True, b_ofs=o["W3"])
+    check(L.crn2_mlp_bias_act_device(p(Y), p(Y), p(theta, o["b3"]), n, K, 0, s))
+    check(L.crn2_mlp_loss_device(p(Y), p(T), p(labels), n, p(dY), p(loss), s))
+    ks = max(1, min(64, n // 1024))
+    mm(H, K, n, A2, 1, H, dY, K, 1, g, K, ksplit=ks, c_ofs=o["W3"])
+    mm(1, K, n, ones, 0, 0, dY, K, 1, g, K, ksplit=ks, c_ofs=o["b3"])
+    mm(n, H, K, dY, K, 1, theta, 1, K, dA, H, round_b=True, b_ofs=o["W3"])
+    check(L.crn2_mlp_gelu_back_device(p(dA), p(Z2), p(dZ), n * H, s))
+    mm(H, H, n, A1, 1, H, dZ, H, 1, g, H, ksplit=ks, c_ofs=o["W2"])
+    mm(1, H, n, ones, 0, 0, dZ, H, 1, g, H, ksplit=ks, c_ofs=o["b2"])
+    mm(n, H, H, dZ, H, 1, theta, 1, H, dA, H, round_b=True, b_ofs=o["W2"])
+    check(L.crn2_mlp_gelu_back_device(p(dA), p(Z1), p(dZ), n * H, s))
+    mm(N, H, n, X, 1, N, dZ, H, 1, g, H, round_a=True, ksplit=ks, c_ofs=o["W1"])
+    mm(1, H, n, ones, 0, 0, dZ, H, 1, g, H, ksplit=ks, c_ofs=o["b1"])
+    return loss, g
+
+
+@pytest.mark.parametrize("n", [1, 300, 5000])
+@pytest.mark.parametrize("labelled", [False, True])
+def test_layers_match_the_fused_gradient(gpu, n, labelled):
+    """The layers' entry points and the fused kernel compute the same loss and
+    gradient.  Both sum in float32 in other orders; an activation near a
+    bfloat16 step can round to either neighbour, which moves one of its 128
+    terms by 2^-9 of itself: 2^-9 / 128 of the whole, for a few rows, or 1.5e-5
+    for one row alone."""
+    print("layers", n, labelled, flush=True)
+    blocks = dxt1.image_blocks(texture.synth(300, 300, n, texture.RGB))[:n]
+    rng = np.random.default_rng(n)
+    t, lab = dev(rng.random((n, 6)).astype(np.float32)), dev(rng.integers(0, 2, n).astype(np.float32))
+    theta = dev(omlp.init_params(n))
+    x = learned.features(dev(blocks))
+    loss, g = learned.Trainer(theta).gradients(x, t, lab if labelled else None)
+    rloss, rg = layered_gradients(theta, x, t, lab if labelled else None)
+    assert abs(float(loss.item()) - float(rloss.item())) <= 2e-5 * max(1.0, abs(float(rloss.item())))
+    assert float((g - rg).norm() / rg.norm()) <= 2e-5
 
 
 def _pair_errors(px, e):
