@@ -938,8 +938,8 @@ namespace four {
 // ring has run dry; that step's read then goes out again.  Tests that asked
 // eight producers and waited for the answer took 700 cycles each.
 // Level 0 of a 2048^2 DXT5 texture (v_readlane from entries of two blocks, one
-// E8 entry per readfirstlane): 4.26 ms, now 2.87 ms, about
-// 140 cycles a step.
+// E8 entry per readfirstlane; 73,700 lookups): 4.26 ms, 58 ns each; now 41,000
+// lookups, 2.87 ms, 70 ns each.
 //
 // The walker reports the segment it has reached; the producers never overwrite
 // that segment or a later unread one.

@@ -21,7 +21,7 @@
 // What bounds it: vector integer work, 14 value distances per candidate and
 // distinct value, two per 16-bit packed operation.  One lane per block with
 // the state in scratch took 35.6 ms for the alpha elements of 16 textures of
-// 64^2 to 1024^2 with mips (one slow lane held 63 up), now 2.7 ms.
+// 64^2 to 1024^2 with mips (one slow lane held 63 up), now 2.6 ms.
 //
 // Block gather for whole images follows crnlib/crn_dxt_image.cpp:330-344
 // (4x4 texels with edge clamp) and :1491-1523 (component index, quality and

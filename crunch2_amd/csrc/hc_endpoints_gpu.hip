@@ -201,6 +201,10 @@ __device__ inline void fit_solve(const FitSums& f, double ax, double bx, double 
 // one addition inside a power of two every further one there moves the sum by
 // the same multiple of its last place (a tie rounds to an even sum, and from
 // an even sum the same way each time), so each power of two takes a few steps.
+// A skip ends one to two additions below the next power of two, so that the
+// second sum of the next pair is the first one past it: the first of a pair that
+// is skipped on is then a sum of two inside (below the power where ties begin,
+// every sum is exact).
 __device__ inline double repeat_sum(double c, uint32_t n)
 {
     double s = 0.0;

@@ -22,7 +22,7 @@
 // What bounds it: the loads and table look-ups of samples where lists are
 // short, one output's serial chain where they are long (dot_long).  3840x2160
 // with the default filter, one output at a time and a texel per load: pass 1
-// 595 us, pass 2 272 us; now 253 and 122 us.  Eight outputs at once would load a
+// 595 us, pass 2 272 us; now 245 and 119 us.  Eight outputs at once would load a
 // quarter less, and multiply by more zeros.
 // The order of the passes is the reference's choice per level: X then Y
 // (always, for the multithreaded resampler) or, where the single-thread

@@ -10,8 +10,8 @@
 //          the 6-D endpoint tree grown to 65,535 leaves; the distinct
 //          dxt_fast selector words counted in a device hash set.
 //   pack   endpoint clusters cut from the tree on the host (depth first);
-//          their texels gathered and searched one wave per cluster by the
-//          cluster endpoint search (dxt1c_gpu.hip) or, at quality 255,
+//          their texels gathered and searched, a workgroup per cluster, by
+//          the cluster endpoint search (dxt1c_gpu.hip) or, at quality 255,
 //          block by block (dxt1_gpu.hip); selector vectors per block; the
 //          threaded selector clusters (three PCA divisions, four trees);
 //          the selector optimisation one wave per selector cluster, lanes =

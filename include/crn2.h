@@ -99,7 +99,9 @@ int crn2_unpack_level_device(crn2_unpack_ctx* ctx, void** dst_dev, uint32_t dst_
                              uint32_t level, void* stream);
 
 /* Transcodes levels [first, first + count) of every face into one device
- * buffer, levels in order, faces in order within a level, minimal pitch. */
+ * buffer, levels in order, faces in order within a level, minimal pitch.  The
+ * context keeps the call's plan (device memory, up to 24 bytes per bit of the
+ * levels' streams) until the next device call or crn2_unpack_end. */
 int crn2_unpack_levels_device(crn2_unpack_ctx* ctx, void* dst_dev, uint64_t dst_size, uint32_t first,
                               uint32_t count, void* stream);
 
@@ -109,9 +111,9 @@ uint64_t crn2_levels_size(crn2_unpack_ctx* ctx, uint32_t first, uint32_t count);
 int crn2_unpack_end(crn2_unpack_ctx* ctx);
 
 /* ------------------------------------------------------ batched transcode */
-/* A plan that transcodes every level of n textures in one parse launch and
- * one write launch (the reference transcodes one level per call; there is no
- * counterpart for the batch).  Texture i is written to dst_dev[i] as
+/* A plan that transcodes every level of n textures in one sequence of launches
+ * (the reference transcodes one level per call; there is no counterpart for
+ * the batch).  Texture i is written to dst_dev[i] as
  * crn2_unpack_levels_device(ctxs[i], dst_dev[i], .., 0, levels) would write
  * it.  The plan shares each context's scratch: two runs that touch the same
  * context must not overlap. */
@@ -224,11 +226,11 @@ int crn2_compress_blocks(const uint32_t* pixels, uint32_t nblocks, uint32_t form
  * aligned) and the device buffer its DXTn blocks go to (8-byte aligned,
  * minimal pitch, the element layout of crn2_encode_image_device); formats
  * DXT1, DXT5, DXT5A, DXN_XY, DXN_YX.  All colour elements of the set run in
- * one launch, all alpha elements in a second, each thread taking elements
- * with a grid stride.  quality 0..4, flags as crn2_encode_image_device.  With
+ * one launch (a wavefront per element), all alpha elements in a second (runs
+ * of elements per wavefront).  quality 0..4, flags as crn2_encode_image_device.  With
  * the autotuner on (crn2_autotune_mode(1)), the first run times six launch
- * shapes (64 / 128 / 256 threads per workgroup, one thread per element or a
- * persistent grid of 8 x 256 threads per CU) on the first 131,072 elements of
+ * shapes (64 / 128 / 256 threads per workgroup, one wavefront per element or
+ * run or a persistent grid of 8 x 256 threads per CU) on the first 131,072 elements of
  * each launch and keeps the fastest.  crn2_encode_set_run_graph captures the
  * two launches into a HIP graph on its first call and replays it afterwards
  * (the items' buffers must stay where they were). */
@@ -268,8 +270,8 @@ int crn2_decompress_blocks(const void* blocks, uint32_t nblocks, uint32_t format
 /* The same search for pixel clusters of any size on the path dxt_hc takes for
  * its endpoint clusters (crn_dxt_hc.cpp:663-754 calling
  * dxt1_endpoint_optimizer::compute with uber quality and no 3-colour blocks;
- * crn_dxt1.cpp:1759-1869 evaluators), one wave per cluster.  rgba: all
- * clusters' texels (RGBA8 words, alpha ignored), cluster c owning texels
+ * crn_dxt1.cpp:1759-1869 evaluators), one workgroup per cluster (one to eight
+ * waves by its texel count).  rgba: all clusters' texels (RGBA8 words, alpha ignored), cluster c owning texels
  * [offsets[c], offsets[c+1]); flags bit0 perceptual, bit1 m_use_alpha_blocks
  * (the uber evaluator with 3-colour blocks, crn_dxt1.cpp:1370-1592, as qdxt1
  * runs it, crn_qdxt1.cpp:616-626), bits 8..15 with bit1: the DXT1A alpha
